@@ -4,13 +4,15 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload dsv3_rank]
 
 A step is one pass of the path over one resident batch, in the configuration `custom_kernel`
-runs: routing + dispatch in one launch, then the combine with the expert stand-in folded in (two
-launches at the default workload), replayed from a hipGraph.  Inputs are in HBM before the timed
+runs: the whole path in one launch at the default workload, the expert stand-in folded in, as plain
+launches and replayed from a hipGraph.  Inputs are in HBM before the timed
 region starts.  Prints ONE JSON line:
 
-  value        achieved GB/s of dispatch+combine: algorithmic bytes (read x once, write R
-               rows; read R rows, write T rows) / summed GPU durations of the routing,
-               dispatch and combine kernels of a step.  Kernel durations come from HIP
+  value        achieved GB/s of dispatch+combine: the bytes that the form has to move (read x once, write
+               R rows, write T rows; a combine that is a kernel of its own reads the R rows as well) /
+               summed GPU durations of the routing, dispatch and combine kernels of a step.
+               `two_pass_equivalent_GBps` is the same time priced on the bytes of a separate dispatch and
+               combine (a figure for comparing times, not a rate of the memory).  Kernel durations come from HIP
                events bound to each launch, on the stream the kernels run on.
   ms_per_step  wall time of a whole step: events around K steps launched back to back from a C loop
                behind an already filled queue (graph_ms_per_step: the same K steps as hipGraph replays,
@@ -226,6 +228,13 @@ FORWARD_KERNELS = ("forward_token", "forward_tile", "dispatch_fold")  # dispatch
 STUB_KERNELS = ("stub_rows", "stub_fp8")
 
 
+def reads_rows_back(lib):
+    """Whether moe_a2a_forward with the stub folded in runs a combine of its own over the dispatched rows."""
+    from kernel_amd import _lib
+
+    return lib.moe_a2a_get_option(_lib.OPT_TWO_LAUNCHES) == 1
+
+
 def per_step(per, names, steps):
     return sum(sum(per.get(n, [])) for n in names) / steps
 
@@ -379,7 +388,9 @@ def phase_times(per, steps, wall_us):
     launches = {k: sum(len(per.get(n, [])) for n in v) / steps for k, v in names.items()}
     kernel = {k: per_step(per, v, steps) for k, v in names.items()}
     n_all = sum(launches.values())
-    gap = max(0.0, wall_us - sum(kernel.values())) / n_all if n_all else 0.0
+    # below zero where a launch that carries events takes longer than the plain launch it stands for (a
+    # kernel of 3.6 us reads 4.1 with its events): the period is the wall clock either way
+    gap = (wall_us - sum(kernel.values())) / n_all if n_all else 0.0
     for k in names:
         t[k + "_kernel"] = kernel[k]
         t[k] = kernel[k] + gap * launches[k]
@@ -434,9 +445,9 @@ def main():
     # stream carry implicit waits on every other stream of the process.
     main = torch.cuda.Stream()
     main.wait_stream(torch.cuda.current_stream())
-    # with the stub folded in, the combine reads the dispatched rows themselves (fp8 bytes and scales
-    # after an fp8 dispatch, not 16-bit expert rows)
-    ab = contract.algorithmic_bytes(T, K, H, 2, 2, fp8, stub_folded=fuse_stub)
+    # with the stub folded in, the weighted sum of a token comes out of the registers that its dispatch
+    # stored from (MOE_A2A_OPT_TWO_LAUNCHES: a combine of its own, which reads the dispatched rows)
+    ab = contract.algorithmic_bytes(T, K, H, 2, 2, fp8, stub_folded=fuse_stub, rows_read_back=reads_rows_back(lib))
     b_dc = ab["dispatch"] + ab["combine"]
     use_graph = not args.no_graph
     dtype = "fp8-e4m3 dispatch, bf16 combine" if fp8 else {"bfloat16": "bf16", "float16": "f16"}[
@@ -514,6 +525,8 @@ def main():
         stub_us=round(t["stub"], 3), combine_us=round(t["combine"], 3), one_launch_us=round(t["forward"], 3),
         launch_overhead_us_per_launch=round(t["gap"], 3),
         pct_of_hbm_peak=round(100.0 * value / HBM_PEAK_GBPS, 2),
+        two_pass_equivalent_GBps=round(sum(contract.algorithmic_bytes(T, K, H, 2, 2, fp8, stub_folded=fuse_stub)[k]
+                                           for k in ("dispatch", "combine")) / t["dc"] / 1e3, 1),
         kernel_only=dict(dispatch_combine_us=round(t["dc_kernel"], 3),
                          pct_of_hbm_peak=round(100.0 * b_dc / t["dc_kernel"] / 1e3 / HBM_PEAK_GBPS, 2),
                          what="sum of the kernels' own durations (HIP events), launch overhead left out"),
@@ -546,7 +559,8 @@ def main():
             o_ms = other.loop_wall(args.steps, args.warmup)
             o_per, _ = other.kernels(args.steps, args.warmup, o_ms * 1e3)
             ot = phase_times(o_per, args.steps, o_ms * 1e3)
-            o_ab = contract.algorithmic_bytes(T, K, H, 2, 2, fp8, stub_folded=leg_fuse)
+            o_ab = contract.algorithmic_bytes(T, K, H, 2, 2, fp8, stub_folded=leg_fuse,
+                                              rows_read_back=reads_rows_back(lib))
             o_bytes = o_ab["dispatch"] + o_ab["combine"]
             out[name] = dict(
                 dispatch_combine_us=round(ot["dc"], 3), dispatch_us=round(ot["dispatch"] + ot["route"], 3),
@@ -634,7 +648,7 @@ def workload_leg(torch, lib, contract, name, main, dev, args):
     ms = leg.loop_wall(steps, args.warmup)
     per, _ = leg.kernels(steps, args.warmup, ms * 1e3)
     t = phase_times(per, steps, ms * 1e3)
-    ab = contract.algorithmic_bytes(T, K, H, 2, 2, fp8, stub_folded=True)
+    ab = contract.algorithmic_bytes(T, K, H, 2, 2, fp8, stub_folded=True, rows_read_back=reads_rows_back(lib))
     b_dc = ab["dispatch"] + ab["combine"]
     if any(n in per for n in FORWARD_KERNELS):
         cand = [(next(n for n in FORWARD_KERNELS if n in per), b_dc)]
@@ -751,7 +765,8 @@ def calibrate_copy(torch, main, dev):
 KERNEL_OF_SYMBOL = (("route_dispatch_fp8_tile_kernel", "route_dispatch_fp8"),
                     ("route_dispatch_tile_kernel", "route_dispatch_tile"), ("route_dispatch_kernel", "route_dispatch"),
                     ("forward_token_kernel", "forward_token"), ("forward_tile_kernel", "forward_tile"),
-                    ("dispatch_fold_kernel", "dispatch_fold"),
+                    ("dispatch_fold_kernel", "dispatch_fold"), ("forward_fp8_tile_kernel", "forward_tile"),
+                    ("dispatch_fold_fp8_kernel", "dispatch_fold"),
                     ("stub_combine_rows_kernel", "stub_combine"), ("stub_combine_fp8_kernel", "stub_combine"),
                     ("combine_rows_kernel", "combine_rows"), ("dispatch_rows_kernel", "dispatch_rows"),
                     ("dispatch_fp8_kernel", "dispatch_fp8"), ("stub_rows_kernel", "stub_rows"),

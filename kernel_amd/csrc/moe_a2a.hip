@@ -15,8 +15,8 @@
 //   route_dispatch_fp8 routing and that copy in one launch, a tile of tokens per workgroup
 //   stub_*             expert stand-in, one factor per row
 //   combine / stub_combine   gather K rows per token, weighted sum
-//   forward_token / forward_tile   the whole path of a token (routing, dispatch, stub, weighted sum)
-//                      in one launch: a workgroup reads back the rows it stored itself
+//   forward_token / forward_tile / forward_fp8_tile   the whole path of a token (routing, dispatch,
+//                      stub, weighted sum) in one launch; the sum comes out of registers
 //   dispatch_fold      dispatch, stub and weighted sum of a token behind a routing of its own
 //   expert_gemm        y[rows of e] = x[rows of e] * W_e^T, 128 x 128 tiles (short segments)
 //   expert_gemm_wide   the same on 256 x 256 tiles, software-pipelined; 16-bit or fp8 rows
@@ -618,12 +618,15 @@ int moe_a2a_dispatch_fp8(const void* x, int x_type, const int32_t* slot_of_entry
 static bool route_dispatch_fp8_ok(int T, int K, int H) {
   return T > 0 && K <= kTileMaxOwn && H % MOE_A2A_FP8_BLOCK == 0;
 }
+// A few hundred tokens or less: as few per tile as it takes to give every CU a workgroup.
 static int fp8_tile_tokens(int T, int K) {
   const int cap = std::max(kTileMaxOwn / K, 1), wave = std::max(kWave / K, 1);
   const int forced = option(MOE_A2A_OPT_FP8_TILE);
   if (forced > 0) return std::min(forced, cap);
-  return std::min(cap, std::max(wave, ceil_div(T, 2 * 256)));
+  const int spread = ceil_div(T, 256);
+  return std::min(cap, spread < wave ? spread : std::max(wave, ceil_div(T, 2 * 256)));
 }
+static int fp8_tile_threads(int E) { return E <= 512 ? 512 : kTileThreads; }
 static int route_dispatch_fp8_impl(const void* x, int x_type, const int32_t* indices, const int32_t* rank_start,
                                    int src_rank, int T, int K, int E, int W, int H, int max_recv, int32_t* counts,
                                    int32_t* offsets, int32_t* slot_of_entry, int32_t* src_of_slot, int32_t* meta,
@@ -639,7 +642,7 @@ static int route_dispatch_fp8_impl(const void* x, int x_type, const int32_t* ind
   const int tile = fp8_tile_tokens(T, K);
   // workgroups of 512 lanes, three to a CU, so that one's table pass runs under another's rows (a thread
   // per expert in the scan: 1024 lanes beyond 512 experts)
-  const int threads = E <= 512 ? 512 : kTileThreads;
+  const int threads = fp8_tile_threads(E);
   dim3 grid((unsigned)ceil_div(T, tile)), block(threads);
   const bool st = streams(T, (long long)T * K, H, 2, 1);
 #define RDF8_T(EL, ST, TH)                                                                                       \
@@ -865,13 +868,16 @@ int moe_a2a_stub_combine(const void* disp, const float* disp_scale, const int32_
 }
 #undef MOE_A2A_SWITCH_KT
 
-// The whole path in one launch (forward_token_kernel): small routing tables, 16-bit rows of one
-// element type, compact layout, stub folded in.
+// The whole path in one launch: rows of one element type, compact layout, stub folded in.
 // 0: no; 1: one token per workgroup (forward_token_kernel); 2: a tile of tokens per workgroup
-// (forward_tile_kernel), wherever moe_a2a_route_dispatch would take its token-tile kernel by itself.
+// (forward_tile_kernel), wherever moe_a2a_route_dispatch would take its token-tile kernel by itself;
+// 3: the same with an fp8 dispatch (forward_fp8_tile_kernel), while the table passes of all its workgroups
+// stay short: up to kFusedMaxRows entries a routing launch of its own costs more than they do.
 static int forward_one_launch_form(int T, int K, int H, int max_recv, int in_type, int out_type, int fp8_dispatch) {
-  if (fp8_dispatch || max_recv > 0 || in_type != out_type || T < 1) return 0;
-  if (option(MOE_A2A_OPT_TWO_LAUNCHES) == 1 || !moe_a2a_fused_ok(T, K, H)) return 0;
+  if (max_recv > 0 || in_type != out_type || T < 1) return 0;
+  if (option(MOE_A2A_OPT_TWO_LAUNCHES) == 1) return 0;
+  if (fp8_dispatch) return route_dispatch_fp8_ok(T, K, H) && (long long)T * K <= kFusedMaxRows ? 3 : 0;
+  if (!moe_a2a_fused_ok(T, K, H)) return 0;
   if (fused_small_ok(T, K, H) && option(MOE_A2A_OPT_ROUTE_TILE) != 1) {
     const RowGeom g = fused_geom(H / 8, T * K);
     if (fused_entries_per_thread(T * K, g.threads) <= 8) return 1;
@@ -889,13 +895,16 @@ static bool dispatch_fold_ok(int T, int K, int H, int max_recv, int in_type, int
                              int fuse_route) {
   if (max_recv > 0 || in_type != out_type || T < 1) return false;
   if (option(MOE_A2A_OPT_TWO_LAUNCHES) == 1) return false;
-  // The fold behind an fp8 dispatch is routed by a launch of its own.  It pays while the rows stay in
-  // the caches (one launch boundary less); at streaming volumes two kernels (routing + dispatch in one,
-  // then stub + combine) move the same bytes about 1 % faster (120.0 against 118.8 us at 16384 tokens,
-  // top-8, H = 7168).
-  if (fp8_dispatch) return !streams(T, 2ll * T * K, H, 2, 1);
+  // the fold behind an fp8 dispatch is routed by a launch of its own
+  if (fp8_dispatch) return true;
   return !(fuse_route == 2 ? K <= kTileMaxOwn : (fuse_route == 1 && moe_a2a_fused_ok(T, K, H)));
 }
+
+// Nothing in a call that folds out of registers reads the dispatched rows, so their stores need not pass
+// through the memory-side cache (256 MB): non-temporal ones leave it to x, which the caller has just
+// written -- 80 -> 72 us at 2500 tokens of 7168 columns, top-8, 92 -> 87 at 5000 of 4096 -- while x is well below
+// the cache's size (at 134 MB of x nothing is kept either way, and write-through rows are 1-2 % ahead).
+static bool fold_rows_nt(int T, int H) { return (long long)T * H * 2 <= (72ll << 20); }
 
 static int dispatch_fold_fp8(const void* x, const int32_t* indices, const float* weights,
                              const int32_t* slot_of_entry, void* disp_q, float* disp_scale, void* out, int T, int K,
@@ -905,13 +914,17 @@ static int dispatch_fold_fp8(const void* x, const int32_t* indices, const float*
   if (!aligned16(out)) return MOE_A2A_E_ALIGN;
   if (!indices || !weights || !slot_of_entry || !disp_scale || !out) return MOE_A2A_E_NULL;
   const int nblk = H / MOE_A2A_FP8_BLOCK, E_l = E / W;
-  const RowGeom g = row_geom(nblk * 8, 8);  // cache-resident volumes only: see dispatch_fold_ok
+  const RowGeom g = row_geom(nblk * 8, 8);
   dim3 grid((unsigned)T * g.nsplit), block(g.threads);
+  const bool nt_out = !fold_rows_nt(T, H);
 #define DF8_ARGS                                                                                                  \
   (const uint4*)x, indices, weights, slot_of_entry, (uint4*)disp_q, disp_scale, (uint4*)out, stub_kind, E, E_l, K, \
       nblk, g.per, g.nsplit, pow2
-#define DF84(EL, MD, KT) \
-  return launch(KID_DISPATCH_FOLD, dispatch_fold_fp8_kernel<EL, MD, KT, 0>, grid, block, 0, stream, DF8_ARGS);
+#define DF84(EL, MD, KT)                                                                                               \
+  {                                                                                                                    \
+    if (nt_out) return launch(KID_DISPATCH_FOLD, dispatch_fold_fp8_kernel<EL, MD, KT, 1>, grid, block, 0, stream, DF8_ARGS); \
+    return launch(KID_DISPATCH_FOLD, dispatch_fold_fp8_kernel<EL, MD, KT, kPlain>, grid, block, 0, stream, DF8_ARGS);  \
+  }
 #define DF83(EL, MD)             \
   {                              \
     switch (K) {                 \
@@ -939,16 +952,16 @@ static int dispatch_fold(const void* x, const int32_t* indices, const float* wei
   if (!aligned16(out)) return MOE_A2A_E_ALIGN;
   if (!indices || !weights || !slot_of_entry || !out) return MOE_A2A_E_NULL;
   const int nvec = H / 8, E_l = E / W;
-  const bool st = streams(T, 2ll * T * K + T, H, 2, 2);
-  const RowGeom g = row_geom(nvec);
+  const RowGeom g = row_geom(nvec, 1, kFoldThreads);
   dim3 grid((unsigned)T * g.nsplit), block(g.threads);
 #define DF_ARGS                                                                                                   \
   (const uint4*)x, indices, weights, slot_of_entry, (uint4*)disp, (uint4*)out, stub_kind, E, E_l, K, nvec, g.per, \
       g.nsplit
-#define DF4(EL, MD, KT)                                                                                            \
-  {                                                                                                                \
-    if (st) return launch(KID_DISPATCH_FOLD, dispatch_fold_kernel<EL, MD, KT, 2>, grid, block, 0, stream, DF_ARGS); \
-    return launch(KID_DISPATCH_FOLD, dispatch_fold_kernel<EL, MD, KT, 0>, grid, block, 0, stream, DF_ARGS);        \
+  const bool nt = fold_rows_nt(T, H);
+#define DF4(EL, MD, KT)                                                                                          \
+  {                                                                                                              \
+    if (nt) return launch(KID_DISPATCH_FOLD, dispatch_fold_kernel<EL, MD, KT, 1>, grid, block, 0, stream, DF_ARGS); \
+    return launch(KID_DISPATCH_FOLD, dispatch_fold_kernel<EL, MD, KT, 0>, grid, block, 0, stream, DF_ARGS);      \
   }
 #define DF3(EL, MD)              \
   {                              \
@@ -993,10 +1006,10 @@ int moe_a2a_forward_launches(int T, int K, int H, int max_recv, int in_type, int
 static int forward_one_launch(const void* x, const int32_t* indices, const float* weights, const int32_t* rank_start,
                               int src_rank, int T, int K, int E, int W, int H, int elem_type, int stub_kind,
                               int combine_mode, int32_t* counts, int32_t* offsets, int32_t* slot_of_entry,
-                              int32_t* src_of_slot, int32_t* meta, int32_t* status, void* disp, void* out,
-                              hipStream_t stream, int32_t* clear_status) {
+                              int32_t* src_of_slot, int32_t* meta, int32_t* status, void* disp, float* disp_scale,
+                              void* out, int fp8_dispatch, hipStream_t stream, int32_t* clear_status) {
   if (int rc = check_route_shape(T, K, E, W)) return rc;
-  if (int rc = check_rows(x, disp, T, K, H, 8)) return rc;
+  if (int rc = check_rows(x, disp, T, K, H, fp8_dispatch ? MOE_A2A_FP8_BLOCK : 8)) return rc;
   if (!aligned16(out)) return MOE_A2A_E_ALIGN;
   if (!counts || !offsets || !indices || !weights || !slot_of_entry || !src_of_slot || !meta || !out)
     return MOE_A2A_E_NULL;
@@ -1004,6 +1017,30 @@ static int forward_one_launch(const void* x, const int32_t* indices, const float
               slot_of_entry, src_of_slot, meta, status, clear_status};
   const int nvec = H / 8;
   const int E_l = E / W;
+  if (fp8_dispatch) {
+    const int tile = fp8_tile_tokens(T, K), threads = fp8_tile_threads(E), nblk = H / MOE_A2A_FP8_BLOCK;
+    dim3 grid((unsigned)ceil_div(T, tile)), block(threads);
+#define FW8(EL, MD, KT, TH)                                                                                      \
+  return launch(KID_FORWARD_TILE, forward_fp8_tile_kernel<EL, MD, KT, TH>, grid, block, 0, stream, a,            \
+                (const uint4*)x, (uint4*)disp, disp_scale, weights, (uint4*)out, stub_kind, E_l, nblk, tile,     \
+                fp8_dispatch == 2)
+#define FW8M(EL, MD)                          \
+  {                                           \
+    if (threads != 512) FW8(EL, MD, 0, kTileThreads); \
+    if (K == 8) FW8(EL, MD, 8, 512);          \
+    FW8(EL, MD, 0, 512);                      \
+  }
+#define FW8E(EL)                                                        \
+  {                                                                     \
+    if (combine_mode == MOE_A2A_COMBINE_STRICT) FW8M(EL, MOE_A2A_COMBINE_STRICT) \
+    FW8M(EL, MOE_A2A_COMBINE_F32)                                       \
+  }
+    if (elem_type == MOE_A2A_BF16) FW8E(Bf16)
+    FW8E(F16)
+#undef FW8E
+#undef FW8M
+#undef FW8
+  }
   if (forward_one_launch_form(T, K, H, 0, elem_type, elem_type, 0) == 2) {
     const int tile = tile_tokens(T, K, H);
     dim3 grid((unsigned)ceil_div(T, tile)), block(kTileThreads);
@@ -1011,10 +1048,10 @@ static int forward_one_launch(const void* x, const int32_t* indices, const float
 #define FWT3(EL, MD)                                                                                              \
   {                                                                                                               \
     switch (K) {                                                                                                  \
-      case 4: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 4>, grid, block, 0, stream, FWT_ARGS);  \
-      case 6: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 6>, grid, block, 0, stream, FWT_ARGS);  \
-      case 8: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 8>, grid, block, 0, stream, FWT_ARGS);  \
-      default: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 0>, grid, block, 0, stream, FWT_ARGS); \
+      case 4: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 4, 1>, grid, block, 0, stream, FWT_ARGS);  \
+      case 6: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 6, 1>, grid, block, 0, stream, FWT_ARGS);  \
+      case 8: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 8, 1>, grid, block, 0, stream, FWT_ARGS);  \
+      default: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 0, 1>, grid, block, 0, stream, FWT_ARGS); \
     }                                                                                                             \
   }
 #define FWT2(EL)                                                        \
@@ -1036,8 +1073,8 @@ static int forward_one_launch(const void* x, const int32_t* indices, const float
 #define FWD4(EPT, VPL, EL, MD)                                                                                   \
   {                                                                                                              \
     if (K == 8)                                                                                                  \
-      return launch(KID_FORWARD_TOKEN, forward_token_kernel<EPT, VPL, EL, MD, 8>, grid, block, 0, stream, FWD_ARGS); \
-    return launch(KID_FORWARD_TOKEN, forward_token_kernel<EPT, VPL, EL, MD, 0>, grid, block, 0, stream, FWD_ARGS); \
+      return launch(KID_FORWARD_TOKEN, forward_token_kernel<EPT, VPL, EL, MD, 8, 1>, grid, block, 0, stream, FWD_ARGS); \
+    return launch(KID_FORWARD_TOKEN, forward_token_kernel<EPT, VPL, EL, MD, 0, 1>, grid, block, 0, stream, FWD_ARGS); \
   }
 #define FWD3(EPT, VPL, EL)                                                      \
   {                                                                             \
@@ -1078,8 +1115,8 @@ static int forward_impl(const void* x, const int32_t* indices, const float* weig
   if (T > 0 && fuse_stub && fuse_route &&
       forward_one_launch_ok(T, K, H, max_recv, in_type, out_type, fp8_dispatch))
     return forward_one_launch(x, indices, weights, rank_start, src_rank, T, K, E, W, H, in_type, stub_kind,
-                              combine_mode, counts, offsets, slot_of_entry, src_of_slot, meta, status, disp, out,
-                              (hipStream_t)stream, clear_status);
+                              combine_mode, counts, offsets, slot_of_entry, src_of_slot, meta, status, disp,
+                              disp_scale, out, fp8_dispatch, (hipStream_t)stream, clear_status);
   if (T > 0 && fuse_stub && dispatch_fold_ok(T, K, H, max_recv, in_type, out_type, fp8_dispatch, fuse_route)) {
     if (int rc = route_impl(indices, rank_start, src_rank, T, K, E, W, max_recv, counts, offsets, slot_of_entry,
                             src_of_slot, meta, status, workspace, workspace_bytes, false, stream, clear_status))
