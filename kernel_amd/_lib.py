@@ -108,6 +108,23 @@ def load() -> C.CDLL:
     return lib
 
 
+_host_module = None
+
+
+def host():
+    """The extension module with the host side of ``forward`` (csrc/host_path.cpp)."""
+    global _host_module
+    if _host_module is None:
+        load()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError("kernel_amd/_host.so is missing or does not load: build it with "
+                               "`python -m kernel_amd.build` (there is no fallback path)") from e
+        _host_module = _host
+    return _host_module
+
+
 def check(code: int, where: str) -> None:
     if code != 0:
         raise MoeA2AError(code, where)

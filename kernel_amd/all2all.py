@@ -146,6 +146,7 @@ class HipAllToAll:
         self.lib = _lib.load()
         self._fused_max_rows = self.lib.moe_a2a_fused_max_rows()
         self._bufs = collections.OrderedDict()  # (T, device) -> two buffer sets; least recently used goes first
+        self._ring = None  # native side of the sets used last, once a forward has run on them (_host.Ring)
 
     # ---- buffers ---------------------------------------------------------------------
     def _buffers(self, T: int, device, advance: bool = False) -> dict:
@@ -161,9 +162,14 @@ class HipAllToAll:
         if ring is None:
             while len(self._bufs) >= self.MAX_CACHED_SHAPES:  # a caller with many token counts keeps the recent ones
                 self._bufs.popitem(last=False)
-            ring = self._bufs[key] = dict(sets=[None, None], cur=0)
+            ring = self._bufs[key] = dict(sets=[None, None], cur=0, native=None)
         else:
             self._bufs.move_to_end(key)
+        native = self._ring = ring["native"]
+        if native is not None:  # which set is next is kept there, where the short way of forward flips it too
+            if advance:
+                native.cur ^= 1
+            return ring["sets"][native.cur]
         if advance:
             ring["cur"] ^= 1
         b = ring["sets"][ring["cur"]]
@@ -207,6 +213,19 @@ class HipAllToAll:
 
     def release_buffers(self) -> None:
         self._bufs.clear()
+        self._ring = None
+
+    def _make_ring(self, T: int, device) -> None:
+        """The native side of the sets of T tokens: later calls of ``forward`` with that shape take it."""
+        ring = self._bufs[(T, device)]
+        if ring["native"] is None:
+            cfg, sets = self.cfg, ring["sets"]
+            blocks = [bytes(_lib.ForwardArgs(*self._forward_args(b, None, None, None, None, 0))) for b in sets]
+            ring["native"] = _lib.host().Ring(T, cfg.experts_per_token, cfg.hidden_dim, self.world_size, device.index,
+                                              cfg.in_dtype, cfg.out_dtype, *blocks, *(b["out"] for b in sets),
+                                              *(self._record(b, T) for b in sets))
+            ring["native"].cur = ring["cur"]
+        self._ring = ring["native"]
 
     # ---- dispatch --------------------------------------------------------------------
     def dispatch(self, dp_x: torch.Tensor, indices: torch.Tensor,
@@ -372,7 +391,7 @@ class HipAllToAll:
     # ---- whole path ------------------------------------------------------------------
     def _forward_args(self, b: dict, x, indices, weights, rank_start, stream: int) -> tuple:
         cfg = self.cfg
-        T, H = x.shape
+        T, H = b["out"].shape
         fuse_route = 2 if self.fuse_route == "always" else int(bool(self.fuse_route))
         return (_ptr(x), _ptr(indices), _ptr(weights), _ptr(rank_start), self.rank, T, cfg.experts_per_token,
                 cfg.num_experts, self.world_size, H, self.max_recv if self.padded else 0, _elem(cfg.in_dtype), _elem(cfg.out_dtype), 2 if self.fp8_dispatch == "pow2" else int(self.fp8_dispatch),
@@ -416,6 +435,12 @@ class HipAllToAll:
         a padded segment with more than ``max_recv`` rows (reference.py:140-146 would write past
         ``expert_x[local_eid]``).  Without it such ids are clamped and the bits stay in
         ``self.last.status`` until the next call."""
+        if self._ring is not None:  # the shape of the last call: None comes back for anything else
+            y = self._ring.forward(self, x, indices, weights, rank_start, out)
+            if y is not None:
+                if check_status:
+                    self.raise_on_status(self.last.status)
+                return y
         cfg = self.cfg
         T = x.shape[0]
         if T == 0:
@@ -426,29 +451,14 @@ class HipAllToAll:
             if out.dtype != cfg.out_dtype or out.dim() != 2 or out.shape[0] < T or out.shape[1] != cfg.hidden_dim:
                 raise ValueError("out must be out_dtype[>=T,H]")
         b = self._buffers(T, x.device, advance=True)
-        # the argument struct of a buffer set is built once; a call patches the caller's pointers in
-        a = b.get("_args")
-        if a is None:
-            a = b["_args"] = _lib.ForwardArgs(*self._forward_args(b, x, indices, weights, rank_start, 0))
-            b["_argp"] = ctypes.pointer(a)
-            b["_record"] = self._record(b, T)
-        a.x, a.indices, a.weights = x.data_ptr(), indices.data_ptr(), weights.data_ptr()
-        a.out = b["out"].data_ptr() if out is None else out.data_ptr()
-        # what rarely changes between two calls is written only when it does (a field of a foreign
-        # struct costs a quarter of a microsecond to set)
-        rs = None if rank_start is None else rank_start.data_ptr()
-        st = _stream(x.device.index)
-        switches = (rs, st, self.stub_kind, self.combine_mode, self.fuse_route, self.fuse_stub)
-        if b.get("_switches") != switches:
-            b["_switches"] = switches
-            a.rank_start, a.stream = rs, st
-            a.stub_kind, a.combine_mode = self.stub_kind, self.combine_mode
-            a.fuse_route = 2 if self.fuse_route == "always" else int(bool(self.fuse_route))
-            a.fuse_stub = int(self.fuse_stub)
-        rc = self.lib.moe_a2a_forward_packed(b["_argp"])
+        a = _lib.ForwardArgs(*self._forward_args(b, x, indices, weights, rank_start, _stream(x.device.index)))
+        if out is not None:
+            a.out = out.data_ptr()
+        rc = self.lib.moe_a2a_forward_packed(ctypes.byref(a))
         if rc:
             raise _lib.MoeA2AError(rc, "moe_a2a_forward")
-        self.last = b["_record"]
+        self.last = self._record(b, T)
+        self._make_ring(T, x.device)
         if check_status:
             self.raise_on_status(b["status"])
         return b["out"] if out is None else out

@@ -1,0 +1,418 @@
+// Host side of the one-call forward for Python callers: a CPython extension (kernel_amd._host).
+//
+// A call of the smallest tables takes the GPU four microseconds, and a launch costs the host two and a
+// half; checking the tensors, allocating the result and filling in the argument block from Python took
+// seven more (9.5 us per call of custom_kernel at 7 tokens).  Here the same steps read the tensors'
+// own C++ records.
+//
+//   Ring   the two alternating buffer sets of one token count: their argument blocks, the tensors a call hands
+//          out, and which set is next.  `forward` takes the caller's tensors, or returns None without side
+//          effects when anything about them is not as the argument blocks were built for (the caller then
+//          goes the long way, which raises the right error or builds the right ring).
+//   Memo   the configurations of recent custom_kernel calls and the host objects they belong to (one process
+//          may run every rank of a world in turn).
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <structmember.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstring>
+
+#include "moe_a2a.h"
+
+namespace {
+
+// interned attribute names
+PyObject *s_stub_kind, *s_combine_mode, *s_fuse_route, *s_fuse_stub, *s_last, *s_ring, *s_num_experts,
+    *s_experts_per_token, *s_hidden_dim, *s_max_num_tokens, *s_in_dtype, *s_out_dtype, *s_x, *s_indices, *s_weights,
+    *s_num_tokens, *s_always;
+
+struct Ref {  // owned reference
+  PyObject* p;
+  explicit Ref(PyObject* p_ = nullptr) : p(p_) {}
+  ~Ref() { Py_XDECREF(p); }
+  Ref(const Ref&) = delete;
+  Ref& operator=(const Ref&) = delete;
+  explicit operator bool() const { return p != nullptr; }
+};
+
+// integer attribute; false (with the error cleared) when it is missing or no integer
+bool int_attr(PyObject* o, PyObject* name, long& v) {
+  Ref a(PyObject_GetAttr(o, name));
+  if (!a) {
+    PyErr_Clear();
+    return false;
+  }
+  v = PyLong_AsLong(a.p);
+  if (v == -1 && PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
+struct Ring {
+  PyObject_HEAD
+  long T, K, H, W;
+  int device, cur;
+  at::ScalarType in_type, out_type;
+  moe_a2a_forward_args args[2];
+  PyObject* outs[2];
+  PyObject* records[2];
+};
+
+PyObject* ring_new(PyTypeObject* type, PyObject* args, PyObject*) {
+  long T, K, H, W;
+  int device;
+  PyObject *in_type, *out_type, *outs[2], *records[2];
+  const char* block[2];
+  Py_ssize_t len[2];
+  if (!PyArg_ParseTuple(args, "lllliO!O!y#y#OOOO", &T, &K, &H, &W, &device, &THPDtypeType, &in_type, &THPDtypeType,
+                        &out_type, &block[0], &len[0], &block[1], &len[1], &outs[0], &outs[1], &records[0],
+                        &records[1]))
+    return nullptr;
+  for (Py_ssize_t n : len)
+    if (n != (Py_ssize_t)sizeof(moe_a2a_forward_args)) {
+      PyErr_SetString(PyExc_ValueError, "an argument block is not a moe_a2a_forward_args");
+      return nullptr;
+    }
+  Ring* r = (Ring*)type->tp_alloc(type, 0);
+  if (!r) return nullptr;
+  r->T = T, r->K = K, r->H = H, r->W = W, r->device = device, r->cur = 0;
+  r->in_type = ((THPDtype*)in_type)->scalar_type;
+  r->out_type = ((THPDtype*)out_type)->scalar_type;
+  for (int i = 0; i < 2; ++i) {
+    std::memcpy(&r->args[i], block[i], sizeof(moe_a2a_forward_args));
+    Py_INCREF(outs[i]);
+    Py_INCREF(records[i]);
+    r->outs[i] = outs[i];
+    r->records[i] = records[i];
+  }
+  return (PyObject*)r;
+}
+
+int ring_clear(Ring* r) {
+  for (int i = 0; i < 2; ++i) {
+    Py_CLEAR(r->outs[i]);
+    Py_CLEAR(r->records[i]);
+  }
+  return 0;
+}
+int ring_traverse(Ring* r, visitproc visit, void* arg) {
+  for (int i = 0; i < 2; ++i) {
+    Py_VISIT(r->outs[i]);
+    Py_VISIT(r->records[i]);
+  }
+  return 0;
+}
+void ring_dealloc(Ring* r) {
+  PyObject_GC_UnTrack(r);
+  ring_clear(r);
+  Py_TYPE(r)->tp_free((PyObject*)r);
+}
+
+bool plain_matrix(const at::Tensor& t, at::ScalarType type, long rows, long cols, int device) {
+  return t.dim() == 2 && t.size(0) == rows && t.size(1) == cols && t.scalar_type() == type && t.is_contiguous() &&
+         t.is_cuda() && t.get_device() == device;
+}
+
+enum Outcome { kDone, kNotThisWay, kError };
+
+// One call on the next set; out: where the result goes (already checked).  Sets a Python error on kError.
+Outcome ring_forward(Ring* r, PyObject* owner, const at::Tensor& x, const at::Tensor& indices,
+                     const at::Tensor& weights, const at::Tensor* rank_start, void* out, int& set) {
+  if (!plain_matrix(x, r->in_type, r->T, r->H, r->device) ||
+      !plain_matrix(indices, at::kInt, r->T, r->K, r->device) ||
+      !plain_matrix(weights, at::kFloat, r->T, r->K, r->device))
+    return kNotThisWay;
+  if (rank_start && !(rank_start->scalar_type() == at::kInt && rank_start->numel() == r->W + 1 &&
+                      rank_start->is_contiguous() && rank_start->is_cuda() && rank_start->get_device() == r->device))
+    return kNotThisWay;
+  if (c10::hip::current_device() != r->device) return kNotThisWay;
+  // switches of the host object that may change between two calls
+  long stub_kind, combine_mode, fuse_route = 2;
+  if (!int_attr(owner, s_stub_kind, stub_kind) || !int_attr(owner, s_combine_mode, combine_mode)) return kNotThisWay;
+  Ref route(PyObject_GetAttr(owner, s_fuse_route)), stub(PyObject_GetAttr(owner, s_fuse_stub));
+  if (!route || !stub) {
+    PyErr_Clear();
+    return kNotThisWay;
+  }
+  if (route.p == Py_True || route.p == Py_False)
+    fuse_route = route.p == Py_True;
+  else if (!PyUnicode_Check(route.p) || PyUnicode_Compare(route.p, s_always) != 0)
+    return kNotThisWay;
+  if (stub.p != Py_True && stub.p != Py_False) return kNotThisWay;
+  set = r->cur ^= 1;
+  moe_a2a_forward_args a = r->args[set];  // a copy: the launch runs without the interpreter's lock
+  a.x = x.const_data_ptr();
+  a.indices = (const int32_t*)indices.const_data_ptr();
+  a.weights = (const float*)weights.const_data_ptr();
+  a.rank_start = rank_start ? (const int32_t*)rank_start->const_data_ptr() : nullptr;
+  if (out) a.out = out;
+  a.stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)r->device).stream();
+  a.stub_kind = (int)stub_kind;
+  a.combine_mode = (int)combine_mode;
+  a.fuse_route = (int)fuse_route;
+  a.fuse_stub = stub.p == Py_True;
+  PyObject* record = r->records[set];
+  Py_INCREF(record);
+  int rc;
+  Py_BEGIN_ALLOW_THREADS;
+  rc = moe_a2a_forward_packed(&a);
+  Py_END_ALLOW_THREADS;
+  if (rc != 0) {
+    Py_DECREF(record);
+    Ref lib(PyImport_ImportModule("kernel_amd._lib"));  // raises MoeA2AError
+    Ref raised(lib ? PyObject_CallMethod(lib.p, "check", "is", rc, "moe_a2a_forward") : nullptr);
+    return kError;
+  }
+  const int bad = PyObject_SetAttr(owner, s_last, record);
+  Py_DECREF(record);
+  return bad ? kError : kDone;
+}
+
+// forward(owner, x, indices, weights, rank_start or None, out or None) -> y, or None: not this way
+PyObject* ring_forward_py(Ring* r, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 6) {
+    PyErr_SetString(PyExc_TypeError, "forward takes owner, x, indices, weights, rank_start, out");
+    return nullptr;
+  }
+  for (int i = 1; i < 6; ++i)
+    if (!THPVariable_Check(args[i]) && !(i >= 4 && args[i] == Py_None)) Py_RETURN_NONE;
+  const at::Tensor* rank_start = args[4] == Py_None ? nullptr : &THPVariable_Unpack(args[4]);
+  void* out = nullptr;
+  if (args[5] != Py_None) {
+    const at::Tensor& o = THPVariable_Unpack(args[5]);
+    if (o.dim() != 2 || o.size(0) < r->T || !plain_matrix(o, r->out_type, o.size(0), r->H, r->device)) Py_RETURN_NONE;
+    out = o.data_ptr();
+  }
+  int set = 0;
+  switch (ring_forward(r, args[0], THPVariable_Unpack(args[1]), THPVariable_Unpack(args[2]), THPVariable_Unpack(args[3]),
+                       rank_start, out, set)) {
+    case kNotThisWay: Py_RETURN_NONE;
+    case kError: return nullptr;
+    case kDone: break;
+  }
+  PyObject* y = out ? args[5] : r->outs[set];
+  Py_INCREF(y);
+  return y;
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef ring_methods[] = {
+    {"forward", (PyCFunction)(void (*)(void))ring_forward_py, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyMemberDef ring_members[] = {{"cur", T_INT, offsetof(Ring, cur), 0, nullptr}, {nullptr, 0, 0, 0, nullptr}};
+PyTypeObject RingType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ---------------------------------------------------------------------------------------
+constexpr int kMemoEntries = 16;
+struct MemoEntry {
+  long config[4], call[4];  // call: rank, world_size, stub_kind, combine_mode
+  PyObject *in_dtype, *out_dtype, *owner;
+};
+struct Memo {
+  PyObject_HEAD
+  int used;
+  MemoEntry entry[kMemoEntries];  // most recently used first
+};
+void entry_drop(MemoEntry& e) {
+  Py_CLEAR(e.in_dtype);
+  Py_CLEAR(e.out_dtype);
+  Py_CLEAR(e.owner);
+}
+// entry i becomes the first
+void entry_front(Memo* m, int i) {
+  if (i == 0) return;
+  const MemoEntry e = m->entry[i];
+  std::memmove(&m->entry[1], &m->entry[0], i * sizeof(MemoEntry));
+  m->entry[0] = e;
+}
+
+// what custom_kernel's instance depends on, read from the config record at every call
+bool memo_read(PyObject* cfg, long (&v)[4], Ref& in_dtype, Ref& out_dtype) {
+  if (!int_attr(cfg, s_num_experts, v[0]) || !int_attr(cfg, s_experts_per_token, v[1]) ||
+      !int_attr(cfg, s_hidden_dim, v[2]) || !int_attr(cfg, s_max_num_tokens, v[3]))
+    return false;
+  in_dtype.p = PyObject_GetAttr(cfg, s_in_dtype);
+  out_dtype.p = PyObject_GetAttr(cfg, s_out_dtype);
+  if (!in_dtype || !out_dtype) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
+// the entry of these values, or -1
+int memo_find(const Memo* m, const long (&config)[4], const long (&call)[4], const PyObject* in_dtype,
+              const PyObject* out_dtype) {
+  for (int i = 0; i < m->used; ++i) {
+    const MemoEntry& e = m->entry[i];
+    if (std::memcmp(e.call, call, sizeof(call)) == 0 && std::memcmp(e.config, config, sizeof(config)) == 0 &&
+        e.in_dtype == in_dtype && e.out_dtype == out_dtype)
+      return i;
+  }
+  return -1;
+}
+
+// remember(cfg, rank, world_size, stub_kind, combine_mode, owner)
+PyObject* memo_remember(Memo* m, PyObject* const* args, Py_ssize_t n) {
+  if (n != 6) {
+    PyErr_SetString(PyExc_TypeError, "remember takes cfg, rank, world_size, stub_kind, combine_mode, owner");
+    return nullptr;
+  }
+  MemoEntry fresh;
+  for (int i = 0; i < 4; ++i) {
+    fresh.call[i] = PyLong_AsLong(args[1 + i]);
+    if (fresh.call[i] == -1 && PyErr_Occurred()) {
+      PyErr_Clear();
+      Py_RETURN_NONE;
+    }
+  }
+  Ref in_dtype, out_dtype;
+  if (!memo_read(args[0], fresh.config, in_dtype, out_dtype)) Py_RETURN_NONE;
+  int at = memo_find(m, fresh.config, fresh.call, in_dtype.p, out_dtype.p);
+  if (at < 0) {
+    if (m->used < kMemoEntries) {
+      at = m->used++;
+    } else {
+      at = kMemoEntries - 1;  // the one not used for longest
+      entry_drop(m->entry[at]);
+    }
+    fresh.in_dtype = in_dtype.p;
+    fresh.out_dtype = out_dtype.p;
+    fresh.owner = nullptr;
+    in_dtype.p = out_dtype.p = nullptr;
+    m->entry[at] = fresh;
+  }
+  Py_INCREF(args[5]);
+  Py_XSETREF(m->entry[at].owner, args[5]);
+  entry_front(m, at);
+  Py_RETURN_NONE;
+}
+
+// run(data, stub_kind, combine_mode) -> y, or None: not this way
+PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 3) {
+    PyErr_SetString(PyExc_TypeError, "run takes data, stub_kind, combine_mode");
+    return nullptr;
+  }
+  if (!PyTuple_CheckExact(args[0]) || PyTuple_GET_SIZE(args[0]) != 4) Py_RETURN_NONE;
+  long call[4];
+  PyObject* given[4] = {PyTuple_GET_ITEM(args[0], 2), PyTuple_GET_ITEM(args[0], 3), args[1], args[2]};
+  for (int i = 0; i < 4; ++i) {
+    call[i] = PyLong_CheckExact(given[i]) ? PyLong_AsLong(given[i]) : -1;
+    if (call[i] < 0) {
+      PyErr_Clear();
+      Py_RETURN_NONE;
+    }
+  }
+  long config[4];
+  Ref in_dtype, out_dtype;
+  if (!memo_read(PyTuple_GET_ITEM(args[0], 0), config, in_dtype, out_dtype)) Py_RETURN_NONE;
+  const int at = memo_find(m, config, call, in_dtype.p, out_dtype.p);
+  if (at < 0) Py_RETURN_NONE;
+  entry_front(m, at);
+  PyObject* rank_data = PyTuple_GET_ITEM(args[0], 1);
+  long num_tokens;
+  Ref x(PyObject_GetAttr(rank_data, s_x)), indices(PyObject_GetAttr(rank_data, s_indices)),
+      weights(PyObject_GetAttr(rank_data, s_weights)), owner(nullptr), ring(nullptr);
+  if (!x || !indices || !weights || !int_attr(rank_data, s_num_tokens, num_tokens) || !THPVariable_Check(x.p) ||
+      !THPVariable_Check(indices.p) || !THPVariable_Check(weights.p)) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  Py_INCREF(m->entry[0].owner);
+  owner.p = m->entry[0].owner;
+  ring.p = PyObject_GetAttr(owner.p, s_ring);
+  if (!ring || Py_TYPE(ring.p) != &RingType) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  Ring* r = (Ring*)ring.p;
+  const at::Tensor& xt = THPVariable_Unpack(x.p);
+  if (num_tokens < 0 || num_tokens > r->T || !plain_matrix(xt, r->in_type, r->T, r->H, r->device)) Py_RETURN_NONE;
+  // the caller owns its result: the combine writes straight into a fresh tensor
+  at::Tensor y = at::empty({r->T, r->H}, xt.options().dtype(r->out_type));
+  int set = 0;
+  switch (ring_forward(r, owner.p, xt, THPVariable_Unpack(indices.p), THPVariable_Unpack(weights.p), nullptr, y.data_ptr(),
+                       set)) {
+    case kNotThisWay: Py_RETURN_NONE;
+    case kError: return nullptr;
+    case kDone: break;
+  }
+  return THPVariable_Wrap(num_tokens == r->T ? y : y.narrow(0, 0, num_tokens));
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* memo_new(PyTypeObject* type, PyObject*, PyObject*) { return type->tp_alloc(type, 0); }
+int memo_clear(Memo* m) {
+  while (m->used > 0) entry_drop(m->entry[--m->used]);
+  return 0;
+}
+int memo_traverse(Memo* m, visitproc visit, void* arg) {
+  for (int i = 0; i < m->used; ++i) Py_VISIT(m->entry[i].owner);
+  return 0;
+}
+void memo_dealloc(Memo* m) {
+  PyObject_GC_UnTrack(m);
+  memo_clear(m);
+  Py_TYPE(m)->tp_free((PyObject*)m);
+}
+PyMethodDef memo_methods[] = {{"remember", (PyCFunction)(void (*)(void))memo_remember, METH_FASTCALL, nullptr},
+                              {"run", (PyCFunction)(void (*)(void))memo_run, METH_FASTCALL, nullptr},
+                              {nullptr, nullptr, 0, nullptr}};
+PyTypeObject MemoType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, nullptr, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) {
+  struct {
+    PyObject*& var;
+    const char* text;
+  } names[] = {{s_stub_kind, "stub_kind"},     {s_combine_mode, "combine_mode"},
+               {s_fuse_route, "fuse_route"},   {s_fuse_stub, "fuse_stub"},
+               {s_last, "last"},               {s_ring, "_ring"},
+               {s_num_experts, "num_experts"}, {s_experts_per_token, "experts_per_token"},
+               {s_hidden_dim, "hidden_dim"},   {s_max_num_tokens, "max_num_tokens"},
+               {s_in_dtype, "in_dtype"},       {s_out_dtype, "out_dtype"},
+               {s_x, "x"},                     {s_indices, "indices"},
+               {s_weights, "weights"},         {s_num_tokens, "num_tokens"},
+               {s_always, "always"}};
+  for (auto& name : names)
+    if (!(name.var = PyUnicode_InternFromString(name.text))) return nullptr;
+  RingType.tp_name = "kernel_amd._host.Ring";
+  RingType.tp_basicsize = sizeof(Ring);
+  RingType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  RingType.tp_new = ring_new;
+  RingType.tp_dealloc = (destructor)ring_dealloc;
+  RingType.tp_traverse = (traverseproc)ring_traverse;
+  RingType.tp_clear = (inquiry)ring_clear;
+  RingType.tp_methods = ring_methods;
+  RingType.tp_members = ring_members;
+  MemoType.tp_name = "kernel_amd._host.Memo";
+  MemoType.tp_basicsize = sizeof(Memo);
+  MemoType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  MemoType.tp_new = memo_new;
+  MemoType.tp_dealloc = (destructor)memo_dealloc;
+  MemoType.tp_traverse = (traverseproc)memo_traverse;
+  MemoType.tp_clear = (inquiry)memo_clear;
+  MemoType.tp_methods = memo_methods;
+  if (PyType_Ready(&RingType) < 0 || PyType_Ready(&MemoType) < 0) return nullptr;
+  PyObject* m = PyModule_Create(&module);
+  if (!m) return nullptr;
+  Py_INCREF(&RingType);
+  Py_INCREF(&MemoType);
+  if (PyModule_AddObject(m, "Ring", (PyObject*)&RingType) < 0 || PyModule_AddObject(m, "Memo", (PyObject*)&MemoType) < 0)
+    return nullptr;
+  return m;
+}

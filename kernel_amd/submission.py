@@ -10,11 +10,13 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib
 from .all2all import HipAllToAll
 from .contract import COMBINE_STRICT, STUB_OWNER_RANK
 
 _instances = {}
 _last = [None, None]  # key and instance of the previous call (a harness calls with one config many times)
+_memo = None  # the same for the native side (_host.Memo), which runs a call that repeats the previous configuration
 
 
 def _instance(cfg, rank: int, world_size: int, device, stub_kind: int, combine_mode: int) -> HipAllToAll:
@@ -45,6 +47,11 @@ def custom_kernel(data, stub_kind: int = STUB_OWNER_RANK, combine_mode: int = CO
     """``check_status=True`` reads the routing status back after the call (one synchronisation) and
     raises where the reference would: ``IndexError`` for an expert id outside ``[0, num_experts)``
     (``token_map[dst_rank]``, reference.py:81-86)."""
+    global _memo
+    if _memo is not None and not check_status:
+        y = _memo.run(data, stub_kind, combine_mode)
+        if y is not None:
+            return y
     cfg, rank_data, rank, world_size = data
     x = rank_data.x
     if not x.is_cuda:
@@ -62,5 +69,8 @@ def custom_kernel(data, stub_kind: int = STUB_OWNER_RANK, combine_mode: int = CO
     else:
         with torch.cuda.device(x.device):
             ata.forward(x, idx, w, out=y, check_status=check_status)
+    if _memo is None:
+        _memo = _lib.host().Memo()
+    _memo.remember(cfg, rank, world_size, stub_kind, combine_mode, ata)
     n = rank_data.num_tokens
     return y if n == T else y[:n]

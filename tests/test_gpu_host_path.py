@@ -1,0 +1,82 @@
+"""The native side of custom_kernel and forward: what it takes over, what it leaves to the long way."""
+import copy
+
+import pytest
+import torch
+
+from kernel_amd import contract as C
+from kernel_amd.all2all import HipAllToAll
+from kernel_amd.submission import custom_kernel
+from oracle import all2all_vec as V
+
+pytestmark = pytest.mark.gpu
+
+
+def case(rank, T, dtype=torch.bfloat16, E=16, K=2, H=256):
+    g = torch.Generator().manual_seed(100 * rank + T)
+    cfg = C.MoEConfig(E, K, H, 64, dtype, dtype)
+    idx = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(T)]).to(torch.int32)
+    rd = C.RankData(T, idx, torch.rand(T, K, generator=g), torch.randn(T, H, generator=g).to(dtype))
+    want = V.run_world(cfg, C.world_of_single_rank(cfg, rd, rank, 8), stub_kind=C.STUB_OWNER_RANK)["y"]
+    return cfg, rd.to("cuda:0"), rank, want
+
+
+def same(y, want):
+    return torch.equal(y.cpu().view(torch.int16), want.view(torch.int16))
+
+
+def test_more_configurations_in_turn_than_are_remembered(gpu_device):
+    cases = [case(r, T, dt) for r in range(8) for T in (5, 9) for dt in (torch.bfloat16, torch.float16)]  # 16 keys, two shapes each
+    for _ in range(3):
+        for cfg, rd, rank, want in cases:
+            assert same(custom_kernel((copy.copy(cfg), rd, rank, 8)), want)
+    one = cases[0]
+    ys = [custom_kernel((one[0], one[1], one[2], 8)) for _ in range(5)]
+    assert len({y.data_ptr() for y in ys}) == 5 and all(same(y, one[3]) for y in ys)  # every result is the caller's own
+
+
+def test_what_the_short_way_does_not_take(gpu_device):
+    cfg, rd, rank, want = case(3, 12)
+    for _ in range(2):
+        assert same(custom_kernel((cfg, rd, rank, 8)), want)
+    part = C.RankData(7, rd.indices, rd.weights, rd.x)  # fewer tokens asked for than there are rows
+    assert same(custom_kernel((cfg, part, rank, 8)), want[:7])
+    strided = C.RankData(12, rd.indices, rd.weights, torch.cat([rd.x, rd.x], 1)[:, : rd.x.shape[1]])
+    assert not strided.x.is_contiguous() and same(custom_kernel((cfg, strided, rank, 8)), want)
+    for bad in (C.RankData(12, rd.indices.long(), rd.weights, rd.x), C.RankData(12, rd.indices, rd.weights.double(), rd.x),
+                C.RankData(12, rd.indices[:, :1].contiguous(), rd.weights, rd.x)):
+        with pytest.raises(ValueError):
+            custom_kernel((cfg, bad, rank, 8))
+    with pytest.raises(RuntimeError):
+        custom_kernel((cfg, C.RankData(12, rd.indices.cpu(), rd.weights, rd.x), rank, 8))
+    assert same(custom_kernel((cfg, rd, rank, 8)), want)
+    changed = copy.copy(cfg)
+    custom_kernel((changed, rd, rank, 8))
+    changed.experts_per_token = 1  # in place, between two calls
+    with pytest.raises(ValueError):
+        custom_kernel((changed, rd, rank, 8))
+
+
+def test_switches_streams_and_phases_between_forwards(gpu_device):
+    cfg, rd, rank, _ = case(0, 20)
+    ata = HipAllToAll(cfg, 0, 8, fuse_stub=True)
+    cpu = rd.to("cpu")
+    want = {(s, m): V.run_world(cfg, C.world_of_single_rank(cfg, cpu, 0, 8), stub_kind=s, combine_mode=m)["y"]
+            for s in (C.STUB_OWNER_RANK, C.STUB_EXPERT_FRACTION) for m in (C.COMBINE_STRICT, C.COMBINE_F32)}
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(2):
+        for (s, m), y in want.items():
+            ata.stub_kind, ata.combine_mode = s, m
+            assert same(ata.forward(rd.x, rd.indices, rd.weights), y)
+            d = ata.dispatch(rd.x, rd.indices)  # flips the sets, in between
+            assert d.disp_x.data_ptr() != ata.last.disp_x.data_ptr()
+            with torch.cuda.stream(side):
+                got = ata.forward(rd.x, rd.indices, rd.weights)
+            side.synchronize()
+            assert same(got, y) and ata.last.disp_x.data_ptr() != d.disp_x.data_ptr()
+    bad = rd.indices.clone()
+    bad[4, 1] = cfg.num_experts
+    with pytest.raises(IndexError):
+        ata.forward(rd.x, bad, rd.weights, check_status=True)
+    assert ata.forward(rd.x[:6], rd.indices[:6], rd.weights[:6]).shape[0] == 6
