@@ -484,3 +484,27 @@ def test_eight_wave_tile_walk_on_odd_segment_tables(gpu_device, options, name, c
         want = V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False)
     torch.cuda.synchronize()
     close(y, want)
+
+
+@pytest.mark.parametrize("early", [False, True], ids=["late-b", "early-b"])
+@pytest.mark.parametrize("H,N", [(256, 256), (384, 640), (1408, 128)])  # two, three and eleven slabs; half a tile
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_expert_gemm_f32_scales_wide_tiles(gpu_device, options, dtype, H, N, early):
+    """fp8 rows and weights with f32 scales on 256 x 256 tiles: segments of 1 row, at, below and above a wave's half
+    (64 rows), a wave (128), 192 and a tile (256), and several tiles.  The partial sums are folded block by block in the
+    order of the 256 x 128 tiles: the same bits, and the f32 matmul within the tolerance of the other forms."""
+    counts = [1, 64, 65, 0, 127, 128, 129, 192, 193, 255, 256, 257, 0, 700, 5]
+    cfg, world, weights = make_counts(counts, H, N, dtype, seed=H + N)
+    wq, ws = V.quantize_weights_fp8(weights)
+    x, idx, w, rs = concat_world(world, gpu_device)
+    ata = HipAllToAll(cfg, 0, 1, fp8_dispatch=True)
+    d = ata.dispatch(x, idx, rs)
+    options.set("GEMM_TILE", 128)
+    options.set("GEMM_STAGED", 3 if early else 4)
+    y = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device)).clone()
+    options.set("GEMM_STAGED", 5)
+    y_narrow = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device))
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), y_narrow.view(torch.int16))
+    o = V.run_world(cfg, world, fp8=True)
+    close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
