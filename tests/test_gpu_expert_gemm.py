@@ -508,3 +508,26 @@ def test_expert_gemm_f32_scales_wide_tiles(gpu_device, options, dtype, H, N, ear
     assert torch.equal(y.view(torch.int16), y_narrow.view(torch.int16))
     o = V.run_world(cfg, world, fp8=True)
     close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
+
+
+TALL_COUNTS = [1, 255, 256, 257, 0, 272, 273, 287, 288, 289, 512, 513, 544, 545, 576, 577, 864, 865]
+
+
+@pytest.mark.parametrize("H,N", [(192, 256), (256, 640), (320, 200)])  # N: one tile, a ragged last one, less than one
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_expert_gemm_16bit_tall_tiles(gpu_device, options, dtype, H, N):
+    """Segments at and around the lengths where tiles of 288 rows save one of 256: every 16-bit kernel walks K in the
+    same order, so the 128 x 128 tiles give the same bits."""
+    cfg, world, weights = make_counts(TALL_COUNTS, H, N, dtype, seed=H + N)
+    x, idx, w, rs = concat_world(world, gpu_device)
+    ata = HipAllToAll(cfg, 0, 1)
+    d = ata.dispatch(x, idx, rs)
+    options.set("GEMM_TILE", 256)
+    options.set("GEMM_STAGED", 4)
+    y = ata.expert_gemm(d, weights.to(gpu_device)).clone()
+    options.set("GEMM_TILE", 128)
+    y_small = ata.expert_gemm(d, weights.to(gpu_device))
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), y_small.view(torch.int16))
+    o = V.run_world(cfg, world)
+    close(y, V.expert_gemm(o["disp_x"], o["offsets"], weights, dtype))
