@@ -531,3 +531,24 @@ def test_expert_gemm_16bit_tall_tiles(gpu_device, options, dtype, H, N):
     assert torch.equal(y.view(torch.int16), y_small.view(torch.int16))
     o = V.run_world(cfg, world)
     close(y, V.expert_gemm(o["disp_x"], o["offsets"], weights, dtype))
+
+
+@pytest.mark.parametrize("H,N", [(256, 256), (384, 640), (1408, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_expert_gemm_power_of_two_tall_tiles(gpu_device, options, dtype, H, N):
+    """The same segments through the kernel with power-of-two scales, with the same bits as its form for short segments,
+    which has tiles of 256 rows only."""
+    cfg, world, weights = make_counts(TALL_COUNTS, H, N, dtype, seed=H + N)
+    wq, ws = V.quantize_weights_fp8(weights, pow2=True)
+    x, idx, w, rs = concat_world(world, gpu_device)
+    ata = HipAllToAll(cfg, 0, 1, fp8_dispatch="pow2")
+    d = ata.dispatch(x, idx, rs)
+    options.set("GEMM_TILE", 256)
+    options.set("GEMM_STAGED", 4)
+    y = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device), scales_pow2=True).clone()
+    options.set("GEMM_STAGED", 3)
+    y_short = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device), scales_pow2=True)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), y_short.view(torch.int16))
+    o = V.run_world(cfg, world, fp8=True, pow2=True)
+    close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
