@@ -320,17 +320,17 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
   const int at = memo_find(m, config, call, in_dtype.p, out_dtype.p);
   if (at < 0) Py_RETURN_NONE;
   entry_front(m, at);
+  Ref owner(m->entry[0].owner), ring(nullptr);  // taken here: the lookups below may run Python code, and other threads
+  Py_INCREF(owner.p);
   PyObject* rank_data = PyTuple_GET_ITEM(args[0], 1);
   long num_tokens;
   Ref x(PyObject_GetAttr(rank_data, s_x)), indices(PyObject_GetAttr(rank_data, s_indices)),
-      weights(PyObject_GetAttr(rank_data, s_weights)), owner(nullptr), ring(nullptr);
+      weights(PyObject_GetAttr(rank_data, s_weights));
   if (!x || !indices || !weights || !int_attr(rank_data, s_num_tokens, num_tokens) || !THPVariable_Check(x.p) ||
       !THPVariable_Check(indices.p) || !THPVariable_Check(weights.p)) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
-  Py_INCREF(m->entry[0].owner);
-  owner.p = m->entry[0].owner;
   ring.p = PyObject_GetAttr(owner.p, s_ring);
   if (!ring || Py_TYPE(ring.p) != &RingType) {
     PyErr_Clear();
