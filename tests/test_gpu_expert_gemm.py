@@ -6,6 +6,7 @@ The summation order differs from torch's, so the comparison is a tolerance, stat
 import pytest
 import torch
 
+from kernel_amd import _lib
 from kernel_amd import contract as C
 from kernel_amd.all2all import HipAllToAll, concat_world
 from oracle import all2all_vec as V
@@ -552,3 +553,22 @@ def test_expert_gemm_power_of_two_tall_tiles(gpu_device, options, dtype, H, N):
     assert torch.equal(y.view(torch.int16), y_short.view(torch.int16))
     o = V.run_world(cfg, world, fp8=True, pow2=True)
     close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
+
+
+@pytest.mark.parametrize("Kd", [3728256, 3728320, 4194240])  # the longest rows of a tall tile, one slab more, and more
+def test_expert_gemm_16bit_longest_rows(gpu_device, Kd):
+    """One segment of 288 rows so long that a tile's offsets come to the end of 32 bits: the sum of every row, the last
+    32 among them, whatever tile they fall to.  Tolerance: one rounding to bf16 (2^-9 of a value) and the f32 sum of
+    Kd products of variance 1 / Kd in any order, whose error stays below sqrt(Kd) * 2^-24 * 4 = 5e-4."""
+    R, N = 288, 256
+    gen = torch.Generator(device=gpu_device).manual_seed(Kd)
+    x = torch.empty(R, Kd, dtype=torch.bfloat16, device=gpu_device).normal_(generator=gen)
+    w = torch.empty(N, Kd, dtype=torch.bfloat16, device=gpu_device).normal_(0.0, Kd ** -0.5, generator=gen)
+    offsets = torch.tensor([0, R], dtype=torch.int32, device=gpu_device)
+    y = torch.empty(R, N, dtype=torch.bfloat16, device=gpu_device)
+    _lib.check(_lib.load().moe_a2a_expert_gemm(x.data_ptr(), w.data_ptr(), offsets.data_ptr(), y.data_ptr(), R, 1, Kd, N, 0,
+                                               _lib.BF16, torch.cuda.current_stream().cuda_stream), "moe_a2a_expert_gemm")
+    want = torch.zeros(R, N, dtype=torch.float64, device=gpu_device)
+    for k in range(0, Kd, 1 << 16):
+        want += (x[:, k:k + (1 << 16)].float() @ w[:, k:k + (1 << 16)].float().T).double()
+    assert bool(((y.double() - want).abs() <= want.abs() * 2 ** -8 + 5e-4).all())
