@@ -17,7 +17,6 @@ torch is used for device memory and the current stream only.
 """
 from __future__ import annotations
 
-import collections
 import copy
 import ctypes
 import dataclasses
@@ -145,8 +144,9 @@ class HipAllToAll:
         self.fuse_stub = fuse_stub
         self.lib = _lib.load()
         self._fused_max_rows = self.lib.moe_a2a_fused_max_rows()
-        self._bufs = collections.OrderedDict()  # (T, device) -> two buffer sets; least recently used goes first
-        self._ring = None  # native side of the sets used last, once a forward has run on them (_host.Ring)
+        # (T, device) -> two buffer sets and their native record (_host.Ring: which is next, when they were used last)
+        self._bufs = {}
+        self._rings = _lib.host().Rings()  # those records, where the short way of forward finds them
 
     # ---- buffers ---------------------------------------------------------------------
     def _buffers(self, T: int, device, advance: bool = False) -> dict:
@@ -157,31 +157,30 @@ class HipAllToAll:
         step never writes what the step before it read; it also means the result of a call
         stays valid until the second-next call.
         """
-        key = (T, device)
-        ring = self._bufs.get(key)
-        if ring is None:
-            while len(self._bufs) >= self.MAX_CACHED_SHAPES:  # a caller with many token counts keeps the recent ones
-                self._bufs.popitem(last=False)
-            ring = self._bufs[key] = dict(sets=[None, None], cur=0, native=None)
-        else:
-            self._bufs.move_to_end(key)
-        native = self._ring = ring["native"]
-        if native is not None:  # which set is next is kept there, where the short way of forward flips it too
-            if advance:
-                native.cur ^= 1
-            return ring["sets"][native.cur]
+        ring = self._bufs.get((T, device)) or self._new_ring(T, device)
+        native, sets = ring["native"], ring["sets"]
+        self._rings.touch(native)
         if advance:
-            ring["cur"] ^= 1
-        b = ring["sets"][ring["cur"]]
-        if b is not None:
-            return b
-        # both sets of a new shape are allocated together, so that the second call with this shape
-        # does not meet an allocation either
-        for i in (0, 1):
-            ring["sets"][i] = self._allocate(T, device)
-        for i in (0, 1):  # a call on one set clears the status word of the other (see Dispatched.status)
-            ring["sets"][i]["partner_status"] = ring["sets"][i ^ 1]["status"]
-        return ring["sets"][ring["cur"]]
+            native.cur ^= 1
+        if sets[0] is None:
+            # both sets of a new shape are allocated together, so that the second call with this shape
+            # does not meet an allocation either
+            fresh = [self._allocate(T, device), self._allocate(T, device)]
+            for i in (0, 1):  # a call on one set clears the status word of the other (see Dispatched.status)
+                fresh[i]["partner_status"] = fresh[i ^ 1]["status"]
+            sets[:] = fresh
+        return sets[native.cur]
+
+    def _new_ring(self, T: int, device) -> dict:
+        while len(self._bufs) >= self.MAX_CACHED_SHAPES:  # a caller with many token counts keeps the recent ones
+            oldest = min(self._bufs, key=lambda key: self._bufs[key]["native"].used)
+            self._rings.drop(self._bufs.pop(oldest)["native"])
+        cfg = self.cfg
+        native = _lib.host().Ring(T, cfg.experts_per_token, cfg.hidden_dim, self.world_size, device.index, cfg.in_dtype,
+                                  cfg.out_dtype)
+        self._rings.add(native)
+        ring = self._bufs[(T, device)] = dict(sets=[None, None], native=native)
+        return ring
 
     def _allocate(self, T: int, device) -> dict:
         cfg = self.cfg
@@ -213,19 +212,18 @@ class HipAllToAll:
 
     def release_buffers(self) -> None:
         self._bufs.clear()
-        self._ring = None
+        self._rings.clear()
 
-    def _make_ring(self, T: int, device) -> None:
-        """The native side of the sets of T tokens: later calls of ``forward`` with that shape take it."""
+    def _bind(self, T: int, device) -> None:
+        """Gives the native record of T tokens what ``forward`` needs of the set that comes next: calls that meet that
+        set again go the short way."""
+        self._buffers(T, device)
         ring = self._bufs[(T, device)]
-        if ring["native"] is None:
-            cfg, sets = self.cfg, ring["sets"]
-            blocks = [bytes(_lib.ForwardArgs(*self._forward_args(b, None, None, None, None, 0))) for b in sets]
-            ring["native"] = _lib.host().Ring(T, cfg.experts_per_token, cfg.hidden_dim, self.world_size, device.index,
-                                              cfg.in_dtype, cfg.out_dtype, *blocks, *(b["out"] for b in sets),
-                                              *(self._record(b, T) for b in sets))
-            ring["native"].cur = ring["cur"]
-        self._ring = ring["native"]
+        native, i = ring["native"], ring["native"].cur ^ 1
+        if not native.bound >> i & 1:
+            b = ring["sets"][i]
+            block = bytes(_lib.ForwardArgs(*self._forward_args(b, None, None, None, None, 0)))
+            native.bind(i, block, b["out"], self._record(b, T))
 
     # ---- dispatch --------------------------------------------------------------------
     def dispatch(self, dp_x: torch.Tensor, indices: torch.Tensor,
@@ -435,21 +433,27 @@ class HipAllToAll:
         a padded segment with more than ``max_recv`` rows (reference.py:140-146 would write past
         ``expert_x[local_eid]``).  Without it such ids are clamped and the bits stay in
         ``self.last.status`` until the next call."""
-        if self._ring is not None:  # the shape of the last call: None comes back for anything else
-            y = self._ring.forward(self, x, indices, weights, rank_start, out)
-            if y is not None:
-                if check_status:
-                    self.raise_on_status(self.last.status)
-                return y
-        cfg = self.cfg
+        y = self._rings.forward(self, x, indices, weights, rank_start, out)
+        if y is None:  # not a shape of an earlier call
+            T = x.shape[0]
+            if T == 0:
+                return torch.empty(0, self.cfg.hidden_dim, dtype=self.cfg.out_dtype, device=x.device)
+            self._check_inputs(x, indices, weights, rank_start)
+            if out is not None:
+                _require_gpu(out, "out")
+                if out.dtype != self.cfg.out_dtype or out.dim() != 2 or out.shape[0] < T \
+                        or out.shape[1] != self.cfg.hidden_dim:
+                    raise ValueError("out must be out_dtype[>=T,H]")
+            self._bind(T, x.device)
+            y = self._rings.forward(self, x, indices, weights, rank_start, out)
+            if y is None:  # another device is the current one, or a switch is of a kind that only Python reads
+                y = self._forward_from_python(x, indices, weights, rank_start, out)
+        if check_status:
+            self.raise_on_status(self.last.status)
+        return y
+
+    def _forward_from_python(self, x, indices, weights, rank_start, out) -> torch.Tensor:
         T = x.shape[0]
-        if T == 0:
-            return torch.empty(0, cfg.hidden_dim, dtype=cfg.out_dtype, device=x.device)
-        self._check_inputs(x, indices, weights, rank_start)
-        if out is not None:
-            _require_gpu(out, "out")
-            if out.dtype != cfg.out_dtype or out.dim() != 2 or out.shape[0] < T or out.shape[1] != cfg.hidden_dim:
-                raise ValueError("out must be out_dtype[>=T,H]")
         b = self._buffers(T, x.device, advance=True)
         a = _lib.ForwardArgs(*self._forward_args(b, x, indices, weights, rank_start, _stream(x.device.index)))
         if out is not None:
@@ -458,9 +462,6 @@ class HipAllToAll:
         if rc:
             raise _lib.MoeA2AError(rc, "moe_a2a_forward")
         self.last = self._record(b, T)
-        self._make_ring(T, x.device)
-        if check_status:
-            self.raise_on_status(b["status"])
         return b["out"] if out is None else out
 
     @staticmethod

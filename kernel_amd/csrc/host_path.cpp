@@ -5,10 +5,13 @@
 // seven more (9.5 us per call of custom_kernel at 7 tokens).  Here the same steps read the tensors'
 // own C++ records.
 //
-//   Ring   the two alternating buffer sets of one token count: their argument blocks, the tensors a call hands
-//          out, and which set is next.  `forward` takes the caller's tensors, or returns None without side
-//          effects when anything about them is not as the argument blocks were built for (the caller then
-//          goes the long way, which raises the right error or builds the right ring).
+//   Ring   the two alternating buffer sets of one token count: which set is next, when they were used last and,
+//          from a set's first forward on (`bind`), its argument block and the tensors a call hands out.
+//   Rings  those of one host object.  `forward` takes the caller's tensors, or returns None without side
+//          effects when no ring is of their shape, its next set is not bound yet, or anything about them is not
+//          as the argument block was built for (the caller then goes the long way, which raises the right
+//          error or binds the set).
+//          Calls whose token counts change from one to the next find their ring here too.
 //   Memo   the configurations of recent custom_kernel calls and the host objects they belong to (one process
 //          may run every rank of a world in turn).
 #define PY_SSIZE_T_CLEAN
@@ -29,7 +32,7 @@
 namespace {
 
 // interned attribute names
-PyObject *s_stub_kind, *s_combine_mode, *s_fuse_route, *s_fuse_stub, *s_last, *s_ring, *s_num_experts,
+PyObject *s_stub_kind, *s_combine_mode, *s_fuse_route, *s_fuse_stub, *s_last, *s_rings, *s_num_experts,
     *s_experts_per_token, *s_hidden_dim, *s_max_num_tokens, *s_in_dtype, *s_out_dtype, *s_x, *s_indices, *s_weights,
     *s_num_tokens, *s_always;
 
@@ -60,7 +63,9 @@ bool int_attr(PyObject* o, PyObject* name, long& v) {
 struct Ring {
   PyObject_HEAD
   long T, K, H, W;
+  long long used;  // the clock of its Rings at the last use: the one with the lowest goes first
   int device, cur;
+  int bound;  // bit i: set i
   at::ScalarType in_type, out_type;
   moe_a2a_forward_args args[2];
   PyObject* outs[2];
@@ -70,34 +75,43 @@ struct Ring {
 PyObject* ring_new(PyTypeObject* type, PyObject* args, PyObject*) {
   long T, K, H, W;
   int device;
-  PyObject *in_type, *out_type, *outs[2], *records[2];
-  const char* block[2];
-  Py_ssize_t len[2];
-  if (!PyArg_ParseTuple(args, "lllliO!O!y#y#OOOO", &T, &K, &H, &W, &device, &THPDtypeType, &in_type, &THPDtypeType,
-                        &out_type, &block[0], &len[0], &block[1], &len[1], &outs[0], &outs[1], &records[0],
-                        &records[1]))
+  PyObject *in_type, *out_type;
+  if (!PyArg_ParseTuple(args, "lllliO!O!", &T, &K, &H, &W, &device, &THPDtypeType, &in_type, &THPDtypeType, &out_type))
     return nullptr;
-  for (Py_ssize_t n : len)
-    if (n != (Py_ssize_t)sizeof(moe_a2a_forward_args)) {
-      PyErr_SetString(PyExc_ValueError, "an argument block is not a moe_a2a_forward_args");
-      return nullptr;
-    }
-  Ring* r = (Ring*)type->tp_alloc(type, 0);
+  Ring* r = (Ring*)type->tp_alloc(type, 0);  // zeroed
   if (!r) return nullptr;
-  r->T = T, r->K = K, r->H = H, r->W = W, r->device = device, r->cur = 0;
+  r->T = T, r->K = K, r->H = H, r->W = W, r->device = device;
   r->in_type = ((THPDtype*)in_type)->scalar_type;
   r->out_type = ((THPDtype*)out_type)->scalar_type;
-  for (int i = 0; i < 2; ++i) {
-    std::memcpy(&r->args[i], block[i], sizeof(moe_a2a_forward_args));
-    Py_INCREF(outs[i]);
-    Py_INCREF(records[i]);
-    r->outs[i] = outs[i];
-    r->records[i] = records[i];
-  }
   return (PyObject*)r;
 }
 
+// bind(set, block, out, record)
+PyObject* ring_bind(Ring* r, PyObject* args) {
+  int set;
+  PyObject *out, *record;
+  const char* block;
+  Py_ssize_t len;
+  if (!PyArg_ParseTuple(args, "iy#OO", &set, &block, &len, &out, &record)) return nullptr;
+  if (set != 0 && set != 1) {
+    PyErr_SetString(PyExc_ValueError, "the sets are 0 and 1");
+    return nullptr;
+  }
+  if (len != (Py_ssize_t)sizeof(moe_a2a_forward_args)) {
+    PyErr_SetString(PyExc_ValueError, "the argument block is not a moe_a2a_forward_args");
+    return nullptr;
+  }
+  std::memcpy(&r->args[set], block, sizeof(moe_a2a_forward_args));
+  Py_INCREF(out);
+  Py_XSETREF(r->outs[set], out);
+  Py_INCREF(record);
+  Py_XSETREF(r->records[set], record);
+  r->bound |= 1 << set;
+  Py_RETURN_NONE;
+}
+
 int ring_clear(Ring* r) {
+  r->bound = 0;
   for (int i = 0; i < 2; ++i) {
     Py_CLEAR(r->outs[i]);
     Py_CLEAR(r->records[i]);
@@ -143,11 +157,11 @@ Outcome ring_forward(Ring* r, PyObject* owner, const at::Tensor& x, const at::Te
     PyErr_Clear();
     return kNotThisWay;
   }
-  if (route.p == Py_True || route.p == Py_False)
-    fuse_route = route.p == Py_True;
+  if (PyLong_Check(route.p))  // (a truth value is one)
+    fuse_route = PyObject_IsTrue(route.p);
   else if (!PyUnicode_Check(route.p) || PyUnicode_Compare(route.p, s_always) != 0)
     return kNotThisWay;
-  if (stub.p != Py_True && stub.p != Py_False) return kNotThisWay;
+  if (!PyLong_Check(stub.p)) return kNotThisWay;
   set = r->cur ^= 1;
   moe_a2a_forward_args a = r->args[set];  // a copy: the launch runs without the interpreter's lock
   a.x = x.const_data_ptr();
@@ -159,7 +173,7 @@ Outcome ring_forward(Ring* r, PyObject* owner, const at::Tensor& x, const at::Te
   a.stub_kind = (int)stub_kind;
   a.combine_mode = (int)combine_mode;
   a.fuse_route = (int)fuse_route;
-  a.fuse_stub = stub.p == Py_True;
+  a.fuse_stub = PyObject_IsTrue(stub.p);
   PyObject* record = r->records[set];
   Py_INCREF(record);
   int rc;
@@ -177,8 +191,38 @@ Outcome ring_forward(Ring* r, PyObject* owner, const at::Tensor& x, const at::Te
   return bad ? kError : kDone;
 }
 
+PyMethodDef ring_methods[] = {{"bind", (PyCFunction)ring_bind, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyMemberDef ring_members[] = {{"cur", T_INT, offsetof(Ring, cur), 0, nullptr},
+                              {"used", T_LONGLONG, offsetof(Ring, used), READONLY, nullptr},
+                              {"bound", T_INT, offsetof(Ring, bound), READONLY, nullptr},
+                              {nullptr, 0, 0, 0, nullptr}};
+PyTypeObject RingType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ---------------------------------------------------------------------------------------
+struct Rings {
+  PyObject_HEAD
+  long long clock;
+  PyObject* all;  // list of Ring
+};
+
+// the ring of these rows, if its next set is bound (a new reference, marked as used), or null
+Ring* rings_find(Rings* rs, const at::Tensor& x) {
+  if (x.dim() != 2 || !x.is_cuda()) return nullptr;
+  const long T = (long)x.size(0);
+  const int device = x.get_device();
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(rs->all); ++i) {
+    Ring* r = (Ring*)PyList_GET_ITEM(rs->all, i);
+    if (r->T == T && r->device == device && (r->bound >> (r->cur ^ 1) & 1)) {
+      r->used = ++rs->clock;
+      Py_INCREF(r);
+      return r;
+    }
+  }
+  return nullptr;
+}
+
 // forward(owner, x, indices, weights, rank_start or None, out or None) -> y, or None: not this way
-PyObject* ring_forward_py(Ring* r, PyObject* const* args, Py_ssize_t n) {
+PyObject* rings_forward(Rings* rs, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 6) {
     PyErr_SetString(PyExc_TypeError, "forward takes owner, x, indices, weights, rank_start, out");
@@ -186,6 +230,10 @@ PyObject* ring_forward_py(Ring* r, PyObject* const* args, Py_ssize_t n) {
   }
   for (int i = 1; i < 6; ++i)
     if (!THPVariable_Check(args[i]) && !(i >= 4 && args[i] == Py_None)) Py_RETURN_NONE;
+  const at::Tensor& x = THPVariable_Unpack(args[1]);
+  Ref ring((PyObject*)rings_find(rs, x));
+  if (!ring) Py_RETURN_NONE;
+  Ring* r = (Ring*)ring.p;
   const at::Tensor* rank_start = args[4] == Py_None ? nullptr : &THPVariable_Unpack(args[4]);
   void* out = nullptr;
   if (args[5] != Py_None) {
@@ -194,8 +242,7 @@ PyObject* ring_forward_py(Ring* r, PyObject* const* args, Py_ssize_t n) {
     out = o.data_ptr();
   }
   int set = 0;
-  switch (ring_forward(r, args[0], THPVariable_Unpack(args[1]), THPVariable_Unpack(args[2]), THPVariable_Unpack(args[3]),
-                       rank_start, out, set)) {
+  switch (ring_forward(r, args[0], x, THPVariable_Unpack(args[2]), THPVariable_Unpack(args[3]), rank_start, out, set)) {
     case kNotThisWay: Py_RETURN_NONE;
     case kError: return nullptr;
     case kDone: break;
@@ -206,10 +253,61 @@ PyObject* ring_forward_py(Ring* r, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef ring_methods[] = {
-    {"forward", (PyCFunction)(void (*)(void))ring_forward_py, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
-PyMemberDef ring_members[] = {{"cur", T_INT, offsetof(Ring, cur), 0, nullptr}, {nullptr, 0, 0, 0, nullptr}};
-PyTypeObject RingType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+PyObject* rings_new(PyTypeObject* type, PyObject*, PyObject*) {
+  Rings* rs = (Rings*)type->tp_alloc(type, 0);
+  if (rs && !(rs->all = PyList_New(0))) Py_CLEAR(rs);
+  return (PyObject*)rs;
+}
+// add(ring)
+PyObject* rings_add(Rings* rs, PyObject* ring) {
+  if (Py_TYPE(ring) != &RingType) {
+    PyErr_SetString(PyExc_TypeError, "add takes a Ring");
+    return nullptr;
+  }
+  if (PyList_Append(rs->all, ring) < 0) return nullptr;
+  Py_RETURN_NONE;
+}
+// touch(ring): used now
+PyObject* rings_touch(Rings* rs, PyObject* ring) {
+  if (Py_TYPE(ring) != &RingType) {
+    PyErr_SetString(PyExc_TypeError, "touch takes a Ring");
+    return nullptr;
+  }
+  ((Ring*)ring)->used = ++rs->clock;
+  Py_RETURN_NONE;
+}
+PyObject* rings_drop(Rings* rs, PyObject* ring) {
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(rs->all); ++i)
+    if (PyList_GET_ITEM(rs->all, i) == ring) {
+      if (PyList_SetSlice(rs->all, i, i + 1, nullptr) < 0) return nullptr;
+      break;
+    }
+  Py_RETURN_NONE;
+}
+PyObject* rings_clear_py(Rings* rs, PyObject*) {
+  if (PyList_SetSlice(rs->all, 0, PyList_GET_SIZE(rs->all), nullptr) < 0) return nullptr;
+  Py_RETURN_NONE;
+}
+int rings_traverse(Rings* rs, visitproc visit, void* arg) {
+  Py_VISIT(rs->all);
+  return 0;
+}
+// (an object in a cycle that is being taken apart may still be asked for: an empty list serves)
+int rings_clear(Rings* rs) {
+  return rs->all ? PyList_SetSlice(rs->all, 0, PyList_GET_SIZE(rs->all), nullptr) : 0;
+}
+void rings_dealloc(Rings* rs) {
+  PyObject_GC_UnTrack(rs);
+  Py_CLEAR(rs->all);
+  Py_TYPE(rs)->tp_free((PyObject*)rs);
+}
+PyMethodDef rings_methods[] = {{"forward", (PyCFunction)(void (*)(void))rings_forward, METH_FASTCALL, nullptr},
+                               {"add", (PyCFunction)rings_add, METH_O, nullptr},
+                               {"touch", (PyCFunction)rings_touch, METH_O, nullptr},
+                               {"drop", (PyCFunction)rings_drop, METH_O, nullptr},
+                               {"clear", (PyCFunction)rings_clear_py, METH_NOARGS, nullptr},
+                               {nullptr, nullptr, 0, nullptr}};
+PyTypeObject RingsType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // ---------------------------------------------------------------------------------------
 constexpr int kMemoEntries = 16;
@@ -320,7 +418,7 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
   const int at = memo_find(m, config, call, in_dtype.p, out_dtype.p);
   if (at < 0) Py_RETURN_NONE;
   entry_front(m, at);
-  Ref owner(m->entry[0].owner), ring(nullptr);  // taken here: the lookups below may run Python code, and other threads
+  Ref owner(m->entry[0].owner), rings, ring;  // taken here: the lookups below may run Python code, and other threads
   Py_INCREF(owner.p);
   PyObject* rank_data = PyTuple_GET_ITEM(args[0], 1);
   long num_tokens;
@@ -331,13 +429,15 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
-  ring.p = PyObject_GetAttr(owner.p, s_ring);
-  if (!ring || Py_TYPE(ring.p) != &RingType) {
+  rings.p = PyObject_GetAttr(owner.p, s_rings);
+  if (!rings || Py_TYPE(rings.p) != &RingsType) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
-  Ring* r = (Ring*)ring.p;
   const at::Tensor& xt = THPVariable_Unpack(x.p);
+  ring.p = (PyObject*)rings_find((Rings*)rings.p, xt);
+  if (!ring) Py_RETURN_NONE;
+  Ring* r = (Ring*)ring.p;
   if (num_tokens < 0 || num_tokens > r->T || !plain_matrix(xt, r->in_type, r->T, r->H, r->device)) Py_RETURN_NONE;
   // the caller owns its result: the combine writes straight into a fresh tensor
   at::Tensor y = at::empty({r->T, r->H}, xt.options().dtype(r->out_type));
@@ -381,7 +481,7 @@ PyMODINIT_FUNC PyInit__host(void) {
     const char* text;
   } names[] = {{s_stub_kind, "stub_kind"},     {s_combine_mode, "combine_mode"},
                {s_fuse_route, "fuse_route"},   {s_fuse_stub, "fuse_stub"},
-               {s_last, "last"},               {s_ring, "_ring"},
+               {s_last, "last"},               {s_rings, "_rings"},
                {s_num_experts, "num_experts"}, {s_experts_per_token, "experts_per_token"},
                {s_hidden_dim, "hidden_dim"},   {s_max_num_tokens, "max_num_tokens"},
                {s_in_dtype, "in_dtype"},       {s_out_dtype, "out_dtype"},
@@ -399,6 +499,14 @@ PyMODINIT_FUNC PyInit__host(void) {
   RingType.tp_clear = (inquiry)ring_clear;
   RingType.tp_methods = ring_methods;
   RingType.tp_members = ring_members;
+  RingsType.tp_name = "kernel_amd._host.Rings";
+  RingsType.tp_basicsize = sizeof(Rings);
+  RingsType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  RingsType.tp_new = rings_new;
+  RingsType.tp_dealloc = (destructor)rings_dealloc;
+  RingsType.tp_traverse = (traverseproc)rings_traverse;
+  RingsType.tp_clear = (inquiry)rings_clear;
+  RingsType.tp_methods = rings_methods;
   MemoType.tp_name = "kernel_amd._host.Memo";
   MemoType.tp_basicsize = sizeof(Memo);
   MemoType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
@@ -407,12 +515,14 @@ PyMODINIT_FUNC PyInit__host(void) {
   MemoType.tp_traverse = (traverseproc)memo_traverse;
   MemoType.tp_clear = (inquiry)memo_clear;
   MemoType.tp_methods = memo_methods;
-  if (PyType_Ready(&RingType) < 0 || PyType_Ready(&MemoType) < 0) return nullptr;
+  if (PyType_Ready(&RingType) < 0 || PyType_Ready(&RingsType) < 0 || PyType_Ready(&MemoType) < 0) return nullptr;
   PyObject* m = PyModule_Create(&module);
   if (!m) return nullptr;
   Py_INCREF(&RingType);
+  Py_INCREF(&RingsType);
   Py_INCREF(&MemoType);
-  if (PyModule_AddObject(m, "Ring", (PyObject*)&RingType) < 0 || PyModule_AddObject(m, "Memo", (PyObject*)&MemoType) < 0)
+  if (PyModule_AddObject(m, "Ring", (PyObject*)&RingType) < 0 ||
+      PyModule_AddObject(m, "Rings", (PyObject*)&RingsType) < 0 || PyModule_AddObject(m, "Memo", (PyObject*)&MemoType) < 0)
     return nullptr;
   return m;
 }

@@ -80,3 +80,40 @@ def test_switches_streams_and_phases_between_forwards(gpu_device):
     with pytest.raises(IndexError):
         ata.forward(rd.x, bad, rd.weights, check_status=True)
     assert ata.forward(rd.x[:6], rd.indices[:6], rd.weights[:6]).shape[0] == 6
+
+
+def test_token_counts_in_turn_take_the_short_way(gpu_device, monkeypatch):
+    """A call whose token count is not the last one's, but an earlier one's, builds nothing anew: not an argument block,
+    not a record; also behind a dispatch of the same shape, and with the least recently used shape dropped."""
+    cases = [case(0, T) for T in range(3, 3 + HipAllToAll.MAX_CACHED_SHAPES)]
+    ata = HipAllToAll(cases[0][0], 0, 8, fuse_stub=True)
+    for _, rd, _, want in cases + cases:  # both sets of every shape
+        assert same(ata.forward(rd.x, rd.indices, rd.weights), want)
+        assert same(custom_kernel((cases[0][0], rd, 0, 8)), want)
+    built = []
+    args, record = HipAllToAll._forward_args, HipAllToAll._record
+    monkeypatch.setattr(HipAllToAll, "_forward_args", lambda *a: built.append("block") or args(*a))
+    monkeypatch.setattr(HipAllToAll, "_record", lambda *a: built.append("record") or record(*a))
+    for turn in range(3):
+        for _, rd, _, want in cases if turn else reversed(cases):
+            y = ata.forward(rd.x, rd.indices, rd.weights)
+            assert same(y, want) and ata.last.num_tokens == y.shape[0]
+            first = ata.last.disp_x.data_ptr()
+            assert ata.dispatch(rd.x, rd.indices).disp_x.data_ptr() != first  # the other of the two sets
+            assert same(custom_kernel((cases[0][0], rd, 0, 8)), want)
+    assert not built
+    # the shape used longest ago, by a forward or by a dispatch, makes room for a new one
+    order = cases[4:] + cases[:4]
+    for i, (_, rd, _, _) in enumerate(order):
+        ata.dispatch(rd.x, rd.indices) if i % 2 else ata.forward(rd.x, rd.indices, rd.weights)
+    _, rd, _, want = case(0, 40)
+    assert same(ata.forward(rd.x, rd.indices, rd.weights), want) and built
+    kept = {key[0] for key in ata._bufs}
+    assert kept == {40} | {c[1].num_tokens for c in order[1:]}
+    del built[:]
+    for _, rd, _, want in order[1:]:
+        assert same(ata.forward(rd.x, rd.indices, rd.weights), want)
+    assert not built
+    ata.release_buffers()
+    _, rd, _, want = cases[0]
+    assert same(ata.forward(rd.x, rd.indices, rd.weights), want) and len(ata._bufs) == 1
