@@ -312,7 +312,7 @@ PyTypeObject RingsType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 // ---------------------------------------------------------------------------------------
 constexpr int kMemoEntries = 16;
 struct MemoEntry {
-  long config[4], call[4];  // call: rank, world_size, stub_kind, combine_mode
+  long config[4], call[5];  // call: rank, world_size, stub_kind, combine_mode, device of the inputs
   PyObject *in_dtype, *out_dtype, *owner;
 };
 struct Memo {
@@ -348,7 +348,7 @@ bool memo_read(PyObject* cfg, long (&v)[4], Ref& in_dtype, Ref& out_dtype) {
 }
 
 // the entry of these values, or -1
-int memo_find(const Memo* m, const long (&config)[4], const long (&call)[4], const PyObject* in_dtype,
+int memo_find(const Memo* m, const long (&config)[4], const long (&call)[5], const PyObject* in_dtype,
               const PyObject* out_dtype) {
   for (int i = 0; i < m->used; ++i) {
     const MemoEntry& e = m->entry[i];
@@ -359,14 +359,14 @@ int memo_find(const Memo* m, const long (&config)[4], const long (&call)[4], con
   return -1;
 }
 
-// remember(cfg, rank, world_size, stub_kind, combine_mode, owner)
+// remember(cfg, rank, world_size, stub_kind, combine_mode, device index, owner)
 PyObject* memo_remember(Memo* m, PyObject* const* args, Py_ssize_t n) {
-  if (n != 6) {
-    PyErr_SetString(PyExc_TypeError, "remember takes cfg, rank, world_size, stub_kind, combine_mode, owner");
+  if (n != 7) {
+    PyErr_SetString(PyExc_TypeError, "remember takes cfg, rank, world_size, stub_kind, combine_mode, device, owner");
     return nullptr;
   }
   MemoEntry fresh;
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 5; ++i) {
     fresh.call[i] = PyLong_AsLong(args[1 + i]);
     if (fresh.call[i] == -1 && PyErr_Occurred()) {
       PyErr_Clear();
@@ -389,8 +389,8 @@ PyObject* memo_remember(Memo* m, PyObject* const* args, Py_ssize_t n) {
     in_dtype.p = out_dtype.p = nullptr;
     m->entry[at] = fresh;
   }
-  Py_INCREF(args[5]);
-  Py_XSETREF(m->entry[at].owner, args[5]);
+  Py_INCREF(args[6]);
+  Py_XSETREF(m->entry[at].owner, args[6]);
   entry_front(m, at);
   Py_RETURN_NONE;
 }
@@ -403,7 +403,7 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
     return nullptr;
   }
   if (!PyTuple_CheckExact(args[0]) || PyTuple_GET_SIZE(args[0]) != 4) Py_RETURN_NONE;
-  long call[4];
+  long call[5];
   PyObject* given[4] = {PyTuple_GET_ITEM(args[0], 2), PyTuple_GET_ITEM(args[0], 3), args[1], args[2]};
   for (int i = 0; i < 4; ++i) {
     call[i] = PyLong_CheckExact(given[i]) ? PyLong_AsLong(given[i]) : -1;
@@ -412,14 +412,6 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
       Py_RETURN_NONE;
     }
   }
-  long config[4];
-  Ref in_dtype, out_dtype;
-  if (!memo_read(PyTuple_GET_ITEM(args[0], 0), config, in_dtype, out_dtype)) Py_RETURN_NONE;
-  const int at = memo_find(m, config, call, in_dtype.p, out_dtype.p);
-  if (at < 0) Py_RETURN_NONE;
-  entry_front(m, at);
-  Ref owner(m->entry[0].owner), rings, ring;  // taken here: the lookups below may run Python code, and other threads
-  Py_INCREF(owner.p);
   PyObject* rank_data = PyTuple_GET_ITEM(args[0], 1);
   long num_tokens;
   Ref x(PyObject_GetAttr(rank_data, s_x)), indices(PyObject_GetAttr(rank_data, s_indices)),
@@ -429,12 +421,21 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
+  const at::Tensor& xt = THPVariable_Unpack(x.p);
+  call[4] = xt.get_device();
+  long config[4];
+  Ref in_dtype, out_dtype;
+  if (!memo_read(PyTuple_GET_ITEM(args[0], 0), config, in_dtype, out_dtype)) Py_RETURN_NONE;
+  const int at = memo_find(m, config, call, in_dtype.p, out_dtype.p);
+  if (at < 0) Py_RETURN_NONE;
+  entry_front(m, at);
+  Ref owner(m->entry[0].owner), rings, ring;  // taken here: the lookups below may run Python code, and other threads
+  Py_INCREF(owner.p);
   rings.p = PyObject_GetAttr(owner.p, s_rings);
   if (!rings || Py_TYPE(rings.p) != &RingsType) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
-  const at::Tensor& xt = THPVariable_Unpack(x.p);
   ring.p = (PyObject*)rings_find((Rings*)rings.p, xt);
   if (!ring) Py_RETURN_NONE;
   Ring* r = (Ring*)ring.p;

@@ -16,7 +16,7 @@ from .contract import COMBINE_STRICT, STUB_OWNER_RANK
 
 _instances = {}
 _last = [None, None]  # key and instance of the previous call (a harness calls with one config many times)
-_memo = None  # the same for the native side (_host.Memo), which runs a call that repeats the previous configuration
+_memo = None  # the same for the native side (_host.Memo): the configurations of the last sixteen, each with its instance
 
 
 def _instance(cfg, rank: int, world_size: int, device, stub_kind: int, combine_mode: int) -> HipAllToAll:
@@ -71,6 +71,6 @@ def custom_kernel(data, stub_kind: int = STUB_OWNER_RANK, combine_mode: int = CO
             ata.forward(x, idx, w, out=y, check_status=check_status)
     if _memo is None:
         _memo = _lib.host().Memo()
-    _memo.remember(cfg, rank, world_size, stub_kind, combine_mode, ata)
+    _memo.remember(cfg, rank, world_size, stub_kind, combine_mode, x.device.index, ata)
     n = rank_data.num_tokens
     return y if n == T else y[:n]

@@ -127,3 +127,26 @@ def test_host_object_keeps_its_own_copy_of_the_config():
     ata = HipAllToAll(cfg, 0, 8)
     cfg.hidden_dim = 64
     assert ata.cfg.hidden_dim == 2048 and ata.cfg is not cfg
+
+
+class _Owner:
+    """Stands in for a HipAllToAll: notes that the native side of custom_kernel has looked it up."""
+
+    def __init__(self):
+        self.asked = 0
+
+    @property
+    def _rings(self):
+        self.asked += 1
+
+
+def test_memo_of_the_native_path_tells_devices_apart():
+    from kernel_amd import _lib
+
+    cfg, rd, rank, world = C.generate_input(8, 2, 64, 8, 5, 0, 8)
+    memo, here, there = _lib.host().Memo(), _Owner(), _Owner()
+    memo.remember(cfg, rank, world, 0, 0, -1, here)  # -1: the index that a CPU tensor reports
+    memo.remember(cfg, rank, world, 0, 0, 1, there)
+    for _ in range(2):
+        assert memo.run((cfg, rd, rank, world), 0, 0) is None  # (no ring there to run on)
+    assert (here.asked, there.asked) == (2, 0)
