@@ -455,7 +455,10 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
 
 PyObject* memo_new(PyTypeObject* type, PyObject*, PyObject*) { return type->tp_alloc(type, 0); }
 int memo_clear(Memo* m) {
-  while (m->used > 0) entry_drop(m->entry[--m->used]);
+  while (m->used > 0) {  // an entry is off the table before what it held goes, which may run Python code
+    MemoEntry e = m->entry[--m->used];
+    entry_drop(e);
+  }
   return 0;
 }
 int memo_traverse(Memo* m, visitproc visit, void* arg) {
@@ -467,7 +470,12 @@ void memo_dealloc(Memo* m) {
   memo_clear(m);
   Py_TYPE(m)->tp_free((PyObject*)m);
 }
-PyMethodDef memo_methods[] = {{"remember", (PyCFunction)(void (*)(void))memo_remember, METH_FASTCALL, nullptr},
+PyObject* memo_clear_py(Memo* m, PyObject*) {
+  memo_clear(m);
+  Py_RETURN_NONE;
+}
+PyMethodDef memo_methods[] = {{"clear", (PyCFunction)memo_clear_py, METH_NOARGS, nullptr},
+                              {"remember", (PyCFunction)(void (*)(void))memo_remember, METH_FASTCALL, nullptr},
                               {"run", (PyCFunction)(void (*)(void))memo_run, METH_FASTCALL, nullptr},
                               {nullptr, nullptr, 0, nullptr}};
 PyTypeObject MemoType = {PyVarObject_HEAD_INIT(nullptr, 0)};

@@ -34,6 +34,9 @@ def _instance(cfg, rank: int, world_size: int, device, stub_kind: int, combine_m
     if ata is None:
         if len(_instances) > 64:
             _instances.clear()
+            _last[:] = None, None
+            if _memo is not None:
+                _memo.clear()
         # the stub is a stand-in for expert compute: folding it into the combine gives the same
         # bits with one launch and one pass over the dispatched rows fewer
         ata = _instances[key] = HipAllToAll(cfg, rank, world_size, stub_kind=stub_kind, combine_mode=combine_mode,

@@ -150,3 +150,26 @@ def test_memo_of_the_native_path_tells_devices_apart():
     for _ in range(2):
         assert memo.run((cfg, rd, rank, world), 0, 0) is None  # (no ring there to run on)
     assert (here.asked, there.asked) == (2, 0)
+
+
+def test_instances_let_go_of_are_not_kept_by_the_native_path(monkeypatch):
+    import gc
+    import weakref
+
+    from kernel_amd import _lib
+    from kernel_amd import submission as S
+
+    monkeypatch.setattr(S, "_instances", {})
+    monkeypatch.setattr(S, "_last", [None, None])
+    monkeypatch.setattr(S, "_memo", _lib.host().Memo())
+    cfg = C.MoEConfig(8, 2, 64, 8)
+    alive = []
+    for rank in range(66):
+        cfg.max_num_tokens = 8 + rank
+        ata = S._instance(cfg, 0, 8, "cuda:0", 0, 0)
+        S._memo.remember(cfg, 0, 8, 0, 0, 0, ata)
+        alive.append(weakref.ref(ata))
+    del ata
+    gc.collect()
+    assert len(S._instances) == 1
+    assert [r() for r in alive] == [None] * 65 + [S._last[1]]
