@@ -45,19 +45,31 @@ struct Ref {  // owned reference
   explicit operator bool() const { return p != nullptr; }
 };
 
-// integer attribute; false (with the error cleared) when it is missing or no integer
-bool int_attr(PyObject* o, PyObject* name, long& v) {
-  Ref a(PyObject_GetAttr(o, name));
-  if (!a) {
-    PyErr_Clear();
-    return false;
-  }
+enum Outcome { kDone, kNotThisWay, kError };
+
+// After a failed lookup or conversion: an attribute that is not there, or of another kind than expected, is for the long
+// way to judge (its error is cleared); whatever else was raised, an interrupt or no memory among them, is the caller's.
+Outcome failed() {
+  if (!PyErr_ExceptionMatches(PyExc_AttributeError) && !PyErr_ExceptionMatches(PyExc_TypeError) &&
+      !PyErr_ExceptionMatches(PyExc_OverflowError))
+    return kError;
+  PyErr_Clear();
+  return kNotThisWay;
+}
+Outcome get_attr(PyObject* o, PyObject* name, Ref& v) {
+  v.p = PyObject_GetAttr(o, name);
+  return v ? kDone : failed();
+}
+Outcome int_attr(PyObject* o, PyObject* name, long& v) {
+  Ref a;
+  if (const Outcome got = get_attr(o, name, a)) return got;
   v = PyLong_AsLong(a.p);
-  if (v == -1 && PyErr_Occurred()) {
-    PyErr_Clear();
-    return false;
-  }
-  return true;
+  return v == -1 && PyErr_Occurred() ? failed() : kDone;
+}
+// what a Python caller gets for it: None, or the exception
+PyObject* outcome(Outcome o) {
+  if (o == kError) return nullptr;
+  Py_RETURN_NONE;
 }
 
 struct Ring {
@@ -136,8 +148,6 @@ bool plain_matrix(const at::Tensor& t, at::ScalarType type, long rows, long cols
          t.is_cuda() && t.get_device() == device;
 }
 
-enum Outcome { kDone, kNotThisWay, kError };
-
 // One call on the next set; out: where the result goes (already checked).  Sets a Python error on kError.
 Outcome ring_forward(Ring* r, PyObject* owner, const at::Tensor& x, const at::Tensor& indices,
                      const at::Tensor& weights, const at::Tensor* rank_start, void* out, int& set) {
@@ -151,12 +161,11 @@ Outcome ring_forward(Ring* r, PyObject* owner, const at::Tensor& x, const at::Te
   if (c10::hip::current_device() != r->device) return kNotThisWay;
   // switches of the host object that may change between two calls
   long stub_kind, combine_mode, fuse_route = 2;
-  if (!int_attr(owner, s_stub_kind, stub_kind) || !int_attr(owner, s_combine_mode, combine_mode)) return kNotThisWay;
-  Ref route(PyObject_GetAttr(owner, s_fuse_route)), stub(PyObject_GetAttr(owner, s_fuse_stub));
-  if (!route || !stub) {
-    PyErr_Clear();
-    return kNotThisWay;
-  }
+  Ref route, stub;
+  Outcome got;
+  if ((got = int_attr(owner, s_stub_kind, stub_kind)) || (got = int_attr(owner, s_combine_mode, combine_mode)) ||
+      (got = get_attr(owner, s_fuse_route, route)) || (got = get_attr(owner, s_fuse_stub, stub)))
+    return got;
   if (PyLong_Check(route.p))  // (a truth value is one)
     fuse_route = PyObject_IsTrue(route.p);
   else if (!PyUnicode_Check(route.p) || PyUnicode_Compare(route.p, s_always) != 0)
@@ -242,11 +251,9 @@ PyObject* rings_forward(Rings* rs, PyObject* const* args, Py_ssize_t n) {
     out = o.data_ptr();
   }
   int set = 0;
-  switch (ring_forward(r, args[0], x, THPVariable_Unpack(args[2]), THPVariable_Unpack(args[3]), rank_start, out, set)) {
-    case kNotThisWay: Py_RETURN_NONE;
-    case kError: return nullptr;
-    case kDone: break;
-  }
+  if (const Outcome got = ring_forward(r, args[0], x, THPVariable_Unpack(args[2]), THPVariable_Unpack(args[3]), rank_start,
+                                       out, set))
+    return outcome(got);
   PyObject* y = out ? args[5] : r->outs[set];
   Py_INCREF(y);
   return y;
@@ -334,17 +341,13 @@ void entry_front(Memo* m, int i) {
 }
 
 // what custom_kernel's instance depends on, read from the config record at every call
-bool memo_read(PyObject* cfg, long (&v)[4], Ref& in_dtype, Ref& out_dtype) {
-  if (!int_attr(cfg, s_num_experts, v[0]) || !int_attr(cfg, s_experts_per_token, v[1]) ||
-      !int_attr(cfg, s_hidden_dim, v[2]) || !int_attr(cfg, s_max_num_tokens, v[3]))
-    return false;
-  in_dtype.p = PyObject_GetAttr(cfg, s_in_dtype);
-  out_dtype.p = PyObject_GetAttr(cfg, s_out_dtype);
-  if (!in_dtype || !out_dtype) {
-    PyErr_Clear();
-    return false;
-  }
-  return true;
+Outcome memo_read(PyObject* cfg, long (&v)[4], Ref& in_dtype, Ref& out_dtype) {
+  Outcome got;
+  if ((got = int_attr(cfg, s_num_experts, v[0])) || (got = int_attr(cfg, s_experts_per_token, v[1])) ||
+      (got = int_attr(cfg, s_hidden_dim, v[2])) || (got = int_attr(cfg, s_max_num_tokens, v[3])) ||
+      (got = get_attr(cfg, s_in_dtype, in_dtype)) || (got = get_attr(cfg, s_out_dtype, out_dtype)))
+    return got;
+  return kDone;
 }
 
 // the entry of these values, or -1
@@ -368,30 +371,29 @@ PyObject* memo_remember(Memo* m, PyObject* const* args, Py_ssize_t n) {
   MemoEntry fresh;
   for (int i = 0; i < 5; ++i) {
     fresh.call[i] = PyLong_AsLong(args[1 + i]);
-    if (fresh.call[i] == -1 && PyErr_Occurred()) {
-      PyErr_Clear();
-      Py_RETURN_NONE;
-    }
+    if (fresh.call[i] == -1 && PyErr_Occurred()) return outcome(failed());
   }
   Ref in_dtype, out_dtype;
-  if (!memo_read(args[0], fresh.config, in_dtype, out_dtype)) Py_RETURN_NONE;
-  int at = memo_find(m, fresh.config, fresh.call, in_dtype.p, out_dtype.p);
-  if (at < 0) {
-    if (m->used < kMemoEntries) {
-      at = m->used++;
-    } else {
-      at = kMemoEntries - 1;  // the one not used for longest
-      entry_drop(m->entry[at]);
-    }
-    fresh.in_dtype = in_dtype.p;
-    fresh.out_dtype = out_dtype.p;
-    fresh.owner = nullptr;
-    in_dtype.p = out_dtype.p = nullptr;
-    m->entry[at] = fresh;
-  }
+  if (const Outcome got = memo_read(args[0], fresh.config, in_dtype, out_dtype)) return outcome(got);
+  const int at = memo_find(m, fresh.config, fresh.call, in_dtype.p, out_dtype.p);
   Py_INCREF(args[6]);
-  Py_XSETREF(m->entry[at].owner, args[6]);
-  entry_front(m, at);
+  if (at >= 0) {
+    PyObject* before = m->entry[at].owner;
+    m->entry[at].owner = args[6];
+    entry_front(m, at);
+    Py_DECREF(before);
+    Py_RETURN_NONE;
+  }
+  fresh.in_dtype = in_dtype.p;
+  fresh.out_dtype = out_dtype.p;
+  fresh.owner = args[6];
+  in_dtype.p = out_dtype.p = nullptr;
+  const bool full = m->used == kMemoEntries;
+  MemoEntry longest_unused = m->entry[kMemoEntries - 1];
+  if (!full) ++m->used;
+  m->entry[m->used - 1] = fresh;
+  entry_front(m, m->used - 1);
+  if (full) entry_drop(longest_unused);  // last: this may run Python code, which finds a whole table
   Py_RETURN_NONE;
 }
 
@@ -407,35 +409,29 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
   PyObject* given[4] = {PyTuple_GET_ITEM(args[0], 2), PyTuple_GET_ITEM(args[0], 3), args[1], args[2]};
   for (int i = 0; i < 4; ++i) {
     call[i] = PyLong_CheckExact(given[i]) ? PyLong_AsLong(given[i]) : -1;
-    if (call[i] < 0) {
-      PyErr_Clear();
-      Py_RETURN_NONE;
-    }
+    if (call[i] == -1 && PyErr_Occurred()) return outcome(failed());
+    if (call[i] < 0) Py_RETURN_NONE;
   }
   PyObject* rank_data = PyTuple_GET_ITEM(args[0], 1);
   long num_tokens;
-  Ref x(PyObject_GetAttr(rank_data, s_x)), indices(PyObject_GetAttr(rank_data, s_indices)),
-      weights(PyObject_GetAttr(rank_data, s_weights));
-  if (!x || !indices || !weights || !int_attr(rank_data, s_num_tokens, num_tokens) || !THPVariable_Check(x.p) ||
-      !THPVariable_Check(indices.p) || !THPVariable_Check(weights.p)) {
-    PyErr_Clear();
-    Py_RETURN_NONE;
-  }
+  Ref x, indices, weights;
+  Outcome got;
+  if ((got = get_attr(rank_data, s_x, x)) || (got = get_attr(rank_data, s_indices, indices)) ||
+      (got = get_attr(rank_data, s_weights, weights)) || (got = int_attr(rank_data, s_num_tokens, num_tokens)))
+    return outcome(got);
+  if (!THPVariable_Check(x.p) || !THPVariable_Check(indices.p) || !THPVariable_Check(weights.p)) Py_RETURN_NONE;
   const at::Tensor& xt = THPVariable_Unpack(x.p);
   call[4] = xt.get_device();
   long config[4];
   Ref in_dtype, out_dtype;
-  if (!memo_read(PyTuple_GET_ITEM(args[0], 0), config, in_dtype, out_dtype)) Py_RETURN_NONE;
+  if ((got = memo_read(PyTuple_GET_ITEM(args[0], 0), config, in_dtype, out_dtype))) return outcome(got);
   const int at = memo_find(m, config, call, in_dtype.p, out_dtype.p);
   if (at < 0) Py_RETURN_NONE;
   entry_front(m, at);
   Ref owner(m->entry[0].owner), rings, ring;  // taken here: the lookups below may run Python code, and other threads
   Py_INCREF(owner.p);
-  rings.p = PyObject_GetAttr(owner.p, s_rings);
-  if (!rings || Py_TYPE(rings.p) != &RingsType) {
-    PyErr_Clear();
-    Py_RETURN_NONE;
-  }
+  if ((got = get_attr(owner.p, s_rings, rings))) return outcome(got);
+  if (Py_TYPE(rings.p) != &RingsType) Py_RETURN_NONE;
   ring.p = (PyObject*)rings_find((Rings*)rings.p, xt);
   if (!ring) Py_RETURN_NONE;
   Ring* r = (Ring*)ring.p;
@@ -443,12 +439,9 @@ PyObject* memo_run(Memo* m, PyObject* const* args, Py_ssize_t n) {
   // the caller owns its result: the combine writes straight into a fresh tensor
   at::Tensor y = at::empty({r->T, r->H}, xt.options().dtype(r->out_type));
   int set = 0;
-  switch (ring_forward(r, owner.p, xt, THPVariable_Unpack(indices.p), THPVariable_Unpack(weights.p), nullptr, y.data_ptr(),
-                       set)) {
-    case kNotThisWay: Py_RETURN_NONE;
-    case kError: return nullptr;
-    case kDone: break;
-  }
+  if ((got = ring_forward(r, owner.p, xt, THPVariable_Unpack(indices.p), THPVariable_Unpack(weights.p), nullptr, y.data_ptr(),
+                          set)))
+    return outcome(got);
   return THPVariable_Wrap(num_tokens == r->T ? y : y.narrow(0, 0, num_tokens));
   END_HANDLE_TH_ERRORS
 }

@@ -173,3 +173,30 @@ def test_instances_let_go_of_are_not_kept_by_the_native_path(monkeypatch):
     gc.collect()
     assert len(S._instances) == 1
     assert [r() for r in alive] == [None] * 65 + [S._last[1]]
+
+
+@pytest.mark.parametrize("where", ["cfg", "rank_data", "owner"])
+@pytest.mark.parametrize("raised", [KeyboardInterrupt, MemoryError, AttributeError, TypeError])
+def test_native_path_passes_on_what_is_not_about_an_attribute(where, raised):
+    """An interrupt or a lack of memory inside a lookup reaches the caller; a missing attribute, or one of another kind, is
+    left to the long way (None)."""
+    import types
+
+    from kernel_amd import _lib
+
+    class Raises:
+        def __getattr__(self, name):
+            raise raised(name)
+
+    cfg, rd, rank, world = C.generate_input(8, 2, 64, 8, 5, 0, 8)
+    memo = _lib.host().Memo()
+    memo.remember(cfg, rank, world, 0, 0, -1, Raises() if where == "owner" else types.SimpleNamespace(_rings=None))
+    data = (Raises() if where == "cfg" else cfg, Raises() if where == "rank_data" else rd, rank, world)
+    if raised in (KeyboardInterrupt, MemoryError):
+        with pytest.raises(raised):
+            memo.run(data, 0, 0)
+        if where == "cfg":
+            with pytest.raises(raised):
+                memo.remember(data[0], rank, world, 0, 0, -1, object())
+    else:
+        assert memo.run(data, 0, 0) is None
