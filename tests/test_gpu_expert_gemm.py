@@ -555,20 +555,97 @@ def test_expert_gemm_power_of_two_tall_tiles(gpu_device, options, dtype, H, N):
     close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
 
 
+def tall_tiles_pay(counts, ntile_n):
+    """The kernels' rule: whether tall tiles save some, and whether the plan with them is the faster one by their estimate."""
+    R, plain, tall = sum(counts), sum(-(-c // 256) for c in counts), sum(-(-c // 288) for c in counts)
+    rounds = {n: -(-(-(-n // 8) * ntile_n) // 32) for n in (plain, tall)}
+    if max(counts) * len(counts) > 2.5 * R:
+        pays = 1.1 * rounds[tall] < rounds[plain]
+    else:
+        pays = (288 * tall + R) * rounds[tall] / tall < (288 * plain + R) * rounds[plain] / plain
+    return tall < plain, pays
+
+
+SKEWED = {  # segment tables where tall tiles save some, and whether the kernels take them (8 n-tiles)
+    "popular-tall": ([min(1500, int(1500 / (e + 1) ** 1.2)) for e in range(24)], True),
+    "popular-256": ([int(2500 / (e + 1) ** 1.2) for e in range(24)], False),
+    "alike-tall": ([281] * 36, True),
+    "alike-256": ([257 + (e * 31) % 40 for e in range(30)], False),
+    "lone-tall": ([0, 0, 8193, 0], True),
+    "lone-256": ([0, 288, 0], False),
+    "ends-256": ([288] + [1] * 7 + [0] * 600 + [288], False),
+}
+
+
+@pytest.mark.parametrize("table", SKEWED)
+@pytest.mark.parametrize("fmt", ["16bit", "mx"])
+def test_tall_tiles_on_skewed_segment_tables(gpu_device, options, table, fmt):
+    """Tables on either side of the rule that weighs tall tiles against 256-row ones, as the kernels decide and with tall
+    tiles wherever they save one: the bits of a form that has no tall tiles, and the f32 matmul within the tolerance of
+    the other forms."""
+    counts, tall = SKEWED[table]
+    dtype, H, N = torch.bfloat16, 256, 1920
+    assert tall_tiles_pay(counts, 8) == (True, tall)
+    R, E = sum(counts), len(counts)
+    g = torch.Generator(device=gpu_device).manual_seed(R)
+    w = (torch.randn(E, N, H, device=gpu_device, generator=g) / H ** 0.5).to(dtype)
+    x = torch.randn(R, H, device=gpu_device, generator=g).to(dtype)
+    offsets = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    at = offsets.to(gpu_device)
+    tail = (R, E, H, N, 0, _lib.BF16, torch.cuda.current_stream().cuda_stream)
+    lib = _lib.load()
+    if fmt == "mx":
+        q, s = torch.empty(R, H, dtype=torch.uint8, device=gpu_device), torch.empty(R, H // 128, device=gpu_device)
+        same = torch.arange(R, dtype=torch.int32, device=gpu_device)
+        _lib.check(lib.moe_a2a_dispatch_fp8(x.data_ptr(), _lib.BF16, same.data_ptr(), q.data_ptr(), s.data_ptr(), R, 1, H,
+                                            _lib.FP8_SCALE_POW2, tail[-1]), "moe_a2a_dispatch_fp8")
+        wq, ws = (t.to(gpu_device) for t in V.quantize_weights_fp8(w.cpu(), pow2=True))
+        x = (q.view(torch.float8_e4m3fn).float().view(R, -1, 128) * s[..., None]).view(R, H)
+        w = (wq.view(torch.float8_e4m3fn).float().view(E, N // 128, 128, H // 128, 128) * ws[:, :, None, :, None]).view(E, N, H)
+
+    def gemm(form):
+        options.set("GEMM_TILE", 256)
+        options.set("GEMM_STAGED", form)
+        y = torch.empty(R, N, dtype=dtype, device=gpu_device)
+        if fmt == "mx":
+            _lib.check(lib.moe_a2a_expert_gemm_mx8(q.data_ptr(), s.data_ptr(), wq.data_ptr(), ws.data_ptr(), at.data_ptr(),
+                                                   y.data_ptr(), *tail), "moe_a2a_expert_gemm_mx8")
+        else:
+            _lib.check(lib.moe_a2a_expert_gemm(x.data_ptr(), w.data_ptr(), at.data_ptr(), y.data_ptr(), *tail),
+                       "moe_a2a_expert_gemm")
+        return y
+
+    want = torch.empty(R, N, device=gpu_device)
+    for e in range(E):
+        rows = slice(int(offsets[e]), int(offsets[e + 1]))
+        want[rows] = x[rows].float() @ w[e].float().T
+    decided, forced, none = gemm(0), gemm(4), gemm(3)
+    torch.cuda.synchronize()
+    assert torch.equal(decided.view(torch.int16), none.view(torch.int16))
+    assert torch.equal(forced.view(torch.int16), none.view(torch.int16))
+    close(forced, want.cpu())
+
+
 @pytest.mark.parametrize("Kd", [3728256, 3728320, 4194240])  # the longest rows of a tall tile, one slab more, and more
-def test_expert_gemm_16bit_longest_rows(gpu_device, Kd):
-    """One segment of 288 rows so long that a tile's offsets come to the end of 32 bits: the sum of every row, the last
-    32 among them, whatever tile they fall to.  Tolerance: one rounding to bf16 (2^-9 of a value) and the f32 sum of
-    Kd products of variance 1 / Kd in any order, whose error stays below sqrt(Kd) * 2^-24 * 4 = 5e-4."""
-    R, N = 288, 256
+def test_expert_gemm_16bit_longest_rows(gpu_device, options, Kd):
+    """A segment of 288 rows, which are one tall tile, so long that the tile's offsets come to the end of 32 bits: the sum
+    of every row, the last 32 among them, whatever tile they fall to.  Tolerance: one rounding to bf16 (2^-9 of a value)
+    and the f32 sum of Kd products of variance 1 / Kd in any order, whose error stays below sqrt(Kd) * 2^-24 * 4 = 5e-4."""
+    counts = [288] + [1] * 7
+    R, E, N = sum(counts), len(counts), 8
     gen = torch.Generator(device=gpu_device).manual_seed(Kd)
     x = torch.empty(R, Kd, dtype=torch.bfloat16, device=gpu_device).normal_(generator=gen)
-    w = torch.empty(N, Kd, dtype=torch.bfloat16, device=gpu_device).normal_(0.0, Kd ** -0.5, generator=gen)
-    offsets = torch.tensor([0, R], dtype=torch.int32, device=gpu_device)
+    w = torch.empty(E, N, Kd, dtype=torch.bfloat16, device=gpu_device).normal_(0.0, Kd ** -0.5, generator=gen)
+    offsets = torch.tensor([0] + counts, dtype=torch.int32).cumsum(0).to(torch.int32)
     y = torch.empty(R, N, dtype=torch.bfloat16, device=gpu_device)
-    _lib.check(_lib.load().moe_a2a_expert_gemm(x.data_ptr(), w.data_ptr(), offsets.data_ptr(), y.data_ptr(), R, 1, Kd, N, 0,
+    options.set("GEMM_TILE", 256)
+    options.set("GEMM_STAGED", 4)
+    at = offsets.to(gpu_device)
+    _lib.check(_lib.load().moe_a2a_expert_gemm(x.data_ptr(), w.data_ptr(), at.data_ptr(), y.data_ptr(), R, E, Kd, N, 0,
                                                _lib.BF16, torch.cuda.current_stream().cuda_stream), "moe_a2a_expert_gemm")
     want = torch.zeros(R, N, dtype=torch.float64, device=gpu_device)
     for k in range(0, Kd, 1 << 16):
-        want += (x[:, k:k + (1 << 16)].float() @ w[:, k:k + (1 << 16)].float().T).double()
+        for e in range(E):
+            rows = slice(int(offsets[e]), int(offsets[e + 1]))
+            want[rows] += (x[rows, k:k + (1 << 16)].float() @ w[e, :, k:k + (1 << 16)].float().T).double()
     assert bool(((y.double() - want).abs() <= want.abs() * 2 ** -8 + 5e-4).all())
