@@ -1048,10 +1048,10 @@ static int forward_one_launch(const void* x, const int32_t* indices, const float
 #define FWT3(EL, MD)                                                                                              \
   {                                                                                                               \
     switch (K) {                                                                                                  \
-      case 4: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 4, 1>, grid, block, 0, stream, FWT_ARGS);  \
-      case 6: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 6, 1>, grid, block, 0, stream, FWT_ARGS);  \
-      case 8: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 8, 1>, grid, block, 0, stream, FWT_ARGS);  \
-      default: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 0, 1>, grid, block, 0, stream, FWT_ARGS); \
+      case 4: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 4>, grid, block, 0, stream, FWT_ARGS);  \
+      case 6: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 6>, grid, block, 0, stream, FWT_ARGS);  \
+      case 8: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 8>, grid, block, 0, stream, FWT_ARGS);  \
+      default: return launch(KID_FORWARD_TILE, forward_tile_kernel<EL, MD, 0>, grid, block, 0, stream, FWT_ARGS); \
     }                                                                                                             \
   }
 #define FWT2(EL)                                                        \
@@ -1073,8 +1073,8 @@ static int forward_one_launch(const void* x, const int32_t* indices, const float
 #define FWD4(EPT, VPL, EL, MD)                                                                                   \
   {                                                                                                              \
     if (K == 8)                                                                                                  \
-      return launch(KID_FORWARD_TOKEN, forward_token_kernel<EPT, VPL, EL, MD, 8, 1>, grid, block, 0, stream, FWD_ARGS); \
-    return launch(KID_FORWARD_TOKEN, forward_token_kernel<EPT, VPL, EL, MD, 0, 1>, grid, block, 0, stream, FWD_ARGS); \
+      return launch(KID_FORWARD_TOKEN, forward_token_kernel<EPT, VPL, EL, MD, 8>, grid, block, 0, stream, FWD_ARGS); \
+    return launch(KID_FORWARD_TOKEN, forward_token_kernel<EPT, VPL, EL, MD, 0>, grid, block, 0, stream, FWD_ARGS); \
   }
 #define FWD3(EPT, VPL, EL)                                                      \
   {                                                                             \
