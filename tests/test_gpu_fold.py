@@ -66,3 +66,63 @@ def test_fold_equals_the_rows_read_back_at_large_x(gpu_device, options, T, fp8):
         got.append((y, ata.last.disp_x, ata.last.slot_of_entry, ata.last.meta))
     for a, b in zip(*got):
         assert torch.equal(bits(a), bits(b))
+
+
+def same_values(got, want):
+    """NaN where the other has NaN (whatever its payload), the same bits elsewhere."""
+    got, want = got.cpu(), want.cpu()
+    if not got.is_floating_point():
+        return torch.equal(got, want)
+    return torch.equal(got.isnan(), want.isnan()) and torch.equal(bits(got.nan_to_num()), bits(want.nan_to_num())) \
+        and torch.equal(got.isinf(), want.isinf())
+
+
+def with_specials(x, w):
+    """Infinities of both signs, NaN, the largest and the smallest finite values, zeros of both signs in the rows; zero,
+    tiny and huge weights."""
+    top = torch.finfo(x.dtype).max
+    values = torch.tensor([float("inf"), float("-inf"), float("nan"), top, -top, torch.finfo(x.dtype).tiny, 0.0, -0.0])
+    T, H = x.shape
+    at = torch.arange(T * H).view(T, H)
+    x = torch.where(at % 11 == 3, values[at // 11 % 8].to(x.dtype), x)
+    w = w.clone()
+    w[::3, 0], w[1::5, -1], w[2::7, 0] = 0.0, 1e-30, 3e38
+    return x.contiguous(), w
+
+
+@pytest.mark.parametrize("E,K,H,T", [
+    (16, 2, 512, 7),        # a workgroup per token
+    (256, 8, 1024, 33),
+    (64, 6, 384, 1003),     # a tile of tokens per workgroup
+    (12, 5, 64, 500),
+    (32, 4, 2048, 9000),    # routed by launches of their own, more rows than the caches hold
+])
+@pytest.mark.parametrize("mode", [C.COMBINE_STRICT, C.COMBINE_F32], ids=["strict", "f32"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_infinities_and_nan_through_the_fold(gpu_device, E, K, H, T, mode, dtype):
+    cfg = C.MoEConfig(E, K, H, T + 1, dtype, dtype)
+    x, idx, w = inputs(E, K, H, T, dtype, E + T)
+    x, w = with_specials(x, w)
+    want = V.run_world(cfg, [C.RankData(T, idx, w, x)], stub_kind=C.STUB_EXPERT_FRACTION, combine_mode=mode)
+    ata = HipAllToAll(cfg, 0, 1, stub_kind=C.STUB_EXPERT_FRACTION, combine_mode=mode, fuse_stub=True)
+    y = ata.forward(x.to(gpu_device), idx.to(gpu_device), w.to(gpu_device))
+    torch.cuda.synchronize()
+    assert torch.equal(bits(ata.last.disp_x.cpu()), bits(want["disp_x"]))  # rows are copied, whatever they hold
+    assert same_values(y, want["y"])
+
+
+@pytest.mark.parametrize("E,K,H,T", [(16, 2, 512, 7), (64, 6, 384, 1003), (32, 4, 2048, 9000)])
+@pytest.mark.parametrize("fp8", [True, "pow2"])
+def test_infinities_and_nan_through_the_fp8_fold(gpu_device, options, E, K, H, T, fp8):
+    """Against the form that reads the quantised rows back."""
+    cfg = C.MoEConfig(E, K, H, T + 1, torch.bfloat16, torch.bfloat16)
+    x, idx, w = inputs(E, K, H, T, torch.bfloat16, E + T)
+    x, w = (t.to(gpu_device) for t in with_specials(x, w))
+    idx, got = idx.to(gpu_device), []
+    for two in (1, 0):
+        options.set("TWO_LAUNCHES", two)
+        ata = HipAllToAll(cfg, 0, 1, stub_kind=C.STUB_EXPERT_FRACTION, fp8_dispatch=fp8, fuse_stub=True)
+        y = ata.forward(x, idx, w)
+        got.append((y, ata.last.disp_x, ata.last.disp_scale, ata.last.slot_of_entry, ata.last.meta))
+    torch.cuda.synchronize()
+    assert all(same_values(a, b) for a, b in zip(*got))

@@ -117,3 +117,35 @@ def test_token_counts_in_turn_take_the_short_way(gpu_device, monkeypatch):
     ata.release_buffers()
     _, rd, _, want = cases[0]
     assert same(ata.forward(rd.x, rd.indices, rd.weights), want) and len(ata._bufs) == 1
+
+
+def test_two_threads_share_a_handle(gpu_device):
+    """Two threads call custom_kernel with one configuration, each with token counts of its own in turn, and forward of
+    one host object with results of their own: every result is that of its call."""
+    import threading
+
+    cfg = case(0, 5)[0]
+    cases = {0: [case(0, T) for T in (5, 9, 21)], 1: [case(0, T) for T in (6, 9, 33)]}
+    ata = HipAllToAll(cfg, 0, 8, fuse_stub=True)
+    wrong = []
+
+    def work(me):
+        try:
+            kept = []
+            for i in range(150):
+                _, rd, _, want = cases[me][i % 3]
+                kept.append((custom_kernel((cfg, rd, 0, 8)), want))
+                out = torch.empty_like(kept[-1][0])
+                assert ata.forward(rd.x, rd.indices, rd.weights, out=out) is out
+                kept.append((out, want))
+            torch.cuda.synchronize()
+            wrong.extend(me for y, want in kept if not same(y, want))
+        except Exception as e:  # an assertion in a thread is not seen by itself
+            wrong.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
