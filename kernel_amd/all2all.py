@@ -20,6 +20,7 @@ from __future__ import annotations
 import copy
 import ctypes
 import dataclasses
+import threading
 from typing import Optional, Sequence
 
 import torch
@@ -147,6 +148,7 @@ class HipAllToAll:
         # (T, device) -> two buffer sets and their native record (_host.Ring: which is next, when they were used last)
         self._bufs = {}
         self._rings = _lib.host().Rings()  # those records, where the short way of forward finds them
+        self._making = threading.RLock()  # held while a token count that is new gets its record and its sets
 
     # ---- buffers ---------------------------------------------------------------------
     def _buffers(self, T: int, device, advance: bool = False) -> dict:
@@ -162,24 +164,27 @@ class HipAllToAll:
         self._rings.touch(native)
         if advance:
             native.cur ^= 1
-        if sets[0] is None:
-            # both sets of a new shape are allocated together, so that the second call with this shape
-            # does not meet an allocation either
-            fresh = [self._allocate(T, device), self._allocate(T, device)]
-            for i in (0, 1):  # a call on one set clears the status word of the other (see Dispatched.status)
-                fresh[i]["partner_status"] = fresh[i ^ 1]["status"]
-            sets[:] = fresh
         return sets[native.cur]
 
     def _new_ring(self, T: int, device) -> dict:
+        with self._making:  # threads that meet one new count share what the first of them makes
+            return self._bufs.get((T, device)) or self._make_ring(T, device)
+
+    def _make_ring(self, T: int, device) -> dict:
         while len(self._bufs) >= self.MAX_CACHED_SHAPES:  # a caller with many token counts keeps the recent ones
             oldest = min(self._bufs, key=lambda key: self._bufs[key]["native"].used)
             self._rings.drop(self._bufs.pop(oldest)["native"])
+        # both sets of a new shape are allocated together, so that the second call with this shape
+        # does not meet an allocation either
+        sets = [self._allocate(T, device), self._allocate(T, device)]
+        for i in (0, 1):  # a call on one set clears the status word of the other (see Dispatched.status)
+            sets[i]["partner_status"] = sets[i ^ 1]["status"]
         cfg = self.cfg
         native = _lib.host().Ring(T, cfg.experts_per_token, cfg.hidden_dim, self.world_size, device.index, cfg.in_dtype,
                                   cfg.out_dtype)
         self._rings.add(native)
-        ring = self._bufs[(T, device)] = dict(sets=[None, None], native=native)
+        self._rings.touch(native)
+        ring = self._bufs[(T, device)] = dict(sets=sets, native=native)
         return ring
 
     def _allocate(self, T: int, device) -> dict:
@@ -217,13 +222,12 @@ class HipAllToAll:
     def _bind(self, T: int, device) -> None:
         """Gives the native record of T tokens what ``forward`` needs of the set that comes next: calls that meet that
         set again go the short way."""
-        self._buffers(T, device)
-        ring = self._bufs[(T, device)]
+        ring = self._bufs.get((T, device)) or self._new_ring(T, device)
         native, i = ring["native"], ring["native"].cur ^ 1
         if not native.bound >> i & 1:
             b = ring["sets"][i]
             block = bytes(_lib.ForwardArgs(*self._forward_args(b, None, None, None, None, 0)))
-            native.bind(i, block, b["out"], self._record(b, T))
+            native.bind(i, block, b["out"], self._record(b, T), b)  # the block's pointers live as long as the set
 
     # ---- dispatch --------------------------------------------------------------------
     def dispatch(self, dp_x: torch.Tensor, indices: torch.Tensor,

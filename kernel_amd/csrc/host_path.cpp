@@ -82,6 +82,7 @@ struct Ring {
   moe_a2a_forward_args args[2];
   PyObject* outs[2];
   PyObject* records[2];
+  PyObject* keep[2];  // what the argument blocks point into
 };
 
 PyObject* ring_new(PyTypeObject* type, PyObject* args, PyObject*) {
@@ -98,13 +99,13 @@ PyObject* ring_new(PyTypeObject* type, PyObject* args, PyObject*) {
   return (PyObject*)r;
 }
 
-// bind(set, block, out, record)
+// bind(set, block, out, record, an object that keeps what the block points into)
 PyObject* ring_bind(Ring* r, PyObject* args) {
   int set;
-  PyObject *out, *record;
+  PyObject *out, *record, *keep;
   const char* block;
   Py_ssize_t len;
-  if (!PyArg_ParseTuple(args, "iy#OO", &set, &block, &len, &out, &record)) return nullptr;
+  if (!PyArg_ParseTuple(args, "iy#OOO", &set, &block, &len, &out, &record, &keep)) return nullptr;
   if (set != 0 && set != 1) {
     PyErr_SetString(PyExc_ValueError, "the sets are 0 and 1");
     return nullptr;
@@ -113,11 +114,14 @@ PyObject* ring_bind(Ring* r, PyObject* args) {
     PyErr_SetString(PyExc_ValueError, "the argument block is not a moe_a2a_forward_args");
     return nullptr;
   }
+  if (r->bound >> set & 1) Py_RETURN_NONE;  // by another thread, since the caller looked
   std::memcpy(&r->args[set], block, sizeof(moe_a2a_forward_args));
   Py_INCREF(out);
-  Py_XSETREF(r->outs[set], out);
   Py_INCREF(record);
-  Py_XSETREF(r->records[set], record);
+  Py_INCREF(keep);
+  r->outs[set] = out;
+  r->records[set] = record;
+  r->keep[set] = keep;
   r->bound |= 1 << set;
   Py_RETURN_NONE;
 }
@@ -127,6 +131,7 @@ int ring_clear(Ring* r) {
   for (int i = 0; i < 2; ++i) {
     Py_CLEAR(r->outs[i]);
     Py_CLEAR(r->records[i]);
+    Py_CLEAR(r->keep[i]);
   }
   return 0;
 }
@@ -134,6 +139,7 @@ int ring_traverse(Ring* r, visitproc visit, void* arg) {
   for (int i = 0; i < 2; ++i) {
     Py_VISIT(r->outs[i]);
     Py_VISIT(r->records[i]);
+    Py_VISIT(r->keep[i]);
   }
   return 0;
 }
@@ -171,6 +177,7 @@ Outcome ring_forward(Ring* r, PyObject* owner, const at::Tensor& x, const at::Te
   else if (!PyUnicode_Check(route.p) || PyUnicode_Compare(route.p, s_always) != 0)
     return kNotThisWay;
   if (!PyLong_Check(stub.p)) return kNotThisWay;
+  if (!(r->bound >> (r->cur ^ 1) & 1)) return kNotThisWay;  // (the lookups above may have run Python code)
   set = r->cur ^= 1;
   moe_a2a_forward_args a = r->args[set];  // a copy: the launch runs without the interpreter's lock
   a.x = x.const_data_ptr();

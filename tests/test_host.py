@@ -200,3 +200,36 @@ def test_native_path_passes_on_what_is_not_about_an_attribute(where, raised):
                 memo.remember(data[0], rank, world, 0, 0, -1, object())
     else:
         assert memo.run(data, 0, 0) is None
+
+
+def test_threads_that_meet_a_new_token_count_share_its_buffers(monkeypatch):
+    """Every thread gets sets of the one record: a set that another thread's replaced would be freed under the pointers that
+    the native side keeps of it."""
+    import threading
+    import time
+
+    made = []
+
+    def allocate(self, T, device):
+        time.sleep(0.01)  # other threads run, as they may in any allocation
+        made.append(T)
+        return dict(status=object(), out=object(), number=len(made))
+
+    monkeypatch.setattr(HipAllToAll, "_allocate", allocate)
+    ata = HipAllToAll(C.MoEConfig(8, 2, 64, 8), 0, 8)
+    device = torch.device("cuda:0")
+    start, got = threading.Barrier(6), []
+
+    def work():
+        start.wait()
+        for T in (3, 4, 3):
+            got.append((T, ata._buffers(T, device)))
+
+    threads = [threading.Thread(target=work) for _ in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert sorted(made) == [3, 3, 4, 4] and len(got) == 18 and len(ata._bufs) == 2
+    for T, b in got:
+        assert any(b is s for s in ata._bufs[(T, device)]["sets"])
