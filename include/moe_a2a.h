@@ -280,8 +280,8 @@ int moe_a2a_forward_launches(int T, int K, int H, int max_recv, int in_type, int
  * less than 192 rows on average in a form that requests the weight rows early, for longer ones in a form whose
  * tiles hold up to 288 rows where the segment table makes that the faster plan; MOE_A2A_OPT_GEMM_STAGED = 3
  * forces the former, 4 the latter with 288 rows wherever they save a tile); 32 x 64 tiles that stream the
- * weights when segments are short (R <= 32 * E, R <= 16 * E if Kd % 128 != 0); 128 x 128 output tiles for what is left.  The option
- * MOE_A2A_OPT_GEMM_TILE = 32, 128 or 256 forces one.
+ * weights when segments are short (R <= 32 * E, R <= 16 * E if Kd % 128 != 0); 128 x 128 output tiles for
+ * what is left.  The option MOE_A2A_OPT_GEMM_TILE = 32, 128 or 256 forces one.
  * Padded layout: a segment longer than max_recv (routing raised MOE_A2A_STATUS_OVERFLOW) is
  * multiplied over its first max_recv rows only, so no tile leaves the segment or the buffers.
  */
