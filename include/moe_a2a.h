@@ -276,10 +276,9 @@ int moe_a2a_forward_launches(int T, int K, int H, int max_recv, int in_type, int
  * this is the grouped matrix product a real MoE layer runs there.
  *   x[rows, Kd], weights[E, N, Kd], y[rows, N]: 16-bit elements of elem_type, f32 accumulation,
  *   Kd % 64 == 0, N % 8 == 0, 16-byte aligned.
- * Three kernels with identical results: 256 x 256 tiles (R > 32 * E and N >= 256; for segments of
- * less than 192 rows on average in a form that requests the weight rows early, for longer ones in a form whose
- * tiles hold up to 288 rows where the segment table makes that the faster plan; MOE_A2A_OPT_GEMM_STAGED = 3
- * forces the former, 4 the latter with 288 rows wherever they save a tile); 32 x 64 tiles that stream the
+ * Three kernels with identical results: 256 x 256 tiles (R > 32 * E and N >= 256; they hold up to
+ * 288 rows where the segment table makes that the faster plan; MOE_A2A_OPT_GEMM_STAGED = 3
+ * forces 256 rows, 4 288 rows wherever they save a tile); 32 x 64 tiles that stream the
  * weights when segments are short (R <= 32 * E, R <= 16 * E if Kd % 128 != 0); 128 x 128 output tiles for
  * what is left.  The option MOE_A2A_OPT_GEMM_TILE = 32, 128 or 256 forces one.
  * Padded layout: a segment longer than max_recv (routing raised MOE_A2A_STATUS_OVERFLOW) is
@@ -391,9 +390,9 @@ const char* moe_a2a_kernel_name(int kernel_id);
 #define MOE_A2A_OPT_GEMM_TILE 1     /* 32 | 128 | 256: tile family of the expert GEMM entry points          */
 #define MOE_A2A_OPT_GEMM_STAGED 2   /* 1: register-staged form of the weight-streaming / scaled-MFMA loops;
                                        2: four-wave forms of moe_a2a_expert_gemm_mx8 / _q8 with fp8 rows;
-                                       3 | 4: the eight-wave loops on 256 x 256 tiles with | without early
-                                       requests for the weight rows (4: and with tiles of 288 rows wherever
-                                       they save one, where the loop has such);
+                                       3 | 4: the eight-wave loops on 256 x 256 tiles, tiles of 256 rows
+                                       only | of 288 wherever they save one, where the loop has such; fp8
+                                       rows: with | without early requests for the weight rows;
                                        5: moe_a2a_expert_gemm_q8 with fp8 rows on 256 x 128 tiles           */
 #define MOE_A2A_OPT_COMBINE_LANES 3 /* lanes of a combine workgroup at cache-resident sizes (64 .. 512)     */
 #define MOE_A2A_OPT_COMBINE_VPL 4   /* 2: two row vectors per lane in the combine at cache-resident sizes   */
