@@ -314,8 +314,8 @@ int moe_a2a_expert_gemm_fp8(const void* x_q, const float* x_scale, const void* w
  *     The option MOE_A2A_OPT_GEMM_STAGED = 1 selects the register-staged form of the same
  *     arithmetic (fp8 rows are then dequantised and rounded once to elem_type first).
  *   longer segments, fp8 rows: both operands enter the fp8 matrix instruction as bytes (eight
- *     waves with the 16x16x128 instruction for Kd >= 256, on 256 x 256 tiles or, where those are few and for
- *     N = 128, on 256 x 128 ones, with the same result; the option
+ *     waves with the 16x16x128 instruction for Kd >= 256, on 256 x 256 tiles or, where those are few, for
+ *     N = 128 and for Kd < 512, on 256 x 128 ones, with the same result; the option
  *     MOE_A2A_OPT_GEMM_STAGED = 2, and Kd = 128, take four waves on 128 x 128 tiles with the
  *     32x32x64 one), each 128-wide K block is summed in f32 and folded with
  *     x_scale[row][kb] * w_scale[n / 128][kb]; nothing is rounded before the output.
@@ -391,8 +391,8 @@ const char* moe_a2a_kernel_name(int kernel_id);
 #define MOE_A2A_OPT_GEMM_STAGED 2   /* 1: register-staged form of the weight-streaming / scaled-MFMA loops;
                                        2: four-wave forms of moe_a2a_expert_gemm_mx8 / _q8 with fp8 rows;
                                        3 | 4: the eight-wave loops on 256 x 256 tiles, tiles of 256 rows
-                                       only | of 288 wherever they save one, where the loop has such; fp8
-                                       rows: with | without early requests for the weight rows;
+                                       only | of 288 wherever they save one, where the loop has such;
+                                       power-of-two scales: with | without early requests for the weights;
                                        5: moe_a2a_expert_gemm_q8 with fp8 rows on 256 x 128 tiles           */
 #define MOE_A2A_OPT_COMBINE_LANES 3 /* lanes of a combine workgroup at cache-resident sizes (64 .. 512)     */
 #define MOE_A2A_OPT_COMBINE_VPL 4   /* 2: two row vectors per lane in the combine at cache-resident sizes   */
