@@ -240,6 +240,25 @@ def test_each_kernel_form(gpu_device, options, form, dtype, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", [0, 256, 129, 131, 132, 130])
+@pytest.mark.parametrize("m,n", [(1200, 4352), (1024, 4872), (1301, 2600), (2304, 2304), (640, 6144), (72, 8192), (2816, 3072)])
+def test_every_tile_of_odd_tile_counts(gpu_device, options, form, m, n):
+    """Tile counts that the dies' blocks and bands cut unevenly (a last group of less than four columns, a last band that is
+    short or empty), as the library multiplies them and in every form on 256 rows or columns: no tile is left out or done
+    twice.  f32 sums of 8 x 72 products, rounded once: within 2^-8 of the f32 product and 1e-6."""
+    options.set("GEMM_TILE", form)
+    W, kl = 8, 72
+    g = torch.Generator(device=gpu_device).manual_seed(m + n)
+    x = torch.empty(W, m, kl, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    w = torch.empty(W, n, kl, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    G.HipGemmReduceScatter(W).forward(x, w, None, out=out)
+    want = x.transpose(0, 1).reshape(m, W * kl).float() @ w.transpose(0, 1).reshape(n, W * kl).float().T
+    torch.cuda.synchronize()
+    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6).all())
+
+
+@pytest.mark.gpu
 def test_local_k_with_a_short_last_slab_and_one_rank(gpu_device):
     """Local K = 360 (five slabs of 64 and one of 40, the reference's 2880 / 8), and a world of one."""
     for W, m, n, k in ((8, 64, 2880, 2880), (1, 130, 136, 72)):
