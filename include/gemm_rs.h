@@ -37,10 +37,10 @@ extern "C" {
  *             - outputs of few tiles spread the shards over groups of workgroups, one f32 partial
  *               product per group (what each rank holds before the reduce-scatter), which a second
  *               launch sums: REQUIRED, MOE_A2A_E_WORKSPACE if missing or too small;
- *             - large outputs whose local K is not a multiple of 64 (rows that start off the
- *               128-byte line grid) are first copied onto zero-padded, aligned rows: OPTIONAL --
- *               with NULL or too few bytes the product runs on the rows as they lie, about a
- *               tenth slower;
+ *             - large outputs whose local K is not a multiple of 32 (rows that start off the
+ *               128-byte line grid) are first copied onto zero-padded, aligned rows where that pays:
+ *               OPTIONAL -- with NULL or too few bytes the product runs on the rows as they lie, up to
+ *               a tenth slower;
  *             - 0 bytes for every other shape.
  *           The form, and with it the size, follows MOE_A2A_OPT_GEMM_TILE at the time of the call: a
  *           size queried under one setting belongs to that setting.
