@@ -345,10 +345,9 @@ int moe_a2a_expert_gemm_q8(const void* x, const float* x_scale, const void* w_q,
  * than 256 rows, go through moe_a2a_expert_gemm_q8 (any f32 scale).  The option
  * MOE_A2A_OPT_GEMM_TILE = 256 forces the tiles, 32 / 128 the kernels of moe_a2a_expert_gemm_q8,
  * MOE_A2A_OPT_GEMM_STAGED = 1 the register-staged four-wave loop of the tiles, 2 the four-wave loop
- * with slabs sent memory -> LDS (Kd % 256 == 0), 3 / 4 the eight-wave loop with / without the early
- * requests for the weight rows that segments of 80 to 192 rows on average get by themselves (4: and with
- * tiles of 288 rows wherever they save one; by itself the kernel takes them where the segment table makes
- * that the faster plan).
+ * with slabs sent memory -> LDS (Kd % 256 == 0), 3 / 4 the eight-wave loop without tiles of 288 rows /
+ * with them wherever they save one (by itself the kernel takes them where the segment table makes that
+ * the faster plan).
  * Arguments as for
  * moe_a2a_expert_gemm_q8 with x_scale required.  No counterpart in the reference.
  */
@@ -392,7 +391,6 @@ const char* moe_a2a_kernel_name(int kernel_id);
                                        2: four-wave forms of moe_a2a_expert_gemm_mx8 / _q8 with fp8 rows;
                                        3 | 4: the eight-wave loops on 256 x 256 tiles, tiles of 256 rows
                                        only | of 288 wherever they save one, where the loop has such;
-                                       power-of-two scales: with | without early requests for the weights;
                                        5: moe_a2a_expert_gemm_q8 with fp8 rows on 256 x 128 tiles           */
 #define MOE_A2A_OPT_COMBINE_LANES 3 /* lanes of a combine workgroup at cache-resident sizes (64 .. 512)     */
 #define MOE_A2A_OPT_COMBINE_VPL 4   /* 2: two row vectors per lane in the combine at cache-resident sizes   */

@@ -576,6 +576,27 @@ def test_expert_gemm_power_of_two_tall_tiles(gpu_device, options, dtype, H, N):
     close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
 
 
+@pytest.mark.parametrize("H", [4224, 4608, 8192])  # 33 (four by four does not go), 36 and 64 slabs
+def test_expert_gemm_power_of_two_exponent_table(gpu_device, options, H):
+    """Rows of more scales than are requested ahead of the operands, and of the most that the table holds, with and without
+    the rows behind a tile's 256th: the same bits from both tilings, and the oracle's results."""
+    counts, N, dtype = [1, 65, 0, 129, 256, 257, 288, 300], 256, torch.bfloat16
+    cfg, world, weights = make_counts(counts, H, N, dtype, seed=H)
+    wq, ws = V.quantize_weights_fp8(weights, pow2=True)
+    x, idx, w, rs = concat_world(world, gpu_device)
+    ata = HipAllToAll(cfg, 0, 1, fp8_dispatch="pow2")
+    d = ata.dispatch(x, idx, rs)
+    options.set("GEMM_TILE", 256)
+    options.set("GEMM_STAGED", 4)
+    y = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device), scales_pow2=True).clone()
+    options.set("GEMM_STAGED", 3)
+    y_plain = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device), scales_pow2=True)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), y_plain.view(torch.int16))
+    o = V.run_world(cfg, world, fp8=True, pow2=True)
+    close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
+
+
 def tall_tiles_pay(counts, ntile_n):
     """The kernels' rule: whether tall tiles save some, and whether the plan with them is the faster one by their estimate."""
     R, plain, tall = sum(counts), sum(-(-c // 256) for c in counts), sum(-(-c // 288) for c in counts)
