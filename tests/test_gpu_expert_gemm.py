@@ -532,6 +532,34 @@ def test_expert_gemm_f32_scales_slab_groups(gpu_device, options, H):
     close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
 
 
+STREAM_COUNTS = {"one": [1], "runs": [33, 0, 0, 97, 32], "last": [0] * 17 + [5], "popular": [1] * 9 + [500, 0, 64, 65]}
+
+
+@pytest.mark.parametrize("counts", STREAM_COUNTS.values(), ids=STREAM_COUNTS.keys())
+@pytest.mark.parametrize("slabs", [1, 2, 3, 5])  # the loops take three at a time
+@pytest.mark.parametrize("rows,ntile", [("16bit", 1), ("16bit", 5), ("w8", 1), ("w8", 3), ("fp8", 1), ("fp8", 3)])
+def test_streaming_kernels_cover_every_tile(gpu_device, options, rows, ntile, slabs, counts):
+    """The kernels for a handful of rows per expert deal their tiles out in runs: fewer tiles than runs, counts that the runs
+    do not divide, several tiles of one stripe of weights, and every remainder of the loop over K."""
+    dtype = torch.bfloat16
+    H, N = (64 * slabs, 64 * ntile - 8) if rows == "16bit" else (128 * slabs, 128 * ntile)
+    cfg, world, weights = make_counts(counts, H, N, dtype, seed=H + N)
+    x, idx, w, rs = concat_world(world, gpu_device)
+    ata = HipAllToAll(cfg, 0, 1, fp8_dispatch=rows == "fp8")
+    d = ata.dispatch(x, idx, rs)
+    options.set("GEMM_TILE", 32)
+    if rows == "16bit":
+        y = ata.expert_gemm(d, weights.to(gpu_device))
+        o = V.run_world(cfg, world)
+        close(y, V.expert_gemm(o["disp_x"], o["offsets"], weights, dtype))
+    else:
+        wq, ws = V.quantize_weights_fp8(weights)
+        y = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device))
+        o = V.run_world(cfg, world, fp8=rows == "fp8")
+        close(y, V.expert_gemm_q8(o["disp_x"], o.get("disp_scale") if rows == "fp8" else None, wq, ws, o["offsets"], dtype,
+                                  round_rows=False))
+
+
 TALL_COUNTS = [1, 255, 256, 257, 0, 272, 273, 287, 288, 289, 512, 513, 544, 545, 576, 577, 864, 865]
 
 
