@@ -259,6 +259,27 @@ def test_every_tile_of_odd_tile_counts(gpu_device, options, form, m, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 33, 64])
+@pytest.mark.parametrize("W,n,kl", [
+    (1, 8, 64), (1, 200, 192), (8, 8, 64), (2, 72, 128), (3, 200, 256),  # fewer slabs than are kept in flight, ragged columns
+    (8, 72, 72), (8, 2880, 360), (2, 4104, 1160), (8, 8200, 456),  # rows that end inside a slab
+    (8, 1000, 320), (8, 2880, 384), (4, 4104, 1024), (8, 8200, 512), (8, 32776, 128),  # tiles of 64 columns, of 128, one group
+])
+def test_few_rows(gpu_device, m, W, n, kl):
+    """The weight-streaming form: every row and column, whatever the tile width and the groups, with a bias.
+    f32 sums of W kl products of up to 0.05^2, rounded once: within 2^-8 of the f32 result and 1e-5."""
+    g = torch.Generator(device=gpu_device).manual_seed(m + n + kl)
+    x = torch.empty(W, m, kl, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    w = torch.empty(W, n, kl, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    bias = torch.empty(n, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.01, 0.01, generator=g)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    G.HipGemmReduceScatter(W).forward(x, w, bias, out=out)
+    want = x.transpose(0, 1).reshape(m, W * kl).float() @ w.transpose(0, 1).reshape(n, W * kl).float().T + W * bias.float()
+    torch.cuda.synchronize()
+    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-5).all())
+
+
+@pytest.mark.gpu
 def test_local_k_with_a_short_last_slab_and_one_rank(gpu_device):
     """Local K = 360 (five slabs of 64 and one of 40, the reference's 2880 / 8), and a world of one."""
     for W, m, n, k in ((8, 64, 2880, 2880), (1, 130, 136, 72)):
