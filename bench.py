@@ -700,8 +700,8 @@ def moe_layer_leg(torch, lib, contract, wl, tensors, main, dev, mode, args):
     with torch.cuda.stream(main):
         step.ey = torch.empty(T * K, H, dtype=cfg.out_dtype, device=dev)
         d, ey, y = step()
-        # (the clocks take up to 0.4 s to settle under this stream of weights: 5.4 ms per launch until then, 3.9 after)
-        spin_up(main, step, 0.8)
+        # (the clocks take up to 1.2 s to settle under this stream of weights: 4.9 ms per launch until then, 3.9 after)
+        spin_up(main, step, 2.0)
         per = kernel_times(lib, lambda n: [step() for _ in range(n)], steps, torch)
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         e0.record(main)
