@@ -532,6 +532,32 @@ def test_expert_gemm_f32_scales_slab_groups(gpu_device, options, H):
     close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
 
 
+@pytest.mark.parametrize("rows", [20, 22, 23, 25, 26, 32, 33])
+@pytest.mark.parametrize("form,E,H,N", [("16bit", 64, 2880, 3072), ("16bit", 64, 3072, 2944), ("16bit", 65, 512, 520),
+                                        ("fp8", 65, 512, 512), ("fp8", 33, 512, 256), ("pow2", 65, 512, 512)])
+def test_either_side_of_the_streaming_kernels(gpu_device, form, E, H, N, rows):
+    """Mean lengths around where the library goes over from the kernels for a handful of rows to tiles of 256 rows."""
+    dtype = torch.bfloat16
+    counts = [rows + (e * 7) % 5 - 2 for e in range(E)]
+    counts[-1] += rows * E - sum(counts)
+    cfg, world, weights = make_counts(counts, H, N, dtype, seed=H + rows)
+    x, idx, w, rs = concat_world(world, gpu_device)
+    ata = HipAllToAll(cfg, 0, 1, fp8_dispatch={"fp8": True, "pow2": "pow2"}.get(form, False))
+    d = ata.dispatch(x, idx, rs)
+    if form == "16bit":
+        y = ata.expert_gemm(d, weights.to(gpu_device))
+        rows_x, w32 = d.disp_x.float(), weights.to(gpu_device).float()
+    else:
+        wq, ws = V.quantize_weights_fp8(weights, pow2=form == "pow2")
+        y = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device), scales_pow2=form == "pow2")
+        o = V.run_world(cfg, world, fp8=True, pow2=form == "pow2")
+        close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
+        return
+    off = d.offsets.tolist()
+    want = torch.cat([rows_x[off[e]:off[e + 1]] @ w32[e].T for e in range(E)])  # f32 on the GPU
+    close(y, want.cpu())
+
+
 STREAM_COUNTS = {"one": [1], "runs": [33, 0, 0, 97, 32], "last": [0] * 17 + [5], "popular": [1] * 9 + [500, 0, 64, 65]}
 
 
