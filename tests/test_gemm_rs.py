@@ -280,6 +280,37 @@ def test_few_rows(gpu_device, m, W, n, kl):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form,W,m", [(0, 4, 64), (0, 1, 5), (256, 4, 392), (129, 4, 392), (131, 4, 392), (132, 4, 392),
+                                      (130, 4, 392), (128, 4, 392), (32, 4, 392)])
+@pytest.mark.parametrize("kl", [72, 352, 360, 456])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_non_finite_elements_of_ragged_shards(gpu_device, options, dtype, kl, form, W, m):
+    """Infinities and NaN in the columns that a last slab which starts early shares with the one before (and elsewhere), in
+    either operand, padded and in place: NaN and infinite of the same sign exactly where the f32 product is, and the other
+    results as everywhere (f32 sums rounded once: 2^-8 or 2^-11 of the result, and 1e-6)."""
+    options.set("GEMM_TILE", form)
+    n, inf, nan = 600, float("inf"), float("nan")
+    shared = range(kl - 64, kl // 64 * 64)  # the first and last of these, and a column behind them
+    g = torch.Generator(device=gpu_device).manual_seed(kl + form)
+    x = torch.empty(W, m, kl, dtype=dtype, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    w = torch.empty(W, n, kl, dtype=dtype, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    for i, (col, value) in enumerate([(shared[0], inf), (shared[-1], -inf), (shared[0], nan), (kl - 1, inf), (0, -inf)]):
+        w[i % W, 7 + 113 * i, col] = value
+    x[W - 1, m // 3, shared[-1]] = inf
+    x[0, m - 1, shared[0]] = nan
+    x[0, 0, shared[0]] = -inf
+    want = x.transpose(0, 1).reshape(m, W * kl).float() @ w.transpose(0, 1).reshape(n, W * kl).float().T
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for pad_ragged in (True, False):
+        out = G.HipGemmReduceScatter(W, pad_ragged=pad_ragged).forward(x, w).float()
+        torch.cuda.synchronize()
+        assert torch.equal(out.isnan(), want.isnan()), pad_ragged
+        assert torch.equal(out.isposinf(), want.isposinf()) and torch.equal(out.isneginf(), want.isneginf()), pad_ragged
+        finite = want.isfinite()
+        assert bool(((out - want).abs() <= want.abs() * ulp + 1e-6)[finite].all()), pad_ragged
+
+
+@pytest.mark.gpu
 def test_local_k_with_a_short_last_slab_and_one_rank(gpu_device):
     """Local K = 360 (five slabs of 64 and one of 40, the reference's 2880 / 8), and a world of one."""
     for W, m, n, k in ((8, 64, 2880, 2880), (1, 130, 136, 72)):
