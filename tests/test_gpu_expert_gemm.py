@@ -511,11 +511,12 @@ def test_expert_gemm_f32_scales_wide_tiles(gpu_device, options, dtype, H, N, ear
     close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
 
 
-@pytest.mark.parametrize("H", [512, 640, 768, 896, 1024])  # the rows' scales come in groups of four slabs: remainders 0..3
-def test_expert_gemm_f32_scales_slab_groups(gpu_device, options, H):
+@pytest.mark.parametrize("counts", [[1, 64, 65, 128, 129, 193, 256, 257, 0, 300], [1]], ids=["segments", "one-row"])
+@pytest.mark.parametrize("H", [256, 384, 512, 640, 768, 896, 1024])  # the rows' scales come in groups of four slabs: less than
+def test_expert_gemm_f32_scales_slab_groups(gpu_device, options, H, counts):  # a group, and remainders 0..3
     """fp8 with f32 scales on 256 x 256 tiles around the groups in which the rows' scales travel (rows of scales off the grid
     of 16 bytes among them), against the 256 x 128 tiles, which take them slab by slab: the same bits."""
-    counts, N, dtype = [1, 64, 65, 128, 129, 193, 256, 257, 0, 300], 384, torch.bfloat16
+    N, dtype = 384, torch.bfloat16
     cfg, world, weights = make_counts(counts, H, N, dtype, seed=H)
     wq, ws = V.quantize_weights_fp8(weights)
     x, idx, w, rs = concat_world(world, gpu_device)
