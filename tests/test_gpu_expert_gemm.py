@@ -559,6 +559,34 @@ def test_either_side_of_the_streaming_kernels(gpu_device, form, E, H, N, rows):
     close(y, want.cpu())
 
 
+def launched(lib, call):
+    """Names of the kernels that call() launches."""
+    import ctypes
+    assert lib.moe_a2a_timer_begin(8) == 0
+    assert call() == 0
+    torch.cuda.synchronize()
+    ids, us = (ctypes.c_int * 8)(), (ctypes.c_float * 8)()
+    return [lib.moe_a2a_kernel_name(ids[i]).decode() for i in range(lib.moe_a2a_timer_end(ids, us, 8))]
+
+
+@pytest.mark.parametrize("E,Kd,N,kernels", [
+    (64, 2880, 3072, {16: "expert_gemm_skinny", 17: "expert_gemm_wide", 21: "expert_gemm_wide"}),  # 1.05 GiB of weights
+    (64, 3072, 2944, {25: "expert_gemm_skinny", 26: "expert_gemm_wide"}),  # 1.08 GiB, the rows on the grid of 128 columns
+    (8, 576, 512, {16: "expert_gemm_skinny", 17: "expert_gemm", 32: "expert_gemm", 33: "expert_gemm_wide"}),
+    (8, 512, 512, {32: "expert_gemm_skinny", 33: "expert_gemm_wide"}),
+])
+def test_16bit_kernel_by_rows_per_expert(gpu_device, E, Kd, N, kernels):
+    lib = _lib.load()
+    w = torch.zeros(E, N, Kd, dtype=torch.bfloat16, device=gpu_device)
+    for rows, name in kernels.items():
+        R = rows * E
+        x = torch.zeros(R, Kd, dtype=torch.bfloat16, device=gpu_device)
+        y = torch.empty(R, N, dtype=torch.bfloat16, device=gpu_device)
+        off = torch.arange(0, R + 1, rows, dtype=torch.int32, device=gpu_device)
+        assert launched(lib, lambda: lib.moe_a2a_expert_gemm(x.data_ptr(), w.data_ptr(), off.data_ptr(), y.data_ptr(), R, E, Kd, N,
+                                                             0, _lib.BF16, torch.cuda.current_stream().cuda_stream)) == [name], rows
+
+
 STREAM_COUNTS = {"one": [1], "runs": [33, 0, 0, 97, 32], "last": [0] * 17 + [5], "popular": [1] * 9 + [500, 0, 64, 65]}
 
 
