@@ -258,6 +258,38 @@ def test_every_tile_of_odd_tile_counts(gpu_device, options, form, m, n):
     assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6).all())
 
 
+def launched(lib, call):
+    """Names of the kernels that call() launches."""
+    assert lib.moe_a2a_timer_begin(8) == 0
+    call()
+    torch.cuda.synchronize()
+    ids, us = (ctypes.c_int * 8)(), (ctypes.c_float * 8)()
+    return [lib.moe_a2a_kernel_name(ids[i]).decode() for i in range(lib.moe_a2a_timer_end(ids, us, 8))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (2816, 2944, 2048, "gemm_rs_narrow"),  # 132 wide tiles, but one round of 253 narrow ones
+    (4300, 1900, 1088, "gemm_rs_narrow"),  # the same off the grid of 128-byte lines, ragged in both directions
+    (1408, 5504, 2048, "gemm_rs_narrow"),  # 132 wide tiles, two rounds of narrow ones with 128 rows in use
+    (1408, 5504, 4608, "gemm_rs_wide"),  # the same with a longer K
+    (1280, 6656, 2048, "gemm_rs_wide"),  # 130 wide tiles, three rounds of 128 rows
+    (264, 16640, 2048, "gemm_rs_wide"),  # few rows
+    (2048, 4096, 2048, "gemm_rs_narrow"),  # 128
+])
+def test_tile_width_where_wide_tiles_begin(gpu_device, m, n, k, kernel):
+    """Either side of the rules that choose the tiles, by the kernel that is launched, and its results: f32 sums of k products
+    of up to 0.05^2, rounded once, within 2^-8 of the f32 product and 1e-5."""
+    W = 8
+    g = torch.Generator(device=gpu_device).manual_seed(m + n + k)
+    x = torch.empty(W, m, k // W, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    w = torch.empty(W, n, k // W, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    assert launched(_lib.load(), lambda: G.HipGemmReduceScatter(W).forward(x, w, None, out=out)) == [kernel]
+    want = x.transpose(0, 1).reshape(m, k).float() @ w.transpose(0, 1).reshape(n, k).float().T
+    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-5).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 33, 64])
 @pytest.mark.parametrize("W,n,kl", [
