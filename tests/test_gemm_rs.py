@@ -146,6 +146,16 @@ def test_host_side_argument_checks():
     assert lib.gemm_rs_workspace_bytes(64, 64, 100, 8) == 0  # invalid shape: no size
 
 
+@pytest.mark.parametrize("m,n,k,groups", [
+    (496, 8192, 12288, 2), (1024, 3456, 9728, 2), (720, 4736, 9216, 2),  # not one group of tiles with 128 rows in use
+    (584, 2432, 24576, 4), (512, 4096, 12288, 4), (128, 4096, 16896, 8), (2048, 2880, 2880, 1), (1088, 5184, 3584, 1),
+])
+def test_groups_of_shards(m, n, k, groups):
+    """Groups that the 256 x 128 tiles spread the shards over, by the room for their partial products: the fastest of 1, 2, 4
+    and 8 where these were timed one against the other."""
+    assert _lib.load().gemm_rs_workspace_bytes(m, n, k, 8) == (groups * m * n * 4 if groups > 1 else 0)
+
+
 def test_no_cpu_path():
     x, w, b = G.generate_input(0, 1, 8, 8, 64, True, 1)
     with pytest.raises(RuntimeError):
