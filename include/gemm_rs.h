@@ -37,6 +37,9 @@ extern "C" {
  *             - outputs of few tiles spread the shards over groups of workgroups, one f32 partial
  *               product per group (what each rank holds before the reduce-scatter), which a second
  *               launch sums: REQUIRED, MOE_A2A_E_WORKSPACE if missing or too small;
+ *             - the same where it pays although the tiles fill most of the chip (160 or more of 256 x 128):
+ *               OPTIONAL -- with NULL or too few bytes all shards are summed by one workgroup per tile, up
+ *               to a fifth slower;
  *             - large outputs whose local K is not a multiple of 32 (rows that start off the
  *               128-byte line grid) are first copied onto zero-padded, aligned rows where that pays:
  *               OPTIONAL -- with NULL or too few bytes the product runs on the rows as they lie, up to

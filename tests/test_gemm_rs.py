@@ -301,6 +301,34 @@ def test_tile_width_where_wide_tiles_begin(gpu_device, m, n, k, kernel):
 
 
 @pytest.mark.gpu
+def test_partial_products_are_optional_for_many_tiles(gpu_device):
+    """185 tiles of 256 x 128 with shards long enough that groups of them pay: the call is accepted without a workspace, with
+    one that is too small and with one off its alignment, and then sums all shards in one place.  f32 sums of k products
+    of up to 0.05^2, rounded once: within 2^-8 of the f32 product and 2e-5."""
+    lib, W, m, n, k = _lib.load(), 8, 1176, 4672, 20160
+    g = torch.Generator(device=gpu_device).manual_seed(3)
+    x = torch.empty(W, m, k // W, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    w = torch.empty(W, n, k // W, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    want = x.transpose(0, 1).reshape(m, k).float() @ w.transpose(0, 1).reshape(n, k).float().T
+    need = lib.gemm_rs_workspace_bytes(m, n, k, W)
+    assert need >= 2 * m * n * 4
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=gpu_device)
+    outs = []
+    for at, size, kernels in ((None, 0, ["gemm_rs_narrow"]), (ws.data_ptr(), need - 1, ["gemm_rs_narrow"]),
+                              (ws.data_ptr() + 8, need, ["gemm_rs_narrow"]),
+                              (ws.data_ptr(), need, ["gemm_rs_narrow", "gemm_rs_reduce"])):
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+
+        def call():
+            assert lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, k, W, 0, 0, _lib.BF16, at, size,
+                                       torch.cuda.current_stream().cuda_stream) == 0
+        assert launched(lib, call) == kernels
+        assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 33, 64])
 @pytest.mark.parametrize("W,n,kl", [
     (1, 8, 64), (1, 200, 192), (8, 8, 64), (2, 72, 128), (3, 200, 256),  # fewer slabs than are kept in flight, ragged columns
