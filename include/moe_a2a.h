@@ -341,7 +341,7 @@ int moe_a2a_expert_gemm_q8(const void* x, const float* x_scale, const void* w_q,
  * travel memory -> LDS directly).  y = sum over K blocks of
  * x_scale * w_scale * (q_x . q_w) in f32, one rounding to elem_type.  ONLY the exponent field of a
  * scale is used: a scale that is not a power of two is silently taken as the power of two below
- * it.  Segments of at most 22 to 32 rows on average (a decode step), and other Kd on segments shorter
+ * it.  Segments of at most 32 rows on average (a decode step), and other Kd on segments shorter
  * than 256 rows, go through moe_a2a_expert_gemm_q8 (any f32 scale).  The option
  * MOE_A2A_OPT_GEMM_TILE = 256 forces the tiles, 32 / 128 the kernels of moe_a2a_expert_gemm_q8,
  * MOE_A2A_OPT_GEMM_STAGED = 1 the register-staged four-wave loop of the tiles, 2 the four-wave loop

@@ -559,6 +559,26 @@ def test_either_side_of_the_streaming_kernels(gpu_device, form, E, H, N, rows):
     close(y, want.cpu())
 
 
+@pytest.mark.parametrize("rows", [8, 23, 25, 32])
+@pytest.mark.parametrize("E,H,N", [(65, 512, 512), (129, 256, 256), (8, 640, 128)])
+def test_short_segments_take_any_scale(gpu_device, E, H, N, rows):
+    """Up to 32 rows per expert the entry point for power-of-two scales multiplies with scales as they are: the bits of the one
+    for any f32 scale."""
+    dtype = torch.bfloat16
+    cfg, world, weights = make_counts([rows] * E, H, N, dtype, seed=E + rows)
+    wq, ws = V.quantize_weights_fp8(weights)  # scales with a mantissa
+    assert bool((torch.frexp(ws)[0] != 0.5).any())
+    x, idx, w, rs = concat_world(world, gpu_device)
+    ata = HipAllToAll(cfg, 0, 1, fp8_dispatch=True)
+    d = ata.dispatch(x, idx, rs)
+    y = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device), scales_pow2=True).clone()
+    y_any = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device))
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), y_any.view(torch.int16))
+    o = V.run_world(cfg, world, fp8=True)
+    close(y, V.expert_gemm_q8(o["disp_x"], o["disp_scale"], wq, ws, o["offsets"], dtype, round_rows=False))
+
+
 def launched(lib, call):
     """Names of the kernels that call() launches."""
     import ctypes
