@@ -607,6 +607,29 @@ def test_16bit_kernel_by_rows_per_expert(gpu_device, E, Kd, N, kernels):
                                                              0, _lib.BF16, torch.cuda.current_stream().cuda_stream)) == [name], rows
 
 
+@pytest.mark.parametrize("staged,rows,name", [(0, 22, "expert_gemm_skinny"), (0, 25, "expert_gemm_f8"), (3, 25, "expert_gemm_f8"),
+                                              (4, 25, "expert_gemm_f8"), (5, 25, "expert_gemm_f8"),
+                                              (1, 25, "expert_gemm_skinny"), (2, 25, "expert_gemm_skinny"),
+                                              (2, 33, "expert_gemm_f8")])
+@pytest.mark.parametrize("entry", ["q8", "mx8"])
+def test_fp8_kernel_by_rows_per_expert_and_option(gpu_device, options, entry, staged, rows, name):
+    """The options that force a form of the eight-wave tiles leave them where they are taken by default; those of the four-wave
+    and register-staged forms leave the border of 32 rows."""
+    lib, E, Kd, N = _lib.load(), 65, 512, 512
+    if entry == "mx8" and rows > 32:
+        name = "expert_gemm_mx"
+    options.set("GEMM_STAGED", staged)
+    R = rows * E
+    x = torch.zeros(R, Kd, dtype=torch.uint8, device=gpu_device)
+    w = torch.zeros(E, N, Kd, dtype=torch.uint8, device=gpu_device)
+    xs, ws = torch.ones(R, Kd // 128, device=gpu_device), torch.ones(E, N // 128, Kd // 128, device=gpu_device)
+    y = torch.empty(R, N, dtype=torch.bfloat16, device=gpu_device)
+    off = torch.arange(0, R + 1, rows, dtype=torch.int32, device=gpu_device)
+    f = getattr(lib, "moe_a2a_expert_gemm_" + entry)
+    assert launched(lib, lambda: f(x.data_ptr(), xs.data_ptr(), w.data_ptr(), ws.data_ptr(), off.data_ptr(), y.data_ptr(), R, E,
+                                   Kd, N, 0, _lib.BF16, torch.cuda.current_stream().cuda_stream)) == [name]
+
+
 STREAM_COUNTS = {"one": [1], "runs": [33, 0, 0, 97, 32], "last": [0] * 17 + [5], "popular": [1] * 9 + [500, 0, 64, 65]}
 
 
