@@ -333,20 +333,26 @@ def test_partial_products_are_optional_for_many_tiles(gpu_device):
 @pytest.mark.parametrize("W,n,kl", [
     (1, 8, 64), (1, 200, 192), (8, 8, 64), (2, 72, 128), (3, 200, 256),  # fewer slabs than are kept in flight, ragged columns
     (8, 72, 72), (8, 2880, 360), (2, 4104, 1160), (8, 8200, 456),  # rows that end inside a slab
-    (8, 1000, 320), (8, 2880, 384), (4, 4104, 1024), (8, 8200, 512), (8, 32776, 128),  # tiles of 64 columns, of 128, one group
+    (8, 1000, 320), (8, 2880, 384), (4, 4104, 1024), (8, 8200, 512), (8, 32760, 128),  # tiles of 64 columns, of 128, one group
+    (1, 200, 200), (8, 32760, 72), (8, 32776, 128),  # one group of rows that end inside a slab; more columns: 256 x 256 tiles
 ])
-def test_few_rows(gpu_device, m, W, n, kl):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_few_rows(gpu_device, dtype, m, W, n, kl):
     """The weight-streaming form: every row and column, whatever the tile width and the groups, with a bias.
-    f32 sums of W kl products of up to 0.05^2, rounded once: within 2^-8 of the f32 result and 1e-5."""
+    f32 sums of W kl products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 result and 1e-5."""
     g = torch.Generator(device=gpu_device).manual_seed(m + n + kl)
-    x = torch.empty(W, m, kl, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
-    w = torch.empty(W, n, kl, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
-    bias = torch.empty(n, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.01, 0.01, generator=g)
-    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
-    G.HipGemmReduceScatter(W).forward(x, w, bias, out=out)
+    x = torch.empty(W, m, kl, dtype=dtype, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    w = torch.empty(W, n, kl, dtype=dtype, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
+    bias = torch.empty(n, dtype=dtype, device=gpu_device).uniform_(-0.01, 0.01, generator=g)
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
+    kernels = launched(_lib.load(), lambda: G.HipGemmReduceScatter(W).forward(x, w, bias, out=out))
+    groups = _lib.load().gemm_rs_workspace_bytes(m, n, W * kl, W) // (4 * m * n)
+    assert kernels[0] == ("gemm_rs_tile" if n <= 32768 else "gemm_rs_wide") and kernels[1:] in ([], ["gemm_rs_reduce"])
+    assert groups or len(kernels) == 1
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     want = x.transpose(0, 1).reshape(m, W * kl).float() @ w.transpose(0, 1).reshape(n, W * kl).float().T + W * bias.float()
     torch.cuda.synchronize()
-    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-5).all())
+    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5).all())
 
 
 @pytest.mark.gpu

@@ -217,7 +217,7 @@ def test_expert_gemm_block_quantised_weights(gpu_device, options, E, K, T, H, N,
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("padded", [False, True], ids=["compact", "padded"])
-@pytest.mark.parametrize("form", [4, 3, 2, 1], ids=["eight", "eight-early-b", "direct", "staged"])
+@pytest.mark.parametrize("form", [4, 3, 2, 1], ids=["eight", "eight-256-rows", "direct", "staged"])
 def test_expert_gemm_power_of_two_scales(gpu_device, options, E, K, T, H, N, W, zipf, dtype, padded, form):
     """fp8 rows and fp8 weights whose scales are powers of two, multiplied by the fp8 matrix
     instruction with the scales as its block exponents, against the f32 matmul of the
@@ -455,20 +455,19 @@ def walk_cases():
 
 
 @pytest.mark.parametrize("name,counts", walk_cases(), ids=[c[0] for c in walk_cases()])
-@pytest.mark.parametrize("fmt", ["16bit", "16bit-early-b", "mx", "mx-early-b", "f32scale"])
+@pytest.mark.parametrize("fmt", ["16bit", "16bit-256-rows", "mx", "mx-256-rows", "f32scale"])
 @pytest.mark.parametrize("N", [256, 640])
 def test_eight_wave_tile_walk_on_odd_segment_tables(gpu_device, options, name, counts, fmt, N):
     """The eight-wave kernels give every expert's m-tiles to one die's workgroups, in groups of at
     most four.  Segment tables that stress that walk: one expert with many tiles, tile-exact and
     one-row segments between runs of empty experts, the largest expert count, rows only at the two
-    ends; one n-tile and a ragged last n-tile; each operand format's eight-wave kernel forced, the two with
-    two slab buffers in both forms (the rows of the weights requested before the slab's last quarter, or
-    early, behind a second barrier, as short segments get them by default)."""
+    ends; one n-tile and a ragged last n-tile; each operand format's eight-wave kernel forced, the two that have
+    tiles of 288 rows with these wherever they save one and without."""
     dtype, H = torch.bfloat16, 256
-    fmt, _, early = fmt.partition("-")
+    fmt, _, plain = fmt.partition("-")
     options.set("GEMM_TILE", "128" if fmt == "f32scale" else "256")
     if fmt != "f32scale":
-        options.set("GEMM_STAGED", 3 if early else 4)
+        options.set("GEMM_STAGED", 3 if plain else 4)
     cfg, world, weights = make_counts(counts, H, N, dtype, seed=len(counts) + N)
     x, idx, w, rs = concat_world(world, gpu_device)
     fp8 = {"16bit": False, "mx": "pow2", "f32scale": True}[fmt]
@@ -487,10 +486,9 @@ def test_eight_wave_tile_walk_on_odd_segment_tables(gpu_device, options, name, c
     close(y, want)
 
 
-@pytest.mark.parametrize("early", [False, True], ids=["late-b", "early-b"])
-@pytest.mark.parametrize("H,N", [(256, 256), (384, 640), (1408, 128)])  # two, three and eleven slabs; half a tile
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-def test_expert_gemm_f32_scales_wide_tiles(gpu_device, options, dtype, H, N, early):
+@pytest.mark.parametrize("H,N", [(256, 256), (384, 640), (512, 640), (640, 256), (1408, 128)])  # two, three, four, five and
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])  # eleven slabs; half a tile
+def test_expert_gemm_f32_scales_wide_tiles(gpu_device, options, dtype, H, N):
     """fp8 rows and weights with f32 scales on 256 x 256 tiles: segments of 1 row, at, below and above a wave's half
     (64 rows), a wave (128), 192 and a tile (256), and several tiles.  The partial sums are folded block by block in the
     order of the 256 x 128 tiles: the same bits, and the f32 matmul within the tolerance of the other forms."""
@@ -501,7 +499,7 @@ def test_expert_gemm_f32_scales_wide_tiles(gpu_device, options, dtype, H, N, ear
     ata = HipAllToAll(cfg, 0, 1, fp8_dispatch=True)
     d = ata.dispatch(x, idx, rs)
     options.set("GEMM_TILE", 128)
-    options.set("GEMM_STAGED", 3 if early else 4)
+    options.set("GEMM_STAGED", 4)
     y = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device)).clone()
     options.set("GEMM_STAGED", 5)
     y_narrow = ata.expert_gemm(d, wq.to(gpu_device), w_scale=ws.to(gpu_device))
@@ -658,6 +656,65 @@ def test_streaming_kernels_cover_every_tile(gpu_device, options, rows, ntile, sl
                                   round_rows=False))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("form", ["16bit", "fp8", "pow2"])
+def test_results_stored_non_temporally(gpu_device, options, form, dtype):
+    """More than 256 MiB of weights under segments of less than 192 rows: the tiles of 256 rows store their results past the
+    caches.  The same bits as from half of the experts at a time, whose results are stored as usual, and the f32 product."""
+    H, lengths = 1024, [60, 1, 64, 65, 129, 47, 96, 31]
+    E, per = (144, 2) if form == "16bit" else (272, 1)
+    N = H
+    assert E * N * H * per > 256 << 20
+    counts = [lengths[e % 8] for e in range(E)]
+    pow2 = form == "pow2"
+    g = torch.Generator(device=gpu_device).manual_seed(5)
+    w = torch.randn(E, N, H, device=gpu_device, generator=g)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    if form == "16bit":
+        w = w.to(dtype)
+        w32 = w.float()
+    else:
+        w = (w * 64).clamp_(-448, 448).to(torch.float8_e4m3fn)
+        scale = lambda *shape: (torch.exp2(torch.randint(-7, -5, shape, device=gpu_device, generator=g).float()) if pow2
+                                else 0.01 * (1 + torch.rand(shape, device=gpu_device, generator=g)))
+        ws = scale(E, N // 128, H // 128)
+        w32 = w.float() * ws.repeat_interleave(128, 1).repeat_interleave(128, 2)
+    R = sum(counts)
+    x = torch.randn(R, H, device=gpu_device, generator=g)
+    if form == "16bit":
+        x = x.to(dtype)
+        x32 = x.float()
+    else:
+        x = (x * 64).clamp_(-448, 448).to(torch.float8_e4m3fn)
+        xs = scale(R, H // 128)
+        x32 = x.float() * xs.repeat_interleave(128, 1)
+    options.set("GEMM_TILE", 256 if form != "fp8" else 128)
+    options.set("GEMM_STAGED", 3)
+
+    def product(rows, off, experts, first):
+        y = torch.empty(rows, N, dtype=dtype, device=gpu_device)
+        et = _lib.BF16 if dtype == torch.bfloat16 else _lib.F16
+        tail = (off.data_ptr(), y.data_ptr(), rows, experts, H, N, 0, et, stream)
+        if form == "16bit":
+            rc = lib.moe_a2a_expert_gemm(x.data_ptr(), w[first].data_ptr(), *tail)
+        else:
+            f = lib.moe_a2a_expert_gemm_mx8 if pow2 else lib.moe_a2a_expert_gemm_q8
+            rc = f(x.data_ptr(), xs.data_ptr(), w[first].data_ptr(), ws[first].data_ptr(), *tail)
+        assert rc == 0
+        return y
+
+    off = torch.tensor([0] + counts, device=gpu_device).cumsum(0).to(torch.int32)
+    y = product(R, off, E, 0)
+    # half of the experts at a time: less than 256 MiB, stored as usual (the offsets of the second half start behind the first)
+    h, mid = E // 2, int(off[E // 2])
+    usual = torch.cat([product(R, off[:h + 1].contiguous(), h, 0)[:mid], product(R, off[h:].contiguous(), E - h, h)[mid:]])
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), usual.view(torch.int16))
+    o = off.tolist()
+    want = torch.cat([x32[o[e]:o[e + 1]] @ w32[e].T for e in range(E)])
+    close(y, want.cpu())
+
+
 TALL_COUNTS = [1, 255, 256, 257, 0, 272, 273, 287, 288, 289, 512, 513, 544, 545, 576, 577, 864, 865]
 
 
@@ -684,8 +741,7 @@ def test_expert_gemm_16bit_tall_tiles(gpu_device, options, dtype, H, N):
 @pytest.mark.parametrize("H,N", [(256, 256), (384, 640), (1408, 128)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 def test_expert_gemm_power_of_two_tall_tiles(gpu_device, options, dtype, H, N):
-    """The same segments through the kernel with power-of-two scales, with the same bits as its form for short segments,
-    which has tiles of 256 rows only."""
+    """The same segments through the kernel with power-of-two scales, with the same bits as with tiles of 256 rows only."""
     cfg, world, weights = make_counts(TALL_COUNTS, H, N, dtype, seed=H + N)
     wq, ws = V.quantize_weights_fp8(weights, pow2=True)
     x, idx, w, rs = concat_world(world, gpu_device)
