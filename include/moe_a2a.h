@@ -276,11 +276,11 @@ int moe_a2a_forward_launches(int T, int K, int H, int max_recv, int in_type, int
  * this is the grouped matrix product a real MoE layer runs there.
  *   x[rows, Kd], weights[E, N, Kd], y[rows, N]: 16-bit elements of elem_type, f32 accumulation,
  *   Kd % 64 == 0, N % 8 == 0, 16-byte aligned.
- * Three kernels with identical results: 256 x 256 tiles (R > 32 * E and N >= 256; they hold up to
+ * Three kernels with identical results: 32 x 64 tiles that stream the weights when segments are
+ * short (R <= 32 * E, 25 * E with more than 1 GiB of weights, 16 * E if Kd % 128 != 0); 256 x 256
+ * tiles for longer ones (N >= 256, and R > 32 * E or more than 1 GiB of weights; they hold up to
  * 288 rows where the segment table makes that the faster plan; MOE_A2A_OPT_GEMM_STAGED = 3
- * forces 256 rows, 4 288 rows wherever they save a tile); 32 x 64 tiles that stream the
- * weights when segments are short (R <= 32 * E, R <= 16 * E if Kd % 128 != 0); 128 x 128 output tiles for
- * what is left.  The option MOE_A2A_OPT_GEMM_TILE = 32, 128 or 256 forces one.
+ * forces 256 rows, 4 288 rows wherever they save a tile); 128 x 128 output tiles for what is left.  The option MOE_A2A_OPT_GEMM_TILE = 32, 128 or 256 forces one.
  * Padded layout: a segment longer than max_recv (routing raised MOE_A2A_STATUS_OVERFLOW) is
  * multiplied over its first max_recv rows only, so no tile leaves the segment or the buffers.
  */
@@ -305,7 +305,8 @@ int moe_a2a_expert_gemm_fp8(const void* x_q, const float* x_scale, const void* w
  * x is 16-bit (x_scale == NULL) or the e4m3fn rows + x_scale[rows, Kd/128] of moe_a2a_dispatch_fp8
  * (dequantised and rounded once to elem_type inside the kernel); y[rows, N] of elem_type.
  * Kd % 128 == 0, N % 128 == 0.  Three kernels, chosen by the mean segment length and the rows:
- *   R <= 32 * E (a decode step, bound by the weight bytes, which cross memory once at one byte per
+ *   R <= 32 * E, 22 * E for fp8 rows where there are more than 128 tiles of 256 x 256 and
+ *     Kd >= 512 (a decode step, bound by the weight bytes, which cross memory once at one byte per
  *     element): 32 x 128 tiles, the operand slabs travel memory -> LDS directly (the weights with
  *     non-temporal loads: they are read once).  16-bit rows: the weight bytes enter the matrix
  *     cores exactly (turned into 16-bit values in registers), each 128-wide K block is summed in
@@ -314,8 +315,8 @@ int moe_a2a_expert_gemm_fp8(const void* x_q, const float* x_scale, const void* w
  *     The option MOE_A2A_OPT_GEMM_STAGED = 1 selects the register-staged form of the same
  *     arithmetic (fp8 rows are then dequantised and rounded once to elem_type first).
  *   longer segments, fp8 rows: both operands enter the fp8 matrix instruction as bytes (eight
- *     waves with the 16x16x128 instruction for Kd >= 256, on 256 x 256 tiles or, where those are few, for
- *     N = 128 and for Kd < 512, on 256 x 128 ones, with the same result; the option
+ *     waves with the 16x16x128 instruction for Kd >= 256, on 256 x 256 tiles or, where those are few
+ *     and for N = 128, on 256 x 128 ones, with the same result; the option
  *     MOE_A2A_OPT_GEMM_STAGED = 2, and Kd = 128, take four waves on 128 x 128 tiles with the
  *     32x32x64 one), each 128-wide K block is summed in f32 and folded with
  *     x_scale[row][kb] * w_scale[n / 128][kb]; nothing is rounded before the output.
