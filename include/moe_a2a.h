@@ -276,7 +276,10 @@ int moe_a2a_forward_launches(int T, int K, int H, int max_recv, int in_type, int
  * this is the grouped matrix product a real MoE layer runs there.
  *   x[rows, Kd], weights[E, N, Kd], y[rows, N]: 16-bit elements of elem_type, f32 accumulation,
  *   Kd % 64 == 0, N % 8 == 0, 16-byte aligned.
- * Three kernels with identical results: 32 x 64 tiles that stream the weights when segments are
+ * Four kernels with identical results: tiles of up to 176 rows by 512 columns from some tens of
+ * rows per expert to 144, and for some 300, where these are at least a round of the CUs
+ * (MOE_A2A_OPT_GEMM_TILE = 512 forces them, wherever they apply, in this and the next entry
+ * points); 32 x 64 tiles that stream the weights when segments are
  * short (R <= 32 * E, 25 * E with more than 1 GiB of weights, 16 * E if Kd % 128 != 0); 256 x 256
  * tiles for longer ones (N >= 256, and R > 32 * E or more than 1 GiB of weights; they hold up to
  * 288 rows where the segment table makes that the faster plan; MOE_A2A_OPT_GEMM_STAGED = 3
@@ -304,7 +307,8 @@ int moe_a2a_expert_gemm_fp8(const void* x_q, const float* x_scale, const void* w
  * w_q[E, N, Kd] e4m3fn bytes with w_scale[E, N/128, Kd/128] f32 (one scale per 128 x 128 block).
  * x is 16-bit (x_scale == NULL) or the e4m3fn rows + x_scale[rows, Kd/128] of moe_a2a_dispatch_fp8
  * (dequantised and rounded once to elem_type inside the kernel); y[rows, N] of elem_type.
- * Kd % 128 == 0, N % 128 == 0.  Three kernels, chosen by the mean segment length and the rows:
+ * Kd % 128 == 0, N % 128 == 0.  Three kernels, chosen by the mean segment length and the rows (and,
+ * for fp8 rows, Kd >= 1024, the tiles of 512 columns of moe_a2a_expert_gemm, with the arithmetic of the longer segments):
  *   R <= 32 * E, 22 * E for fp8 rows where there are more than 128 tiles of 256 x 256 and
  *     Kd >= 512 (a decode step, bound by the weight bytes, which cross memory once at one byte per
  *     element): 32 x 128 tiles, the operand slabs travel memory -> LDS directly (the weights with
@@ -387,7 +391,7 @@ const char* moe_a2a_kernel_name(int kernel_id);
  * hipGraph captured under it, belongs to that setting.
  */
 #define MOE_A2A_OPT_ROUTE_TILE 0    /* 1: moe_a2a_route_dispatch takes the token-tile kernel at any size   */
-#define MOE_A2A_OPT_GEMM_TILE 1     /* 32 | 128 | 256: tile family of the expert GEMM entry points          */
+#define MOE_A2A_OPT_GEMM_TILE 1     /* 32 | 128 | 256 | 512: tile family of the expert GEMM entry points    */
 #define MOE_A2A_OPT_GEMM_STAGED 2   /* 1: register-staged form of the weight-streaming / scaled-MFMA loops;
                                        2: four-wave forms of moe_a2a_expert_gemm_mx8 / _q8 with fp8 rows;
                                        3 | 4: the eight-wave loops on 256 x 256 tiles, tiles of 256 rows
