@@ -307,8 +307,8 @@ int moe_a2a_expert_gemm_fp8(const void* x_q, const float* x_scale, const void* w
  * w_q[E, N, Kd] e4m3fn bytes with w_scale[E, N/128, Kd/128] f32 (one scale per 128 x 128 block).
  * x is 16-bit (x_scale == NULL) or the e4m3fn rows + x_scale[rows, Kd/128] of moe_a2a_dispatch_fp8
  * (dequantised and rounded once to elem_type inside the kernel); y[rows, N] of elem_type.
- * Kd % 128 == 0, N % 128 == 0.  Three kernels, chosen by the mean segment length and the rows (and,
- * for fp8 rows, Kd >= 1024, the tiles of 512 columns of moe_a2a_expert_gemm, with the arithmetic of the longer segments):
+ * Kd % 128 == 0, N % 128 == 0.  Kernels chosen by the mean segment length and the rows (for fp8
+ * rows and Kd >= 1024 the tiles of 512 columns of moe_a2a_expert_gemm too, with the arithmetic of the longer segments):
  *   R <= 32 * E, 22 * E for fp8 rows where there are more than 128 tiles of 256 x 256 and
  *     Kd >= 512 (a decode step, bound by the weight bytes, which cross memory once at one byte per
  *     element): 32 x 128 tiles, the operand slabs travel memory -> LDS directly (the weights with
@@ -324,6 +324,9 @@ int moe_a2a_expert_gemm_fp8(const void* x_q, const float* x_scale, const void* w
  *     MOE_A2A_OPT_GEMM_STAGED = 2, and Kd = 128, take four waves on 128 x 128 tiles with the
  *     32x32x64 one), each 128-wide K block is summed in f32 and folded with
  *     x_scale[row][kb] * w_scale[n / 128][kb]; nothing is rounded before the output.
+ *   16-bit rows, more than 24 rows per expert where there are at least 512 tiles of 512 columns, or 32
+ *     where there are at least 256: tiles of up to 160 rows by 512 columns, with the arithmetic of the
+ *     decode step (nothing is rounded before the output);
  *   longer segments, 16-bit rows (and N >= 256): the 256 x 256 kernel; a weight enters the matrix
  *     cores as elem(f32(q) * scale), i.e. dequantised and rounded once to elem_type on its way into
  *     LDS -- the result of dequantising the weights to 16 bits and calling moe_a2a_expert_gemm,

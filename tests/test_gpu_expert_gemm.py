@@ -881,12 +881,13 @@ STRIP_COUNTS = [1, 16, 17, 64, 65, 96, 97, 112, 113, 0, 128, 129, 144, 145, 160,
 
 @pytest.mark.parametrize("counts", [STRIP_COUNTS, [1], [0, 0, 5]], ids=["segments", "one-row", "first-empty"])
 @pytest.mark.parametrize("form,slabs,N", [("16bit", 1, 8), ("16bit", 2, 520), ("16bit", 5, 1032), ("fp8", 8, 128), ("fp8", 11, 640),
-                                          ("fp8", 16, 1152), ("pow2", 9, 512), ("pow2", 15, 640)])
+                                          ("fp8", 16, 1152), ("pow2", 9, 512), ("pow2", 15, 640), ("w8", 1, 128), ("w8", 2, 640),
+                                          ("w8", 9, 1152)])
 @pytest.mark.parametrize("padded", [False, True], ids=["compact", "padded"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 def test_strips(gpu_device, options, dtype, padded, form, slabs, N, counts):
     """Tiles of 512 columns: every form of a tile, a last one of any width, one slab to several groups of scales with a rest, the
-    padded layout with a segment longer than its room.  The bits of the 256 x 256 tiles, and the f32 product."""
+    padded layout with a segment longer than its room.  The bits of the 256 x 256 tiles, where there are such, and the f32 product."""
     H = slabs * (64 if form == "16bit" else 128)
     cfg, world, weights = make_counts(counts, H, N, dtype, seed=H + N + len(counts))
     x, idx, w, rs = concat_world(world, gpu_device)
@@ -904,10 +905,10 @@ def test_strips(gpu_device, options, dtype, padded, form, slabs, N, counts):
         wq, ws = V.quantize_weights_fp8(weights, pow2=form == "pow2")
         wd = wq.to(gpu_device)
         kw = dict(w_scale=ws.to(gpu_device), scales_pow2=form == "pow2")
-        x32 = d.disp_x.view(torch.float8_e4m3fn).float() * d.disp_scale.repeat_interleave(128, 1)
+        x32 = d.disp_x.float() if form == "w8" else d.disp_x.view(torch.float8_e4m3fn).float() * d.disp_scale.repeat_interleave(128, 1)
         w32 = wd.view(torch.float8_e4m3fn).float() * kw["w_scale"].repeat_interleave(128, 1).repeat_interleave(128, 2)
     got = {}
-    for tile, staged in ((512, 0), (256 if form != "fp8" else 128, 3)):
+    for tile, staged in ((512, 0), (128 if form == "fp8" else 32 if form == "w8" else 256, 3)):
         options.set("GEMM_TILE", tile)
         options.set("GEMM_STAGED", staged)
         got[tile] = ata.expert_gemm(d, wd, **kw)[rows].clone()
@@ -915,8 +916,9 @@ def test_strips(gpu_device, options, dtype, padded, form, slabs, N, counts):
     want = torch.cat([x32[(first := e * room if padded else int(off[e])):first + n] @ w32[e].T for e, n in enumerate(lens)])
     close(got[512], want.cpu())
     first, second = got.values()
-    # (power-of-two scales of up to 32 rows on average take the kernels for any scale, in another order of the sums' parts)
-    if form != "pow2" or sum(counts) > 32 * len(counts):
+    # (fp8 weights: the streaming kernel walks K in another order; power-of-two scales of up to 32 rows on average take the kernels
+    # for any scale)
+    if form not in ("pow2", "w8") or (form == "pow2" and sum(counts) > 32 * len(counts)):
         assert torch.equal(first.view(torch.int16), second.view(torch.int16))
 
 
@@ -926,6 +928,8 @@ def test_strips(gpu_device, options, dtype, padded, form, slabs, N, counts):
     ("fp8", 256, 896, 1536, {100: "expert_gemm_f8"}),  # less than eight slabs
     ("pow2", 256, 1024, 512, {95: "expert_gemm_mx", 96: "strip", 128: "strip", 129: "expert_gemm_mx", 290: "strip"}),
     ("fp8", 255, 1024, 512, {100: "expert_gemm_f8"}),  # less than one round
+    ("w8", 256, 256, 1024, {24: "expert_gemm_skinny", 25: "strip", 700: "strip"}),
+    ("w8", 256, 256, 512, {32: "expert_gemm_skinny", 33: "strip"}),
 ])
 def test_where_strips_are_taken(gpu_device, options, form, E, Kd, N, kernels):
     """Lengths on both sides of every border: strips go by the name of their format's 256 x 256 tiles.  Products of ones."""
@@ -933,12 +937,11 @@ def test_where_strips_are_taken(gpu_device, options, form, E, Kd, N, kernels):
     for rows, name in kernels.items():
         R = rows * E
         one = 0x38  # 1.0 in e4m3fn
-        if form == "16bit":
-            x, w = torch.ones(R, Kd, dtype=torch.bfloat16, device=gpu_device), torch.ones(E, N, Kd, dtype=torch.bfloat16, device=gpu_device)
-        else:
-            x = torch.full((R, Kd), one, dtype=torch.uint8, device=gpu_device)
-            w = torch.full((E, N, Kd), one, dtype=torch.uint8, device=gpu_device)
-            xs, ws = torch.ones(R, Kd // 128, device=gpu_device), torch.ones(E, N // 128, Kd // 128, device=gpu_device)
+        ones = lambda *shape: torch.ones(shape, dtype=torch.bfloat16, device=gpu_device)
+        bytes_ = lambda *shape: torch.full(shape, one, dtype=torch.uint8, device=gpu_device)
+        x = (ones if form in ("16bit", "w8") else bytes_)(R, Kd)
+        w = (ones if form == "16bit" else bytes_)(E, N, Kd)
+        xs, ws = torch.ones(R, Kd // 128, device=gpu_device), torch.ones(E, N // 128, Kd // 128, device=gpu_device)
         y = torch.zeros(R, N, dtype=torch.bfloat16, device=gpu_device)
         off = torch.arange(0, R + 1, rows, dtype=torch.int32, device=gpu_device)
         tail = (off.data_ptr(), y.data_ptr(), R, E, Kd, N, 0, _lib.BF16, torch.cuda.current_stream().cuda_stream)
@@ -946,8 +949,8 @@ def test_where_strips_are_taken(gpu_device, options, form, E, Kd, N, kernels):
             call = lambda: lib.moe_a2a_expert_gemm(x.data_ptr(), w.data_ptr(), *tail)
         else:
             f = lib.moe_a2a_expert_gemm_mx8 if form == "pow2" else lib.moe_a2a_expert_gemm_q8
-            call = lambda: f(x.data_ptr(), xs.data_ptr(), w.data_ptr(), ws.data_ptr(), *tail)
+            call = lambda: f(x.data_ptr(), None if form == "w8" else xs.data_ptr(), w.data_ptr(), ws.data_ptr(), *tail)
         got = launched(lib, call)
-        family = {"16bit": "expert_gemm_wide", "fp8": "expert_gemm_f8", "pow2": "expert_gemm_mx"}[form]
+        family = {"16bit": "expert_gemm_wide", "fp8": "expert_gemm_f8", "pow2": "expert_gemm_mx", "w8": "expert_gemm_wide"}[form]
         assert got == [family if name == "strip" else name], rows
         assert bool((y == Kd).all()), rows
