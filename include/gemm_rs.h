@@ -37,7 +37,10 @@ extern "C" {
  *             - outputs of few tiles spread the shards over groups of workgroups, one f32 partial
  *               product per group (what each rank holds before the reduce-scatter), which a second
  *               launch sums: REQUIRED, MOE_A2A_E_WORKSPACE if missing or too small;
- *             - the same where it pays although the tiles fill most of the chip (160 or more of 256 x 128):
+ *             - some hundreds of rows and a long K, most of all a local K that is not a multiple of 64: groups on 256 x 256
+ *               tiles.  OPTIONAL in so far as with NULL, too few bytes or a pointer off its alignment the call goes on
+ *               as if this form did not exist (and may then be one of the first kind);
+ *             - groups where they pay although the tiles fill most of the chip (160 or more of 256 x 128):
  *               OPTIONAL -- with NULL or too few bytes all shards are summed by one workgroup per tile, up
  *               to a fifth slower;
  *             - large outputs whose local K is not a multiple of 32 (rows that start off the
@@ -49,7 +52,8 @@ extern "C" {
  *           size queried under one setting belongs to that setting.
  * MOE_A2A_OPT_GEMM_TILE forces a form where the shape allows it: 256 the 256 x 256 tiles, 129 the
  * 256 x 128 tiles (131 / 132: with 192 / 128 of a tile's rows in use, as the library chooses by itself
- * when that fills the CUs better), 130 those with one partial product per shard, 128 the 128 x 128
+ * when that fills the CUs better), 130 those with one partial product per shard, 133 the 256 x 256 tiles with
+ * one partial product per shard, 128 the 128 x 128
  * tiles, 32 those with one partial product per shard.  All unsplit forms give identical bits.
  */
 size_t gemm_rs_workspace_bytes(int M, int N, int K, int W);

@@ -464,3 +464,76 @@ def test_replays_of_a_captured_graph_follow_their_inputs(gpu_device, shape):
         assert torch.equal(got.view(torch.int16), eager.view(torch.int16))
         ok, worst = within_one_rounding(got.cpu(), O.exact_world([(x[s].cpu(), w[s].cpu(), b.cpu()) for s in range(W)]))
         assert ok, worst
+
+
+def product(x, w, bias=None):
+    """The f32 product of concatenated shards."""
+    W, m, kl = x.shape
+    y = x.transpose(0, 1).reshape(m, W * kl).float() @ w.transpose(0, 1).reshape(w.shape[1], W * kl).float().T
+    return y if bias is None else y + W * bias.float()
+
+
+def uniform(shape, dtype, dev, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    return torch.empty(*shape, dtype=dtype, device=dev).uniform_(-0.05, 0.05, generator=g)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,m,n,kl", [
+    (2, 65, 8, 64), (2, 256, 256, 72), (8, 257, 260, 64), (4, 392, 600, 360), (8, 72, 4100, 96), (3, 520, 2052, 200),
+    (4, 1040, 1000, 128),  # more than a round of tiles
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_wide_tiles_with_the_shards_in_groups(gpu_device, options, dtype, W, m, n, kl):
+    """Every row and column at the edges of tiles, slabs and groups, with a bias and an infinite element on either side.  f32
+    sums of W kl products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 product and 1e-5."""
+    options.set("GEMM_TILE", 133)
+    x, w, bias = (uniform(s, dtype, gpu_device, m + n + i) for i, s in enumerate(((W, m, kl), (W, n, kl), (n,))))
+    x[W - 1, m - 1, kl - 1] = float("inf")
+    w[0, n - 1, kl - 8] = float("-inf")
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
+    kernels = launched(_lib.load(), lambda: G.HipGemmReduceScatter(W).forward(x, w, bias, out=out))
+    assert kernels == ["gemm_rs_narrow", "gemm_rs_reduce"]
+    want = product(x, w, bias)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
+    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,m,n,k,groups", [(8, 512, 5440, 17024, 4), (8, 240, 4480, 24128, 8), (8, 1096, 6400, 6464, 2),
+                                            (4, 304, 5696, 11328, 4), (8, 120, 4160, 11008, 8)])
+def test_room_for_the_groups_is_optional(gpu_device, W, m, n, k, groups):
+    """Shapes that take 256 x 256 tiles in groups: room for their partial products is what is asked for, and with less of it, or off its
+    alignment, the call is answered as it is without that form: on the 256 x 128 tiles, with what they need, or MOE_A2A_E_WORKSPACE.
+    Shards that lie apart as well.  Tolerance as above, 2e-5."""
+    lib = _lib.load()
+    pad = 64
+    x, w = uniform((W, m * (k // W) + pad), torch.bfloat16, gpu_device, 5), uniform((W, n * (k // W) + pad), torch.bfloat16, gpu_device, 6)
+    want = product(x[:, :-pad].reshape(W, m, -1), w[:, :-pad].reshape(W, n, -1))
+    need = lib.gemm_rs_workspace_bytes(m, n, k, W)
+    assert need == groups * m * n * 4
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=gpu_device)
+    answers = []
+    for at, size in ((ws.data_ptr(), need), (ws.data_ptr(), need - 1), (ws.data_ptr() + 8, need), (None, 0)):
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+        rc = lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, k, W, m * (k // W) + pad, n * (k // W) + pad,
+                                 _lib.BF16, at, size, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        answers.append(rc)
+        if rc == 0:
+            assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
+        else:
+            assert rc in (E_WORKSPACE, E_ALIGN) and bool(out.isnan().all())
+    assert answers[0] == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n", [(2304, 6656), (2200, 6500), (6736, 2240), (3576, 4416), (7288, 4160)])
+def test_wide_tiles_dealt_out_in_column_order(gpu_device, m, n):
+    """Numbers of 256 x 256 tiles that bands or blocks would make more rounds of: none left out or done twice."""
+    x, w = uniform((8, m, 72), torch.bfloat16, gpu_device, m), uniform((8, n, 72), torch.bfloat16, gpu_device, n)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    assert launched(_lib.load(), lambda: G.HipGemmReduceScatter(8).forward(x, w, out=out)) == ["gemm_rs_wide"]
+    want = product(x, w)
+    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6).all())
