@@ -69,7 +69,7 @@ extern "C" {
 #define MOE_A2A_E_DTYPE (-3)     /* unknown element type, stub kind or combine mode   */
 #define MOE_A2A_E_WORKSPACE (-4) /* workspace missing or smaller than workspace_bytes */
 #define MOE_A2A_E_ALIGN (-5)     /* a row buffer is not 16-byte aligned               */
-#define MOE_A2A_E_STATE (-6)     /* launch timer used out of order                    */
+#define MOE_A2A_E_STATE (-6)     /* launch timer used out of order; not one launch     */
 #define MOE_A2A_E_CAPACITY (-7)  /* table beyond the static scratch of moe_a2a_route_noalloc */
 
 typedef void* moe_a2a_stream_t; /* hipStream_t */
@@ -264,6 +264,14 @@ typedef struct moe_a2a_forward_args {
   int32_t* clear_status;
 } moe_a2a_forward_args;
 int moe_a2a_forward_packed(const moe_a2a_forward_args* args);
+
+/*
+ * Routing and dispatch alone (all2all/reference.py:68-148), in one launch: the index arrays, counts and dispatched rows of
+ * `args`, compact (max_recv 0), in 16 bits or fp8; weights, expert_y, out, workspace and clear_status are not looked at.  Status is
+ * written, not OR-ed into: it describes this call, with no launch spent on clearing it.  MOE_A2A_E_STATE, with nothing launched,
+ * where this shape or these switches take more than one launch (moe_a2a_route and moe_a2a_dispatch or _fp8 do).
+ */
+int moe_a2a_dispatch_once(const moe_a2a_forward_args* args);
 
 /* Kernel launches moe_a2a_forward issues for this shape and these switches (host logic only). */
 int moe_a2a_forward_launches(int T, int K, int H, int max_recv, int in_type, int out_type, int fp8_dispatch,

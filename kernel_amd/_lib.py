@@ -10,6 +10,7 @@ import os
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmoe_a2a.so")
 
 ABI_VERSION = 5
+E_STATE = -6  # MOE_A2A_E_STATE
 F16, BF16 = 0, 1
 FP8_SCALE_F32, FP8_SCALE_POW2 = 0, 1
 STATUS_BAD_EXPERT, STATUS_OVERFLOW = 1, 2  # bits of the routing status word
@@ -70,6 +71,7 @@ class ForwardArgs(C.Structure):
 
 
 PROTOTYPES["moe_a2a_forward_packed"] = (_int, [C.POINTER(ForwardArgs)])
+PROTOTYPES["moe_a2a_dispatch_once"] = (_int, [C.POINTER(ForwardArgs)])
 
 # include/gemm_rs.h (same library)
 GEMM_RS_PROTOTYPES = {

@@ -251,6 +251,9 @@ class HipAllToAll:
             if rank_start.dtype != torch.int32 or rank_start.numel() != W + 1:
                 raise ValueError("rank_start must be int32[world_size + 1]")
         b = self._buffers(T, dp_x.device, advance=True)
+        if self.fuse_route and not self.padded and self._dispatch_once(b, dp_x, indices, rank_start):
+            return Dispatched(cfg, W, T, b["counts"], b["offsets"], b["slot_of_entry"], b["src_of_slot"], b["meta"],
+                              b["disp_x"], b["disp_scale"], b["status"], 0)
         b["status"].zero_()  # the phase-by-phase entry points only ever set bits: the record describes this call
         lib, st = self.lib, _stream()
         pad = self.max_recv if self.padded else 0
@@ -275,6 +278,26 @@ class HipAllToAll:
                            "moe_a2a_dispatch")
         return Dispatched(cfg, W, T, b["counts"], b["offsets"], b["slot_of_entry"], b["src_of_slot"], b["meta"],
                           b["disp_x"], b["disp_scale"], b["status"], pad)
+
+    def _dispatch_once(self, b: dict, dp_x, indices, rank_start) -> bool:
+        """One launch for routing and rows, which writes the status word as well; False: not for this shape."""
+        block = b.get("dispatch_block")
+        if block is None:  # (its pointers are the set's own)
+            cfg = self.cfg
+            own = {name: _ptr(b[name]) for name in ("counts", "offsets", "slot_of_entry", "src_of_slot", "meta", "status",
+                                                    "disp_scale")}
+            block = b["dispatch_block"] = bytes(_lib.ForwardArgs(
+                T=b["out"].shape[0], K=cfg.experts_per_token, E=cfg.num_experts, W=self.world_size, H=cfg.hidden_dim,
+                in_type=_elem(cfg.in_dtype), out_type=_elem(cfg.out_dtype), disp=_ptr(b["disp_x"]),
+                fp8_dispatch=2 if self.fp8_dispatch == "pow2" else int(self.fp8_dispatch), **own))
+        a = _lib.ForwardArgs.from_buffer_copy(block)  # (a copy: other threads make theirs)
+        a.x, a.indices, a.rank_start, a.stream = _ptr(dp_x), _ptr(indices), _ptr(rank_start), _stream()
+        a.src_rank = self.rank
+        a.fuse_route = 2 if self.fuse_route == "always" else 1
+        rc = self.lib.moe_a2a_dispatch_once(ctypes.byref(a))
+        if rc != _lib.E_STATE:
+            _lib.check(rc, "moe_a2a_dispatch_once")
+        return rc == 0
 
     # ---- expert stub -----------------------------------------------------------------
     def expert_stub(self, d: Dispatched) -> torch.Tensor:

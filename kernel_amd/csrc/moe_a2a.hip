@@ -529,14 +529,14 @@ int moe_a2a_fused_ok(int T, int K, int H) {
 static int route_dispatch_impl(const void* x, const int32_t* indices, const int32_t* rank_start, int src_rank, int T,
                                int K, int E, int W, int H, int max_recv, int32_t* counts, int32_t* offsets,
                                int32_t* slot_of_entry, int32_t* src_of_slot, int32_t* meta, int32_t* status,
-                               void* disp_x, moe_a2a_stream_t stream_, int32_t* clear_status) {
+                               void* disp_x, moe_a2a_stream_t stream_, int32_t* clear_status, int own_status = 0) {
   if (int rc = check_route_shape(T, K, E, W)) return rc;
   if (max_recv < 0 || (long long)max_recv * E > (long long)INT32_MAX / 8) return MOE_A2A_E_SHAPE;
   if (int rc = check_rows(x, disp_x, T, K, H, 8)) return rc;
   if (!counts || !offsets) return MOE_A2A_E_NULL;
   if (T > 0 && (!indices || !slot_of_entry || !src_of_slot || !meta)) return MOE_A2A_E_NULL;
   RouteArgs a{indices, rank_start, src_rank, T, K, E, W, T * K, id_bits(E), max_recv, counts, offsets,
-              slot_of_entry, src_of_slot, meta, status, clear_status};
+              slot_of_entry, src_of_slot, meta, status, clear_status, own_status};
   const int nvec = H / 8;
   if (!fused_small_ok(T, K, H) || option(MOE_A2A_OPT_ROUTE_TILE) == 1) {  // token tiles: any table size
     if (T == 0) return route_impl(indices, rank_start, src_rank, T, K, E, W, max_recv, counts, offsets, slot_of_entry,
@@ -626,18 +626,23 @@ static int fp8_tile_tokens(int T, int K) {
   const int spread = ceil_div(T, 256);
   return std::min(cap, spread < wave ? spread : std::max(wave, ceil_div(T, 2 * 256)));
 }
+// Longest table of a dispatch on its own that takes it (moe_a2a_dispatch_once): every workgroup's pass over the table grows with it.
+// us, cleared status, routing and rows as three launches / one: top-8 of 256, 7168 columns, 64 tokens 13.5 / 6.3, 500 14.6 / 9.3, 1000
+// 19.7 / 15.9, 4000 70.5 / 72.1; top-6 of 64, 2048 columns, 2000 15.1 / 9.7, 16000 65 / 79; top-4 of 128, 4096 columns, 2000 16.8 / 13.2,
+// 4000 26.1 / 26.8.
+constexpr long long kDispatchOnceFp8Rows = 12288;
 static int fp8_tile_threads(int E) { return E <= 512 ? 512 : kTileThreads; }
 static int route_dispatch_fp8_impl(const void* x, int x_type, const int32_t* indices, const int32_t* rank_start,
                                    int src_rank, int T, int K, int E, int W, int H, int max_recv, int32_t* counts,
                                    int32_t* offsets, int32_t* slot_of_entry, int32_t* src_of_slot, int32_t* meta,
                                    int32_t* status, void* disp_q, float* disp_scale, int pow2, hipStream_t stream,
-                                   int32_t* clear_status) {
+                                   int32_t* clear_status, int own_status = 0) {
   if (int rc = check_route_shape(T, K, E, W)) return rc;
   if (max_recv < 0 || (long long)max_recv * E > (long long)INT32_MAX / 8) return MOE_A2A_E_SHAPE;
   if (int rc = check_rows(x, disp_q, T, K, H, MOE_A2A_FP8_BLOCK)) return rc;
   if (!counts || !offsets || !indices || !slot_of_entry || !src_of_slot || !meta || !disp_scale) return MOE_A2A_E_NULL;
   RouteArgs a{indices, rank_start, src_rank, T, K, E, W, T * K, id_bits(E), max_recv, counts, offsets,
-              slot_of_entry, src_of_slot, meta, status, clear_status};
+              slot_of_entry, src_of_slot, meta, status, clear_status, own_status};
   const int nblk = H / MOE_A2A_FP8_BLOCK;
   const int tile = fp8_tile_tokens(T, K);
   // workgroups of 512 lanes, three to a CU, so that one's table pass runs under another's rows (a thread
@@ -661,6 +666,24 @@ static int route_dispatch_fp8_impl(const void* x, int x_type, const int32_t* ind
   RDF8(F16, 0);
 #undef RDF8_T
 #undef RDF8
+}
+
+// (16-bit rows, cleared status and one launch / one launch: 64 tokens, top-6 of 64, 2048 columns 11.2 / 6.8 us, 2000 13.6 / 12.2)
+int moe_a2a_dispatch_once(const moe_a2a_forward_args* a) {
+  if (!a) return MOE_A2A_E_NULL;
+  const int T = a->T, K = a->K, H = a->H;
+  const long long R = (long long)T * K;
+  if (T < 1 || K < 1 || a->max_recv != 0 || !a->fuse_route) return MOE_A2A_E_STATE;
+  if (a->fp8_dispatch) {
+    if (!route_dispatch_fp8_ok(T, K, H) || R > kDispatchOnceFp8Rows) return MOE_A2A_E_STATE;
+    if (a->in_type != MOE_A2A_F16 && a->in_type != MOE_A2A_BF16) return MOE_A2A_E_DTYPE;
+    return route_dispatch_fp8_impl(a->x, a->in_type, a->indices, a->rank_start, a->src_rank, T, K, a->E, a->W, H, 0, a->counts,
+                                   a->offsets, a->slot_of_entry, a->src_of_slot, a->meta, a->status, a->disp, a->disp_scale,
+                                   a->fp8_dispatch == 2, (hipStream_t)a->stream, nullptr, 1);
+  }
+  if (!(a->fuse_route == 2 && R <= moe_a2a_fused_max_rows()) && !moe_a2a_fused_ok(T, K, H)) return MOE_A2A_E_STATE;
+  return route_dispatch_impl(a->x, a->indices, a->rank_start, a->src_rank, T, K, a->E, a->W, H, 0, a->counts, a->offsets,
+                             a->slot_of_entry, a->src_of_slot, a->meta, a->status, a->disp, a->stream, nullptr, 1);
 }
 
 static bool known_type(int t) { return t == MOE_A2A_F16 || t == MOE_A2A_BF16; }

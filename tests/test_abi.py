@@ -248,3 +248,21 @@ def test_headers_are_plain_c_and_link_from_c(tmp_path):
     subprocess.run(["gcc", "-std=c99", "-I", inc, str(src), "-o", str(exe), "-L", lib_dir, "-lmoe_a2a",
                     "-Wl,-rpath," + lib_dir], check=True)
     assert subprocess.run([str(exe)]).returncode == _lib.ABI_VERSION
+
+
+def test_dispatch_once_argument_checks(lib):
+    def once(**changes):
+        fields = dict(x=A, indices=A, src_rank=0, T=64, K=4, E=64, W=8, H=2048, max_recv=0, in_type=_lib.BF16, out_type=_lib.BF16,
+                      fp8_dispatch=0, fuse_route=1, counts=A, offsets=A, slot_of_entry=A, src_of_slot=A, meta=A, disp=A, disp_scale=A)
+        return lib.moe_a2a_dispatch_once(ctypes.byref(_lib.ForwardArgs(**{**fields, **changes})))
+
+    assert lib.moe_a2a_dispatch_once(None) == E_NULL
+    for fp8 in (0, 1, 2):
+        assert once(fp8_dispatch=fp8, T=0) == once(fp8_dispatch=fp8, fuse_route=0) == once(fp8_dispatch=fp8, max_recv=9) == E_STATE
+        assert once(fp8_dispatch=fp8, E=63) == E_SHAPE
+        assert once(fp8_dispatch=fp8, meta=None) == once(fp8_dispatch=fp8, x=None) == E_NULL
+        assert once(fp8_dispatch=fp8, disp=A + 8) == E_ALIGN
+    assert once(fp8_dispatch=1, T=3073) == E_STATE  # a longer table than one launch takes
+    assert once(fp8_dispatch=1, H=2056) == E_STATE and once(fp8_dispatch=1, in_type=9) == E_DTYPE
+    assert once(fp8_dispatch=1, disp_scale=None) == E_NULL
+    assert once(T=16384, H=4096) == E_STATE  # streaming sizes

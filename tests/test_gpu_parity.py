@@ -768,3 +768,32 @@ def test_buffer_sets_alternate_and_old_token_counts_are_dropped(gpu_device):
     torch.cuda.synchronize()
     assert torch.equal(bits(y.cpu()), bits(want))
     assert len(ata._bufs) == ata.MAX_CACHED_SHAPES
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,K,H,T", [(8, 2, 128, 1), (64, 6, 2048, 65), (64, 6, 256, 2048), (64, 6, 256, 2049), (256, 8, 1024, 300),
+                                     (1024, 8, 128, 33), (100, 3, 384, 700)])
+@pytest.mark.parametrize("fp8", [False, True, "pow2"])
+def test_dispatch_in_one_launch_is_the_separate_launches(gpu_device, E, K, H, T, fp8):
+    """The same buffers, byte for byte, either side of the longest fp8 table that takes one launch (12288 entries), and a status word
+    that describes its own call: set by an id outside [0, E) anywhere in the table, clear again two calls later, on the same set of
+    buffers, and not set by what the caller leaves in it."""
+    cfg = C.MoEConfig(E, K, H, T + 1, in_dtype=torch.bfloat16, out_dtype=torch.bfloat16)
+    g = torch.Generator(device=gpu_device).manual_seed(T)
+    x = torch.randn(T, H, device=gpu_device, generator=g).to(torch.bfloat16)
+    ids = torch.randint(0, E, (T, K), device=gpu_device, generator=g, dtype=torch.int32)
+    W = 4 if E % 4 == 0 else 1
+    starts = torch.tensor([0] + [T * (r + 1) // W for r in range(W)], dtype=torch.int32, device=gpu_device)
+    one, apart = (HipAllToAll(cfg, 0, W, fp8_dispatch=fp8, fuse_route=f) for f in (True, False))
+    for place, bad in ((None, 0), ((T - 1, K - 1), E), ((0, 0), -1), (None, 0), (None, 0)):
+        table = ids.clone()
+        if place is not None:
+            table[place] = bad
+        for rank_start in (None, starts):
+            a, b = one.dispatch(x, table, rank_start), apart.dispatch(x, table, rank_start)
+            for name in ("counts", "offsets", "slot_of_entry", "src_of_slot", "meta", "status"):
+                assert torch.equal(getattr(a, name), getattr(b, name)), (name, place)
+            assert int(a.status.item()) == (_lib.STATUS_BAD_EXPERT if place is not None else 0)
+            assert torch.equal(a.disp_x.view(torch.uint8), b.disp_x.view(torch.uint8))
+            assert a.disp_scale is None or torch.equal(a.disp_scale, b.disp_scale)
+            a.status.fill_(2)
