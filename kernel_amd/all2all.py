@@ -78,8 +78,8 @@ class Dispatched:
     disp_scale: Optional[torch.Tensor] = None  # [R,H/128] f32 (fp8 only)
     # [1] int32, bits: 1 an expert id was out of range, 2 a padded segment overflowed.  It describes
     # the call that produced this record and stays readable until the next call on the same
-    # ``HipAllToAll`` is enqueued (that call clears the word for the call after it: the host class
-    # alternates between two buffer sets, and each call clears the other set's word)
+    # ``HipAllToAll`` is enqueued (the host class alternates between two buffer sets; a forward clears the
+    # other set's word for the call after it, a dispatch writes or clears its own)
     status: Optional[torch.Tensor] = None
     max_recv: int = 0  # > 0: padded layout, expert e owns rows [e*max_recv, (e+1)*max_recv)
 
