@@ -267,9 +267,10 @@ int moe_a2a_forward_packed(const moe_a2a_forward_args* args);
 
 /*
  * Routing and dispatch alone (all2all/reference.py:68-148), in one launch: the index arrays, counts and dispatched rows of
- * `args`, compact (max_recv 0), in 16 bits or fp8; weights, expert_y, out, workspace and clear_status are not looked at.  Status is
- * written, not OR-ed into: it describes this call, with no launch spent on clearing it.  MOE_A2A_E_STATE, with nothing launched,
- * where this shape or these switches take more than one launch (moe_a2a_route and moe_a2a_dispatch or _fp8 do).
+ * `args`, compact (max_recv 0), in 16 bits or fp8; weights, expert_y, out and workspace are not looked at.  Status is
+ * written, not OR-ed into: it describes this call, with no launch spent on clearing it.  clear_status as in a forward: where forwards
+ * run on the same pair of buffer sets, the word that the next of them ORs into.  MOE_A2A_E_STATE, with nothing launched, where
+ * this shape or these switches take more than one launch (moe_a2a_route and moe_a2a_dispatch or _fp8 do).
  */
 int moe_a2a_dispatch_once(const moe_a2a_forward_args* args);
 

@@ -77,9 +77,10 @@ class Dispatched:
     disp_x: torch.Tensor  # [R,H] in_dtype, or uint8 e4m3fn bits for fp8 dispatch
     disp_scale: Optional[torch.Tensor] = None  # [R,H/128] f32 (fp8 only)
     # [1] int32, bits: 1 an expert id was out of range, 2 a padded segment overflowed.  It describes
-    # the call that produced this record and stays readable until the next call on the same
-    # ``HipAllToAll`` is enqueued (the host class alternates between two buffer sets; a forward clears the
-    # other set's word for the call after it, a dispatch writes or clears its own)
+    # the call that produced this record.  A forward's stays readable until the next call on the same
+    # ``HipAllToAll`` is enqueued (the host class alternates between two buffer sets; every call clears the
+    # forward's word of the other set, for the call after it), a dispatch's, which is another word, as long as
+    # its buffers
     status: Optional[torch.Tensor] = None
     max_recv: int = 0  # > 0: padded layout, expert e owns rows [e*max_recv, (e+1)*max_recv)
 
@@ -177,8 +178,9 @@ class HipAllToAll:
         # both sets of a new shape are allocated together, so that the second call with this shape
         # does not meet an allocation either
         sets = [self._allocate(T, device), self._allocate(T, device)]
-        for i in (0, 1):  # a call on one set clears the status word of the other (see Dispatched.status)
-            sets[i]["partner_status"] = sets[i ^ 1]["status"]
+        for b, other in zip(sets, reversed(sets)):  # a call on one set clears the status word of the other (see Dispatched.status)
+            b.update(partner_status=other["status"], dispatch_status=other.get("lent_status"),
+                     dispatch_clears=other.get("lent_clears"))
         cfg = self.cfg
         native = _lib.host().Ring(T, cfg.experts_per_token, cfg.hidden_dim, self.world_size, device.index, cfg.in_dtype,
                                   cfg.out_dtype)
@@ -193,13 +195,17 @@ class HipAllToAll:
         R = T * K
         rows = E * self.max_recv if self.padded else R  # rows of the dispatched buffers
         i32 = dict(dtype=torch.int32, device=device)
+        # this set's word of a forward and the other set's of a dispatch, which a dispatch there clears together; a line each
+        words = torch.zeros(2, 32, **i32)
         b = dict(
             counts=torch.empty(E, **i32),
             offsets=torch.empty(E + 1, **i32),
             slot_of_entry=torch.empty(R, **i32),
             src_of_slot=torch.empty(rows, **i32),
             meta=torch.empty(rows, META_DIM, **i32),
-            status=torch.zeros(1, **i32),
+            status=words[0, :1],
+            lent_status=words[1, :1],
+            lent_clears=words[:, :1],
             workspace=torch.empty(max(self.lib.moe_a2a_workspace_bytes(T, K, E), 256), dtype=torch.uint8,
                                   device=device),
             # the stub's output rows exist only where the stub is a launch of its own (expert_stub
@@ -253,12 +259,12 @@ class HipAllToAll:
         b = self._buffers(T, dp_x.device, advance=True)
         if self.fuse_route and not self.padded and self._dispatch_once(b, dp_x, indices, rank_start):
             return Dispatched(cfg, W, T, b["counts"], b["offsets"], b["slot_of_entry"], b["src_of_slot"], b["meta"],
-                              b["disp_x"], b["disp_scale"], b["status"], 0)
-        b["status"].zero_()  # the phase-by-phase entry points only ever set bits: the record describes this call
+                              b["disp_x"], b["disp_scale"], b["dispatch_status"], 0)
+        b["dispatch_clears"].zero_()  # the phase-by-phase entry points only ever set bits: the record describes this call
         lib, st = self.lib, _stream()
         pad = self.max_recv if self.padded else 0
         route_out = (_ptr(b["counts"]), _ptr(b["offsets"]), _ptr(b["slot_of_entry"]), _ptr(b["src_of_slot"]),
-                     _ptr(b["meta"]), _ptr(b["status"]))
+                     _ptr(b["meta"]), _ptr(b["dispatch_status"]))
         if self.fuse_route and not self.fp8_dispatch and (
                 self.fuse_route == "always" and 0 < T * K <= self._fused_max_rows
                 or self.lib.moe_a2a_fused_ok(T, K, H)):
@@ -277,15 +283,15 @@ class HipAllToAll:
                 _lib.check(lib.moe_a2a_dispatch(_ptr(dp_x), _ptr(b["slot_of_entry"]), _ptr(b["disp_x"]), T, K, H, st),
                            "moe_a2a_dispatch")
         return Dispatched(cfg, W, T, b["counts"], b["offsets"], b["slot_of_entry"], b["src_of_slot"], b["meta"],
-                          b["disp_x"], b["disp_scale"], b["status"], pad)
+                          b["disp_x"], b["disp_scale"], b["dispatch_status"], pad)
 
     def _dispatch_once(self, b: dict, dp_x, indices, rank_start) -> bool:
         """One launch for routing and rows, which writes the status word as well; False: not for this shape."""
         block = b.get("dispatch_block")
         if block is None:  # (its pointers are the set's own)
             cfg = self.cfg
-            own = {name: _ptr(b[name]) for name in ("counts", "offsets", "slot_of_entry", "src_of_slot", "meta", "status",
-                                                    "disp_scale")}
+            own = {name: _ptr(b[name]) for name in ("counts", "offsets", "slot_of_entry", "src_of_slot", "meta", "disp_scale")}
+            own.update(status=_ptr(b["dispatch_status"]), clear_status=_ptr(b["partner_status"]))
             block = b["dispatch_block"] = bytes(_lib.ForwardArgs(
                 T=b["out"].shape[0], K=cfg.experts_per_token, E=cfg.num_experts, W=self.world_size, H=cfg.hidden_dim,
                 in_type=_elem(cfg.in_dtype), out_type=_elem(cfg.out_dtype), disp=_ptr(b["disp_x"]),

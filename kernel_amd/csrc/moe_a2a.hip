@@ -679,11 +679,11 @@ int moe_a2a_dispatch_once(const moe_a2a_forward_args* a) {
     if (a->in_type != MOE_A2A_F16 && a->in_type != MOE_A2A_BF16) return MOE_A2A_E_DTYPE;
     return route_dispatch_fp8_impl(a->x, a->in_type, a->indices, a->rank_start, a->src_rank, T, K, a->E, a->W, H, 0, a->counts,
                                    a->offsets, a->slot_of_entry, a->src_of_slot, a->meta, a->status, a->disp, a->disp_scale,
-                                   a->fp8_dispatch == 2, (hipStream_t)a->stream, nullptr, 1);
+                                   a->fp8_dispatch == 2, (hipStream_t)a->stream, a->clear_status, 1);
   }
   if (!(a->fuse_route == 2 && R <= moe_a2a_fused_max_rows()) && !moe_a2a_fused_ok(T, K, H)) return MOE_A2A_E_STATE;
   return route_dispatch_impl(a->x, a->indices, a->rank_start, a->src_rank, T, K, a->E, a->W, H, 0, a->counts, a->offsets,
-                             a->slot_of_entry, a->src_of_slot, a->meta, a->status, a->disp, a->stream, nullptr, 1);
+                             a->slot_of_entry, a->src_of_slot, a->meta, a->status, a->disp, a->stream, a->clear_status, 1);
 }
 
 static bool known_type(int t) { return t == MOE_A2A_F16 || t == MOE_A2A_BF16; }

@@ -650,6 +650,34 @@ def test_status_describes_the_call_that_produced_it(gpu_device, name, fp8, fuse_
         assert int(ata.dispatch(x, ids, rs).status.item()) == bits_want
 
 
+@pytest.mark.parametrize("first", ["forward", "dispatch"])
+@pytest.mark.parametrize("fp8,fuse_route,padded", [(False, True, False), (True, True, False), ("pow2", True, False),
+                                                   (False, False, False), (True, False, False), (False, True, True)])
+@pytest.mark.parametrize("name", ["tiny", "dsv3_rank", "skew_world"])
+def test_status_of_mixed_calls(gpu_device, name, fp8, fuse_route, padded, first):
+    """Forwards and dispatches of one token count share two buffer sets: a call with bad ids on one set, a dispatch on the
+    other, and the forward that meets the first set again reports its own ids, which are good.  The record of a dispatch keeps
+    its word behind a second dispatch."""
+    wl = C.generate_workload(name)
+    x, idx, w, rs = concat_world(wl.world, gpu_device)
+    bad = idx.clone()
+    bad[-1, -1] = -1
+    ata = HipAllToAll(wl.cfg, 0, wl.world_size, stub_kind=wl.stub_kind, fp8_dispatch=fp8, fuse_route=fuse_route, padded=padded)
+    for _ in range(2):  # either set first
+        for between in ((idx,), (bad, idx, idx), (idx, bad, idx)):  # an odd number: the other set last
+            if first == "forward":
+                ata.forward(x, bad, w, rs)
+                assert int(ata.last.status.item()) == _lib.STATUS_BAD_EXPERT
+            else:
+                assert int(ata.dispatch(x, bad, rs).status.item()) == _lib.STATUS_BAD_EXPERT
+            for ids in between:
+                assert int(ata.dispatch(x, ids, rs).status.item()) == (_lib.STATUS_BAD_EXPERT if ids is bad else 0)
+            ata.forward(x, idx, w, rs, check_status=True)
+        one, two = ata.dispatch(x, bad, rs), ata.dispatch(x, idx, rs)
+        assert (int(one.status.item()), int(two.status.item())) == (_lib.STATUS_BAD_EXPERT, 0)
+        ata.forward(x, idx, w, rs, check_status=True)
+
+
 def test_custom_kernel_check_status_and_config_changed_in_place(gpu_device):
     """`custom_kernel(data, check_status=True)` raises on an id the reference would fail on; a config
     object changed in place between two calls gets the instance of its new values."""
