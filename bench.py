@@ -883,7 +883,7 @@ def expert_gemm_leg(args, lib, torch, wl, x, idx, rs, dev):
         e1.record(main)
         main.synchronize()
     ms_step = e0.elapsed_time(e1) / args.steps
-    kernel = next(k for k in ("expert_gemm_mx", "expert_gemm_f8", "expert_gemm_wide", "expert_gemm_skinny", "expert_gemm") if k in per)
+    kernel = next(k for k in per if k.startswith("expert_gemm"))
     t_us = statistics.fmean(per[kernel])
     flops = 2.0 * R * H * N
     tflops = flops / t_us / 1e6
@@ -901,8 +901,9 @@ def expert_gemm_leg(args, lib, torch, wl, x, idx, rs, dev):
     # the output); if that takes longer at 8 TB/s than the flops at the MFMA peak, the launch is HBM-bound
     live = int((d.counts > 0).sum())
     # the kernel with both operands fp8 multiplies on the fp8 matrix instruction (dense peak 5.0 PFLOP/s)
-    mfma_peak = FP8_MFMA_PEAK_TFLOPS if kernel in ("expert_gemm_f8", "expert_gemm_mx") else MFMA_PEAK_TFLOPS
-    if kernel in ("expert_gemm_f8", "expert_gemm_mx") or (fp8 and args.fp8_weights):
+    fp8_kernel = kernel.endswith(("_f8", "_mx"))
+    mfma_peak = FP8_MFMA_PEAK_TFLOPS if fp8_kernel else MFMA_PEAK_TFLOPS
+    if fp8_kernel or (fp8 and args.fp8_weights):
         out["dtype"] = "fp8"
     gemm_bytes = R * H * (1 + 4 / 128 if fp8 else 2) + live * N * H * (1 if args.fp8_weights else 2) + R * N * 2
     if gemm_bytes / (HBM_PEAK_GBPS * 1e3) > flops / (mfma_peak * 1e6):

@@ -301,11 +301,12 @@ def test_tile_width_where_wide_tiles_begin(gpu_device, m, n, k, kernel):
 
 
 @pytest.mark.gpu
-def test_partial_products_are_optional_for_many_tiles(gpu_device):
+@pytest.mark.parametrize("k,grouped", [(20160, "gemm_rs_split"), (16384, "gemm_rs_narrow")])
+def test_partial_products_are_optional_for_many_tiles(gpu_device, k, grouped):
     """185 tiles of 256 x 128 with shards long enough that groups of them pay: the call is accepted without a workspace, with
     one that is too small and with one off its alignment, and then sums all shards in one place.  f32 sums of k products
     of up to 0.05^2, rounded once: within 2^-8 of the f32 product and 2e-5."""
-    lib, W, m, n, k = _lib.load(), 8, 1176, 4672, 20160
+    lib, W, m, n = _lib.load(), 8, 1176, 4672
     g = torch.Generator(device=gpu_device).manual_seed(3)
     x = torch.empty(W, m, k // W, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
     w = torch.empty(W, n, k // W, dtype=torch.bfloat16, device=gpu_device).uniform_(-0.05, 0.05, generator=g)
@@ -316,7 +317,7 @@ def test_partial_products_are_optional_for_many_tiles(gpu_device):
     outs = []
     for at, size, kernels in ((None, 0, ["gemm_rs_narrow"]), (ws.data_ptr(), need - 1, ["gemm_rs_narrow"]),
                               (ws.data_ptr() + 8, need, ["gemm_rs_narrow"]),
-                              (ws.data_ptr(), need, ["gemm_rs_narrow", "gemm_rs_reduce"])):
+                              (ws.data_ptr(), need, [grouped, "gemm_rs_reduce"])):
         out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
 
         def call():
@@ -493,7 +494,7 @@ def test_wide_tiles_with_the_shards_in_groups(gpu_device, options, dtype, W, m, 
     w[0, n - 1, kl - 8] = float("-inf")
     out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
     kernels = launched(_lib.load(), lambda: G.HipGemmReduceScatter(W).forward(x, w, bias, out=out))
-    assert kernels == ["gemm_rs_narrow", "gemm_rs_reduce"]
+    assert kernels == ["gemm_rs_split", "gemm_rs_reduce"]
     want = product(x, w, bias)
     assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
     ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
@@ -501,12 +502,14 @@ def test_wide_tiles_with_the_shards_in_groups(gpu_device, options, dtype, W, m, 
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("W,m,n,k,groups", [(8, 512, 5440, 17024, 4), (8, 240, 4480, 24128, 8), (8, 1096, 6400, 6464, 2),
-                                            (4, 304, 5696, 11328, 4), (8, 120, 4160, 11008, 8)])
-def test_room_for_the_groups_is_optional(gpu_device, W, m, n, k, groups):
+@pytest.mark.parametrize("W,m,n,k,groups,narrow", [(8, 512, 5440, 17024, 4, "groups"), (8, 240, 4480, 24128, 8, "groups"),
+                                                   (8, 1096, 6400, 6464, 2, "whole"), (4, 304, 5696, 11328, 4, "groups"),
+                                                   (8, 120, 4160, 11008, 8, "groups")])
+def test_room_for_the_groups_is_optional(gpu_device, options, W, m, n, k, groups, narrow):
     """Shapes that take 256 x 256 tiles in groups: room for their partial products is what is asked for, and with less of it, or off its
-    alignment, the call is answered as it is without that form: on the 256 x 128 tiles, with what they need, or MOE_A2A_E_WORKSPACE.
-    Shards that lie apart as well.  Tolerance as above, 2e-5."""
+    alignment, the call is answered as it is without that form: on the 256 x 128 tiles, in fewer groups, which have to have room (or
+    MOE_A2A_E_WORKSPACE, MOE_A2A_E_ALIGN), or, where these give most CUs a tile (250 of them), whole, with no room at all and
+    the bits of that form.  Shards that lie apart as well.  Tolerance as above, 2e-5."""
     lib = _lib.load()
     pad = 64
     x, w = uniform((W, m * (k // W) + pad), torch.bfloat16, gpu_device, 5), uniform((W, n * (k // W) + pad), torch.bfloat16, gpu_device, 6)
@@ -514,18 +517,25 @@ def test_room_for_the_groups_is_optional(gpu_device, W, m, n, k, groups):
     need = lib.gemm_rs_workspace_bytes(m, n, k, W)
     assert need == groups * m * n * 4
     ws = torch.empty(need + 16, dtype=torch.uint8, device=gpu_device)
-    answers = []
-    for at, size in ((ws.data_ptr(), need), (ws.data_ptr(), need - 1), (ws.data_ptr() + 8, need), (None, 0)):
+
+    def call(at, size):
         out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
-        rc = lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, k, W, m * (k // W) + pad, n * (k // W) + pad,
-                                 _lib.BF16, at, size, torch.cuda.current_stream().cuda_stream)
-        torch.cuda.synchronize()
-        answers.append(rc)
-        if rc == 0:
-            assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
-        else:
-            assert rc in (E_WORKSPACE, E_ALIGN) and bool(out.isnan().all())
-    assert answers[0] == 0
+        rc = []
+        kernels = launched(lib, lambda: rc.append(lib.gemm_rs_forward(
+            x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, k, W, m * (k // W) + pad, n * (k // W) + pad, _lib.BF16, at, size,
+            torch.cuda.current_stream().cuda_stream)))
+        assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all()) if rc == [0] else bool(out.isnan().all())
+        return rc + kernels, out
+
+    assert call(ws.data_ptr(), need)[0] == [0, "gemm_rs_split", "gemm_rs_reduce"]
+    less = (ws.data_ptr(), need - 1), (ws.data_ptr() + 8, need), (None, 0)
+    if narrow == "groups":
+        assert [call(*room)[0] for room in less] == [[0, "gemm_rs_narrow", "gemm_rs_reduce"], [E_ALIGN], [E_WORKSPACE]]
+    else:
+        got = [call(*room) for room in less]
+        options.set("GEMM_TILE", 129)
+        got.append(call(None, 0))
+        assert all(how == [0, "gemm_rs_narrow"] and torch.equal(out, got[0][1]) for how, out in got)
 
 
 @pytest.mark.gpu

@@ -875,6 +875,7 @@ def test_expert_gemm_16bit_longest_rows(gpu_device, options, Kd):
     assert bool(((y.double() - want).abs() <= want.abs() * 2 ** -8 + 5e-4).all())
 
 
+STRIP_NAMES = {"16bit": "expert_gemm_strip", "fp8": "expert_gemm_strip_f8", "pow2": "expert_gemm_strip_mx", "w8": "expert_gemm_strip_w8"}
 # rows of a segment around the forms of a strip (64, 96, 112, 128, 144, 160, 176) and of two and more of them
 STRIP_COUNTS = [1, 16, 17, 64, 65, 96, 97, 112, 113, 0, 128, 129, 144, 145, 160, 161, 175, 176, 177, 352, 353, 900]
 
@@ -907,17 +908,21 @@ def test_strips(gpu_device, options, dtype, padded, form, slabs, N, counts):
         kw = dict(w_scale=ws.to(gpu_device), scales_pow2=form == "pow2")
         x32 = d.disp_x.float() if form == "w8" else d.disp_x.view(torch.float8_e4m3fn).float() * d.disp_scale.repeat_interleave(128, 1)
         w32 = wd.view(torch.float8_e4m3fn).float() * kw["w_scale"].repeat_interleave(128, 1).repeat_interleave(128, 2)
+    # (power-of-two scales of up to 32 rows on average take the kernels for any scale)
+    strip = STRIP_NAMES["fp8" if form == "pow2" and sum(counts) <= 32 * len(counts) else form]
     got = {}
     for tile, staged in ((512, 0), (128 if form == "fp8" else 32 if form == "w8" else 256, 3)):
         options.set("GEMM_TILE", tile)
         options.set("GEMM_STAGED", staged)
-        got[tile] = ata.expert_gemm(d, wd, **kw)[rows].clone()
+        result = []
+        names = launched(ata.lib, lambda: result.append(ata.expert_gemm(d, wd, **kw)) or 0)
+        assert len(names) == 1 and (names[0] == strip if tile == 512 else "strip" not in names[0]), names
+        got[tile] = result[0][rows].clone()
     torch.cuda.synchronize()
     want = torch.cat([x32[(first := e * room if padded else int(off[e])):first + n] @ w32[e].T for e, n in enumerate(lens)])
     close(got[512], want.cpu())
     first, second = got.values()
-    # (fp8 weights: the streaming kernel walks K in another order; power-of-two scales of up to 32 rows on average take the kernels
-    # for any scale)
+    # (fp8 weights: the streaming kernel walks K in another order)
     if form not in ("pow2", "w8") or (form == "pow2" and sum(counts) > 32 * len(counts)):
         assert torch.equal(first.view(torch.int16), second.view(torch.int16))
 
@@ -932,7 +937,7 @@ def test_strips(gpu_device, options, dtype, padded, form, slabs, N, counts):
     ("w8", 256, 256, 512, {32: "expert_gemm_skinny", 33: "strip"}),
 ])
 def test_where_strips_are_taken(gpu_device, options, form, E, Kd, N, kernels):
-    """Lengths on both sides of every border: strips go by the name of their format's 256 x 256 tiles.  Products of ones."""
+    """Lengths on both sides of every border.  Products of ones."""
     lib = _lib.load()
     for rows, name in kernels.items():
         R = rows * E
@@ -951,6 +956,5 @@ def test_where_strips_are_taken(gpu_device, options, form, E, Kd, N, kernels):
             f = lib.moe_a2a_expert_gemm_mx8 if form == "pow2" else lib.moe_a2a_expert_gemm_q8
             call = lambda: f(x.data_ptr(), None if form == "w8" else xs.data_ptr(), w.data_ptr(), ws.data_ptr(), *tail)
         got = launched(lib, call)
-        family = {"16bit": "expert_gemm_wide", "fp8": "expert_gemm_f8", "pow2": "expert_gemm_mx", "w8": "expert_gemm_wide"}[form]
-        assert got == [family if name == "strip" else name], rows
+        assert got == [STRIP_NAMES[form] if name == "strip" else name], rows
         assert bool((y == Kd).all()), rows
