@@ -927,6 +927,52 @@ def test_strips(gpu_device, options, dtype, padded, form, slabs, N, counts):
         assert torch.equal(first.view(torch.int16), second.view(torch.int16))
 
 
+def product_of(lib, form, x, xs, w, ws, off, y):
+    """y = x w^T through the form's entry point; the kernels that were launched."""
+    E, N, Kd = w.shape
+    tail = (off.data_ptr(), y.data_ptr(), x.shape[0], E, Kd, N, 0, _lib.BF16, torch.cuda.current_stream().cuda_stream)
+    if form == "16bit":
+        return launched(lib, lambda: lib.moe_a2a_expert_gemm(x.data_ptr(), w.data_ptr(), *tail))
+    f = lib.moe_a2a_expert_gemm_mx8 if form == "pow2" else lib.moe_a2a_expert_gemm_q8
+    return launched(lib, lambda: f(x.data_ptr(), None if form == "w8" else xs.data_ptr(), w.data_ptr(), ws.data_ptr(), *tail))
+
+
+@pytest.mark.parametrize("form,rows,Kd,fits", [("16bit", 176, 2097088, True), ("16bit", 176, 2097152, False), ("fp8", 176, 4194176, True),
+                                               ("pow2", 176, 4194176, True), ("w8", 160, 2097024, True)])
+def test_longest_rows_of_a_strip(gpu_device, options, form, rows, Kd, fits):
+    """A full strip of rows so long that its 512 rows of weights come to the end of 31 bits, and a slab more, which is left to the
+    256 x 256 tiles.  x is zero but for the first and the last 128 columns, so that a row, a column or a slab that is fetched from a place
+    other than its own shows.  Tolerance: one rounding to bf16, and f32 sums of 256 products, 2^-24 of their absolute sum each."""
+    N = 512
+    g = torch.Generator(device=gpu_device).manual_seed(Kd)
+    cols = torch.cat([torch.arange(128), torch.arange(Kd - 128, Kd)]).to(gpu_device)
+    part = torch.randn(rows, 256, device=gpu_device, generator=g)
+    if form == "16bit":
+        w = torch.empty(1, N, Kd, dtype=torch.bfloat16, device=gpu_device).normal_(generator=g)
+        w32 = w[0][:, cols].float()
+    else:
+        w = torch.empty(1, N, Kd, dtype=torch.uint8, device=gpu_device).random_(0x20, 0x48, generator=g)  # 2^-4 .. 4, no NaN
+        w32 = w[0][:, cols].view(torch.float8_e4m3fn).float()
+    scales = lambda *shape: torch.exp2(torch.randint(-2, 3, shape, device=gpu_device, generator=g).float()) * (1.0 if form == "pow2" else 1.3)
+    xs, ws = (scales(rows, Kd // 128), scales(1, N // 128, Kd // 128)) if form != "16bit" else (None, None)
+    dtype = torch.bfloat16 if form in ("16bit", "w8") else torch.float8_e4m3fn
+    part = part.to(dtype)
+    x = torch.zeros(rows, Kd, dtype=torch.uint8 if dtype == torch.float8_e4m3fn else dtype, device=gpu_device)
+    x[:, cols] = part.view(x.dtype)
+    x32 = part.float()
+    if form != "16bit":
+        if form != "w8":
+            x32 = x32 * xs[:, cols // 128]
+        w32 = w32 * ws[0][:, cols // 128].repeat_interleave(128, 0)
+    y = torch.full((rows, N), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    off = torch.tensor([0, rows], dtype=torch.int32, device=gpu_device)
+    options.set("GEMM_TILE", 512)
+    names = product_of(_lib.load(), form, x, xs, w, ws, off, y)
+    assert names == [STRIP_NAMES[form] if fits else "expert_gemm"]
+    want, size = x32.double() @ w32.double().T, x32.double().abs() @ w32.double().abs().T
+    assert bool(((y.double() - want).abs() <= want.abs() * 2 ** -8 + size * 2.0 ** -16).all())
+
+
 @pytest.mark.parametrize("form,E,Kd,N,kernels", [
     ("16bit", 256, 512, 1024, {15: "expert_gemm_skinny", 16: "strip", 144: "strip", 145: "expert_gemm_wide", 290: "strip", 311: "expert_gemm_wide"}),
     ("fp8", 256, 1024, 1024, {15: "expert_gemm_skinny", 16: "strip", 144: "strip", 145: "expert_gemm_f8", 250: "strip", 311: "expert_gemm_f8"}),
@@ -949,12 +995,6 @@ def test_where_strips_are_taken(gpu_device, options, form, E, Kd, N, kernels):
         xs, ws = torch.ones(R, Kd // 128, device=gpu_device), torch.ones(E, N // 128, Kd // 128, device=gpu_device)
         y = torch.zeros(R, N, dtype=torch.bfloat16, device=gpu_device)
         off = torch.arange(0, R + 1, rows, dtype=torch.int32, device=gpu_device)
-        tail = (off.data_ptr(), y.data_ptr(), R, E, Kd, N, 0, _lib.BF16, torch.cuda.current_stream().cuda_stream)
-        if form == "16bit":
-            call = lambda: lib.moe_a2a_expert_gemm(x.data_ptr(), w.data_ptr(), *tail)
-        else:
-            f = lib.moe_a2a_expert_gemm_mx8 if form == "pow2" else lib.moe_a2a_expert_gemm_q8
-            call = lambda: f(x.data_ptr(), None if form == "w8" else xs.data_ptr(), w.data_ptr(), ws.data_ptr(), *tail)
-        got = launched(lib, call)
+        got = product_of(lib, form, x, xs, w, ws, off, y)
         assert got == [STRIP_NAMES[form] if name == "strip" else name], rows
         assert bool((y == Kd).all()), rows
