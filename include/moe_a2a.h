@@ -286,7 +286,7 @@ int moe_a2a_forward_launches(int T, int K, int H, int max_recv, int in_type, int
  *   x[rows, Kd], weights[E, N, Kd], y[rows, N]: 16-bit elements of elem_type, f32 accumulation,
  *   Kd % 64 == 0, N % 8 == 0, 16-byte aligned.
  * Four kernels with identical results: tiles of up to 176 rows by 512 columns from some tens of
- * rows per expert to 144, and for some 300, where these are at least a round of the CUs
+ * rows per expert to 104 .. 144, and for some 300, where these are a round and a half of the CUs or more
  * (MOE_A2A_OPT_GEMM_TILE = 512 forces them, wherever they apply, in this and the next entry
  * points); 32 x 64 tiles that stream the weights when segments are
  * short (R <= 32 * E, 25 * E with more than 1 GiB of weights, 16 * E if Kd % 128 != 0); 256 x 256
@@ -333,7 +333,7 @@ int moe_a2a_expert_gemm_fp8(const void* x_q, const float* x_scale, const void* w
  *     MOE_A2A_OPT_GEMM_STAGED = 2, and Kd = 128, take four waves on 128 x 128 tiles with the
  *     32x32x64 one), each 128-wide K block is summed in f32 and folded with
  *     x_scale[row][kb] * w_scale[n / 128][kb]; nothing is rounded before the output.
- *   16-bit rows, more than 24 rows per expert where there are at least 512 tiles of 512 columns, or 32
+ *   16-bit rows, more than 24 rows per expert where there are at least 2048 tiles of 512 columns, or 32
  *     where there are at least 256: tiles of up to 160 rows by 512 columns, with the arithmetic of the
  *     decode step (nothing is rounded before the output);
  *   longer segments, 16-bit rows (and N >= 256): the 256 x 256 kernel; a weight enters the matrix

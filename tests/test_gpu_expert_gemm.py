@@ -974,13 +974,24 @@ def test_longest_rows_of_a_strip(gpu_device, options, form, rows, Kd, fits):
 
 
 @pytest.mark.parametrize("form,E,Kd,N,kernels", [
-    ("16bit", 256, 512, 1024, {15: "expert_gemm_skinny", 16: "strip", 144: "strip", 145: "expert_gemm_wide", 290: "strip", 311: "expert_gemm_wide"}),
-    ("fp8", 256, 1024, 1024, {15: "expert_gemm_skinny", 16: "strip", 144: "strip", 145: "expert_gemm_f8", 250: "strip", 311: "expert_gemm_f8"}),
+    ("16bit", 256, 512, 1024, {15: "expert_gemm_skinny", 16: "strip", 140: "strip", 141: "expert_gemm_wide", 289: "expert_gemm_wide",
+                               290: "strip", 310: "strip", 311: "expert_gemm_wide"}),
+    ("16bit", 256, 512, 2048, {104: "strip", 105: "expert_gemm_wide"}),  # four rounds
+    ("16bit", 256, 512, 768, {23: "expert_gemm_skinny", 24: "strip", 112: "strip", 113: "expert_gemm_wide", 300: "expert_gemm_wide"}),
+    ("16bit", 255, 512, 768, {100: "expert_gemm_wide"}),
+    ("fp8", 256, 1024, 1024, {15: "expert_gemm_skinny", 16: "strip", 144: "strip", 145: "expert_gemm_f8", 249: "expert_gemm_f8",
+                              250: "strip", 310: "strip", 311: "expert_gemm_f8"}),
+    ("fp8", 256, 1024, 768, {23: "expert_gemm_f8", 24: "strip", 120: "strip", 121: "expert_gemm_f8", 300: "expert_gemm_f8"}),
+    ("fp8", 256, 1024, 512, {95: "expert_gemm_f8", 96: "strip", 128: "strip", 129: "expert_gemm_f8", 300: "expert_gemm_f8"}),
     ("fp8", 256, 896, 1536, {100: "expert_gemm_f8"}),  # less than eight slabs
-    ("pow2", 256, 1024, 512, {95: "expert_gemm_mx", 96: "strip", 128: "strip", 129: "expert_gemm_mx", 290: "strip"}),
     ("fp8", 255, 1024, 512, {100: "expert_gemm_f8"}),  # less than one round
-    ("w8", 256, 256, 1024, {24: "expert_gemm_skinny", 25: "strip", 700: "strip"}),
+    ("pow2", 256, 1024, 512, {95: "expert_gemm_mx", 96: "strip", 128: "strip", 129: "expert_gemm_mx"}),
+    ("pow2", 256, 1024, 1024, {33: "strip", 140: "strip", 141: "expert_gemm_mx", 300: "expert_gemm_mx"}),
+    ("pow2", 256, 1024, 4096, {144: "strip", 145: "expert_gemm_mx", 289: "expert_gemm_mx", 290: "strip", 310: "strip", 311: "expert_gemm_mx"}),
+    ("w8", 256, 256, 4096, {24: "expert_gemm_skinny", 25: "strip"}),
+    ("w8", 256, 256, 1024, {32: "expert_gemm_skinny", 33: "strip", 700: "strip"}),
     ("w8", 256, 256, 512, {32: "expert_gemm_skinny", 33: "strip"}),
+    ("w8", 255, 256, 512, {33: "expert_gemm_wide"}),
 ])
 def test_where_strips_are_taken(gpu_device, options, form, E, Kd, N, kernels):
     """Lengths on both sides of every border.  Products of ones."""
