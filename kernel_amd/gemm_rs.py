@@ -9,6 +9,7 @@ is in ``libmoe_a2a.so``; torch supplies device memory and the current stream.
 """
 from __future__ import annotations
 
+import threading
 from typing import List, Optional, Sequence, Tuple
 
 import torch
@@ -73,7 +74,9 @@ def pack_world(datas: Sequence[Data], device: torch.device):
 
 class HipGemmReduceScatter:
     """``forward(input[W, M, Kl], weight[W, N, Kl], bias)`` -> ``out[M, N]``; ``out[r*M/W:(r+1)*M/W]``
-    is what rank r of the reference returns."""
+    is what rank r of the reference returns.  Calls may run on several streams, and come from several threads, at once."""
+
+    MAX_WORKSPACES = 4  # streams whose workspace is kept between calls
 
     def __init__(self, world_size: int, pad_ragged: bool = True):
         self.world_size = int(world_size)
@@ -81,15 +84,23 @@ class HipGemmReduceScatter:
         # a zero-padded, line-aligned copy of the operands) is multiplied in place, without it
         self.pad_ragged = bool(pad_ragged)
         self.lib = _lib.load()
-        self._workspace = None
+        self._workspaces = {}  # (device, stream) -> workspace of the calls on that stream
+        self._making = threading.Lock()
 
     def workspace_for(self, m: int, n: int, k: int, device) -> Optional[torch.Tensor]:
         need = int(self.lib.gemm_rs_workspace_bytes(m, n, k, self.world_size))
         if need == 0:
             return None
-        if self._workspace is None or self._workspace.numel() < need or self._workspace.device != device:
-            self._workspace = torch.empty(need, dtype=torch.uint8, device=device)
-        return self._workspace
+        if torch.cuda.is_current_stream_capturing():  # the graph's own: it may outlive this object and run beside other calls
+            return torch.empty(need, dtype=torch.uint8, device=device)
+        key = device, torch.cuda.current_stream(device).cuda_stream
+        ws = self._workspaces.get(key)
+        if ws is None or ws.numel() < need:
+            with self._making:
+                while key not in self._workspaces and len(self._workspaces) >= self.MAX_WORKSPACES:
+                    del self._workspaces[next(iter(self._workspaces))]  # (torch reuses its memory behind the work of its stream)
+                ws = self._workspaces[key] = torch.empty(need, dtype=torch.uint8, device=device)
+        return ws
 
     def forward(self, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
                 out: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -547,3 +547,41 @@ def test_wide_tiles_dealt_out_in_column_order(gpu_device, m, n):
     assert launched(_lib.load(), lambda: G.HipGemmReduceScatter(8).forward(x, w, out=out)) == ["gemm_rs_wide"]
     want = product(x, w)
     assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6).all())
+
+
+@pytest.mark.gpu
+def test_workspace_of_a_stream_and_of_a_graph(gpu_device):
+    """Calls on two streams at once do not share their partial products, and a captured graph has room of its own, which the handle's
+    later calls, or its end, do not take away.  A kept workspace belongs to one stream and is found again; four are kept."""
+    W, m, n, k = 8, 1096, 6400, 6464
+    h = G.HipGemmReduceScatter(W)
+    streams = [torch.cuda.Stream() for _ in range(6)]
+
+    def room(stream):
+        with torch.cuda.stream(stream):
+            return h.workspace_for(m, n, k, gpu_device)
+
+    a, b = room(streams[0]), room(streams[1])
+    assert a.data_ptr() != b.data_ptr() and room(streams[0]) is a and room(streams[1]) is b
+    with torch.cuda.stream(streams[1]):
+        assert h.workspace_for(64, 256, 1024, gpu_device) is b  # (a smaller one)
+    graph, held = torch.cuda.CUDAGraph(), []
+    x, w = uniform((W, m, k // W), torch.bfloat16, gpu_device, 1), uniform((W, n, k // W), torch.bfloat16, gpu_device, 2)
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=gpu_device)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        held.append(h.workspace_for(m, n, k, gpu_device).data_ptr())
+        h.forward(x, w, out=out)
+    assert held[0] not in (a.data_ptr(), b.data_ptr()) and room(streams[0]) is a
+    for s in streams:
+        room(s)
+    assert len(h._workspaces) == h.MAX_WORKSPACES and room(streams[5]) is room(streams[5])
+    del h, a, b
+    other = [torch.full((need,), 7, dtype=torch.uint8, device=gpu_device) for need in [2 * m * n * 4] * 8]  # whatever was given back
+    want = product(x, w)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
+        assert all(bool((o == 7).all()) for o in other)
