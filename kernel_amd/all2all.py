@@ -178,9 +178,8 @@ class HipAllToAll:
         # both sets of a new shape are allocated together, so that the second call with this shape
         # does not meet an allocation either
         sets = [self._allocate(T, device), self._allocate(T, device)]
-        for b, other in zip(sets, reversed(sets)):  # a call on one set clears the status word of the other (see Dispatched.status)
-            b.update(partner_status=other["status"], dispatch_status=other.get("lent_status"),
-                     dispatch_clears=other.get("lent_clears"))
+        for i in (0, 1):  # a call on one set clears the status word of the other (see Dispatched.status)
+            sets[i]["partner_status"] = sets[i ^ 1]["status"]
         cfg = self.cfg
         native = _lib.host().Ring(T, cfg.experts_per_token, cfg.hidden_dim, self.world_size, device.index, cfg.in_dtype,
                                   cfg.out_dtype)
@@ -195,17 +194,13 @@ class HipAllToAll:
         R = T * K
         rows = E * self.max_recv if self.padded else R  # rows of the dispatched buffers
         i32 = dict(dtype=torch.int32, device=device)
-        # this set's word of a forward and the other set's of a dispatch, which a dispatch there clears together; a line each
-        words = torch.zeros(2, 32, **i32)
         b = dict(
             counts=torch.empty(E, **i32),
             offsets=torch.empty(E + 1, **i32),
             slot_of_entry=torch.empty(R, **i32),
             src_of_slot=torch.empty(rows, **i32),
             meta=torch.empty(rows, META_DIM, **i32),
-            status=words[0, :1],
-            lent_status=words[1, :1],
-            lent_clears=words[:, :1],
+            status=torch.zeros(1, **i32),
             workspace=torch.empty(max(self.lib.moe_a2a_workspace_bytes(T, K, E), 256), dtype=torch.uint8,
                                   device=device),
             # the stub's output rows exist only where the stub is a launch of its own (expert_stub
@@ -257,10 +252,14 @@ class HipAllToAll:
             if rank_start.dtype != torch.int32 or rank_start.numel() != W + 1:
                 raise ValueError("rank_start must be int32[world_size + 1]")
         b = self._buffers(T, dp_x.device, advance=True)
+        if "dispatch_status" not in b:  # the set's first dispatch
+            with self._making:
+                b.setdefault("dispatch_status", torch.empty_like(b["status"]))
         if self.fuse_route and not self.padded and self._dispatch_once(b, dp_x, indices, rank_start):
             return Dispatched(cfg, W, T, b["counts"], b["offsets"], b["slot_of_entry"], b["src_of_slot"], b["meta"],
                               b["disp_x"], b["disp_scale"], b["dispatch_status"], 0)
-        b["dispatch_clears"].zero_()  # the phase-by-phase entry points only ever set bits: the record describes this call
+        # the phase-by-phase entry points only ever set bits: the record describes this call (one launch)
+        torch._foreach_zero_((b["dispatch_status"], b["partner_status"]))
         lib, st = self.lib, _stream()
         pad = self.max_recv if self.padded else 0
         route_out = (_ptr(b["counts"]), _ptr(b["offsets"]), _ptr(b["slot_of_entry"]), _ptr(b["src_of_slot"]),

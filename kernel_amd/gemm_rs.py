@@ -15,6 +15,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
+from .all2all import _stream
 
 # the reference's test and benchmark specs (gemm_rs/task.yml:59-79)
 TEST_SPECS = [
@@ -93,7 +94,8 @@ class HipGemmReduceScatter:
             return None
         if torch.cuda.is_current_stream_capturing():  # the graph's own: it may outlive this object and run beside other calls
             return torch.empty(need, dtype=torch.uint8, device=device)
-        key = device, torch.cuda.current_stream(device).cuda_stream
+        index = torch.device(device).index
+        key = index, _stream(index)
         ws = self._workspaces.get(key)
         if ws is None or ws.numel() < need:
             with self._making:
@@ -122,7 +124,7 @@ class HipGemmReduceScatter:
             return self.lib.gemm_rs_forward(
                 x.data_ptr(), w.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(), M, N, Kl * W,
                 W, 0, 0, _lib.BF16 if x.dtype == torch.bfloat16 else _lib.F16, ws.data_ptr() if ws is not None else None,
-                ws.numel() if ws is not None else 0, torch.cuda.current_stream(x.device).cuda_stream)
+                ws.numel() if ws is not None else 0, _stream(x.device.index))
 
         rc = call(None) if not self.pad_ragged else -4
         if rc == -4:  # MOE_A2A_E_WORKSPACE: this shape's form needs its workspace (nothing was launched)
