@@ -286,7 +286,7 @@ int moe_a2a_forward_launches(int T, int K, int H, int max_recv, int in_type, int
  *   x[rows, Kd], weights[E, N, Kd], y[rows, N]: 16-bit elements of elem_type, f32 accumulation,
  *   Kd % 64 == 0, N % 8 == 0, 16-byte aligned.
  * Four kernels with identical results: tiles of up to 176 rows by 512 columns from some tens of
- * rows per expert to 104 .. 144, and for some 300, where these are a round and a half of the CUs or more
+ * rows per expert to 112 .. 144 (of 16 bits up to 104 MiB), and for some 300, where these are a round and a half of the CUs or more
  * (MOE_A2A_OPT_GEMM_TILE = 512 forces them, wherever they apply, in this and the next entry
  * points); 32 x 64 tiles that stream the weights when segments are
  * short (R <= 32 * E, 25 * E with more than 1 GiB of weights, 16 * E if Kd % 128 != 0); 256 x 256

@@ -976,7 +976,9 @@ def test_longest_rows_of_a_strip(gpu_device, options, form, rows, Kd, fits):
 @pytest.mark.parametrize("form,E,Kd,N,kernels", [
     ("16bit", 256, 512, 1024, {15: "expert_gemm_skinny", 16: "strip", 140: "strip", 141: "expert_gemm_wide", 289: "expert_gemm_wide",
                                290: "strip", 310: "strip", 311: "expert_gemm_wide"}),
-    ("16bit", 256, 512, 2048, {104: "strip", 105: "expert_gemm_wide"}),  # four rounds
+    ("16bit", 256, 512, 2048, {140: "strip", 141: "expert_gemm_wide"}),
+    ("16bit", 256, 2048, 1024, {104: "strip", 105: "expert_gemm_wide"}),  # 104 MiB of rows
+    ("16bit", 64, 8192, 5120, {128: "strip", 129: "expert_gemm_wide"}),  # more, 40 columns per row
     ("16bit", 256, 512, 768, {23: "expert_gemm_skinny", 24: "strip", 112: "strip", 113: "expert_gemm_wide", 300: "expert_gemm_wide"}),
     ("16bit", 255, 512, 768, {100: "expert_gemm_wide"}),
     ("fp8", 256, 1024, 1024, {15: "expert_gemm_skinny", 16: "strip", 144: "strip", 145: "expert_gemm_f8", 249: "expert_gemm_f8",
