@@ -678,6 +678,34 @@ def test_status_of_mixed_calls(gpu_device, name, fp8, fuse_route, padded, first)
         ata.forward(x, idx, w, rs, check_status=True)
 
 
+@pytest.mark.parametrize("fp8,fuse_route", [(False, True), (True, True), (False, False), ("pow2", False)])
+def test_status_of_a_captured_dispatch(gpu_device, fp8, fuse_route):
+    """Every replay of a captured dispatch reports the ids that it meets, and clears the word that the next forward of the eager
+    program, on the other set, would otherwise find as it left it."""
+    wl = C.generate_workload("skew_world")
+    x, idx, w, rs = concat_world(wl.world, gpu_device)
+    bad, table = idx.clone(), idx.clone()
+    bad[3, 0] = wl.cfg.num_experts + 7
+    ata = HipAllToAll(wl.cfg, 0, wl.world_size, stub_kind=wl.stub_kind, fp8_dispatch=fp8, fuse_route=fuse_route)
+    for _ in range(2):
+        ata.dispatch(x, table, rs)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        d = ata.dispatch(x, table, rs)
+    for ids in (idx, bad, idx, bad, bad, idx):
+        ata.forward(x, bad, w, rs)  # on the set that the graph is not on
+        table.copy_(ids)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert int(d.status.item()) == (_lib.STATUS_BAD_EXPERT if ids is bad else 0)
+        want = ata.dispatch(x, ids.clamp(0, wl.cfg.num_experts - 1), rs)  # (on the graph's set, whose buffers the next replay fills again)
+        assert int(want.status.item()) == 0
+        ata.forward(x, idx, w, rs, check_status=True)
+        ata.dispatch(x, idx, rs)
+
+
 def test_custom_kernel_check_status_and_config_changed_in_place(gpu_device):
     """`custom_kernel(data, check_status=True)` raises on an id the reference would fail on; a config
     object changed in place between two calls gets the instance of its new values."""
