@@ -357,6 +357,42 @@ def test_few_rows(gpu_device, dtype, m, W, n, kl):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 37, 64])
+@pytest.mark.parametrize("W,n,kl,at", [
+    (8, 8200, 680, 0), (8, 8190, 712, 3),  # rows that start a line every eighth time; operands that start 48 bytes into one
+    (8, 8200, 736, 4), (3, 32744, 456, 1),  # on half lines; groups that do not divide the dies
+    (1, 32760, 1352, 5), (2, 32766, 696, 0),  # one group; an odd number of results in the last tile
+    (8, 7176, 2056, 7),  # more weights than stay in the memory-side cache
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_few_rows_by_whole_lines(gpu_device, dtype, m, W, n, kl, at):
+    """Rows off the grid of cache lines and more than 84 MiB of weights: chunks that lag a request behind, at the shards' first and
+    last slabs, with an infinite element in either operand's last column.  Shards 24 and 40 elements apart whose gaps hold NaN.
+    f32 sums of W kl products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 result and 1e-5."""
+    lib, gaps = _lib.load(), (24, 40)
+    flat, parts = [], []
+    for rows, gap, seed in ((m, gaps[0], 1), (n, gaps[1], 2)):
+        t = torch.full((8 * at + W * (rows * kl + gap),), float("nan"), dtype=dtype, device=gpu_device)
+        part = t[8 * at:].view(W, rows * kl + gap)[:, :rows * kl].unflatten(1, (rows, kl))
+        part.copy_(uniform((W, rows, kl), dtype, gpu_device, seed + kl))
+        flat.append(t)
+        parts.append(part)
+    x, w = parts
+    x[W - 1, m - 1, kl - 1] = float("inf")
+    w[0, n - 1, kl - 1] = float("-inf")
+    w[W - 1, 5, 0] = float("inf")
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
+    ws = torch.empty(max(16, lib.gemm_rs_workspace_bytes(m, n, kl * W, W)), dtype=torch.uint8, device=gpu_device)
+    assert lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, kl * W, W, m * kl + gaps[0], n * kl + gaps[1],
+                               _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(),
+                               torch.cuda.current_stream().cuda_stream) == 0
+    want = product(x, w)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
+    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("form,W,m", [(0, 4, 64), (0, 1, 5), (256, 4, 392), (129, 4, 392), (131, 4, 392), (132, 4, 392),
                                       (130, 4, 392), (128, 4, 392), (32, 4, 392)])
 @pytest.mark.parametrize("kl", [72, 352, 360, 456])
