@@ -991,7 +991,7 @@ def gemm_rs_leg(args, lib, torch, dev):
         kernel = max(per, key=lambda kk: statistics.fmean(per[kk]))
         flops = 2.0 * m * n * k
         tflops = flops / t_us / 1e6
-        ws = int(lib.gemm_rs_workspace_bytes(m, n, k, W))
+        ws = int(lib.gemm_rs_workspace_used(m, n, k, W))
         line = dict(metric=f"GEMM + reduce-scatter TFLOP/s, 8 K-shards on one GPU, m{m} n{n} k{k}", value=round(tflops, 1),
                     unit="TFLOP/s", n_gpus=1, steps=args.steps, warmup=args.warmup, ms_per_step=round(ms_step, 5),
                     higher_is_better=True, scaling="weak", vs_baseline=None, dtype="bf16", data="synthetic",

@@ -43,10 +43,9 @@ extern "C" {
  *             - groups where they pay although the tiles fill most of the chip (160 or more of 256 x 128):
  *               OPTIONAL -- with NULL or too few bytes all shards are summed by one workgroup per tile, up
  *               to a fifth slower;
- *             - large outputs whose local K is not a multiple of 32 (rows that start off the
- *               128-byte line grid) are first copied onto zero-padded, aligned rows where that pays:
- *               OPTIONAL -- with NULL or too few bytes the product runs on the rows as they lie, up to
- *               a tenth slower;
+ *             - large outputs whose local K is not a multiple of 32 (rows that start off the 128-byte line
+ *               grid): the bytes of a padded copy of the operands, as ever, but nothing is put there and NULL
+ *               is as good (gemm_rs_workspace_used: the bytes without these);
  *             - 0 bytes for every other shape.
  *           The form, and with it the size, follows MOE_A2A_OPT_GEMM_TILE at the time of the call: a
  *           size queried under one setting belongs to that setting.
@@ -54,9 +53,11 @@ extern "C" {
  * 256 x 128 tiles (131 / 132: with 192 / 128 of a tile's rows in use, as the library chooses by itself
  * when that fills the CUs better), 130 those with one partial product per shard, 133 the 256 x 256 tiles with
  * one partial product per shard, 128 the 128 x 128
- * tiles, 32 those with one partial product per shard.  All unsplit forms give identical bits.
+ * tiles, 32 those with one partial product per shard.  All unsplit forms give identical bits, except that the
+ * 256 x 256 tiles sum in another order where the local K is not a multiple of 64.
  */
 size_t gemm_rs_workspace_bytes(int M, int N, int K, int W);
+size_t gemm_rs_workspace_used(int M, int N, int K, int W);
 int gemm_rs_forward(const void* input, const void* weight, const void* bias, void* out, int M, int N, int K, int W,
                     long long input_shard_stride, long long weight_shard_stride, int elem_type, void* workspace,
                     size_t workspace_bytes, moe_a2a_stream_t stream);

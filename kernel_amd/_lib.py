@@ -76,6 +76,7 @@ PROTOTYPES["moe_a2a_dispatch_once"] = (_int, [C.POINTER(ForwardArgs)])
 # include/gemm_rs.h (same library)
 GEMM_RS_PROTOTYPES = {
     "gemm_rs_workspace_bytes": (C.c_size_t, [_int, _int, _int, _int]),
+    "gemm_rs_workspace_used": (C.c_size_t, [_int, _int, _int, _int]),
     "gemm_rs_forward": (_int, [_vp, _vp, _vp, _vp, _int, _int, _int, _int, C.c_longlong, C.c_longlong, _int, _vp,
                                C.c_size_t, _vp]),
 }

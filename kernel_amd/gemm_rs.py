@@ -81,15 +81,15 @@ class HipGemmReduceScatter:
 
     def __init__(self, world_size: int, pad_ragged: bool = True):
         self.world_size = int(world_size)
-        # False: a shape whose workspace is optional (ragged shards on 256 x 256 tiles, which run faster on
-        # a zero-padded, line-aligned copy of the operands) is multiplied in place, without it
+        # False: a shape whose workspace is optional (partial products of groups of shards, where they only pay) is
+        # multiplied without it
         self.pad_ragged = bool(pad_ragged)
         self.lib = _lib.load()
         self._workspaces = {}  # (device, stream) -> workspace of the calls on that stream
         self._making = threading.Lock()
 
     def workspace_for(self, m: int, n: int, k: int, device) -> Optional[torch.Tensor]:
-        need = int(self.lib.gemm_rs_workspace_bytes(m, n, k, self.world_size))
+        need = int(self.lib.gemm_rs_workspace_used(m, n, k, self.world_size))
         if need == 0:
             return None
         if torch.cuda.is_current_stream_capturing():  # the graph's own: it may outlive this object and run beside other calls

@@ -538,6 +538,44 @@ def test_wide_tiles_with_the_shards_in_groups(gpu_device, options, dtype, W, m, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form,W,m,n,kl,at", [
+    (256, 8, 2056, 264, 712, 0), (256, 3, 1030, 520, 728, 3), (256, 2, 520, 260, 1000, 5),  # rows alike eight, four apart, too few
+    (256, 1, 300, 256, 904, 7), (256, 2, 4104, 72, 720, 1), (256, 4, 1291, 40, 744, 2),  # one shard; half lines; classes of unequal length
+    (133, 8, 1030, 264, 72, 3), (133, 2, 1040, 260, 136, 5), (133, 4, 530, 520, 200, 6), (133, 2, 257, 256, 264, 1),  # two slabs, three, four, five
+    (129, 4, 520, 264, 136, 3), (131, 3, 400, 264, 200, 6), (132, 2, 264, 520, 72, 1), (130, 4, 300, 264, 456, 7),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_tiles_by_whole_lines(gpu_device, options, dtype, form, W, m, n, kl, at):
+    """Rows off the grid of cache lines on the tiles of eight waves: chunks that lag a request behind, at the first and last slabs of
+    shards and past the last one, rows of x that lie alike dealt to the same tile, with an infinite element in either operand's last column
+    and its first.  Operands that start 16 `at` bytes into a line, and shards 24 and 40 elements apart whose gaps hold NaN.  f32 sums
+    of W kl products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 result and 1e-5."""
+    lib, gaps = _lib.load(), (24, 40)
+    options.set("GEMM_TILE", form)
+    flat, parts = [], []
+    for rows, gap, seed in ((m, gaps[0], 1), (n, gaps[1], 2)):
+        t = torch.full((8 * at + W * (rows * kl + gap),), float("nan"), dtype=dtype, device=gpu_device)
+        part = t[8 * at:].view(W, rows * kl + gap)[:, :rows * kl].unflatten(1, (rows, kl))
+        part.copy_(uniform((W, rows, kl), dtype, gpu_device, seed + kl))
+        flat.append(t)
+        parts.append(part)
+    x, w = parts
+    x[W - 1, m - 1, kl - 1] = float("inf")
+    x[0, m // 2, 0] = float("-inf")
+    w[0, n - 1, kl - 1] = float("-inf")
+    w[W - 1, 5, 0] = float("inf")
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
+    ws = torch.empty(max(16, lib.gemm_rs_workspace_bytes(m, n, kl * W, W)), dtype=torch.uint8, device=gpu_device)
+    assert lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, kl * W, W, m * kl + gaps[0], n * kl + gaps[1],
+                               _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(),
+                               torch.cuda.current_stream().cuda_stream) == 0
+    want = product(x, w)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
+    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("W,m,n,k,groups,narrow", [(8, 512, 5440, 17024, 4, "groups"), (8, 240, 4480, 24128, 8, "groups"),
                                                    (8, 1096, 6400, 6464, 2, "whole"), (4, 304, 5696, 11328, 4, "groups"),
                                                    (8, 120, 4160, 11008, 8, "groups")])
