@@ -37,9 +37,9 @@ extern "C" {
  *             - outputs of few tiles spread the shards over groups of workgroups, one f32 partial
  *               product per group (what each rank holds before the reduce-scatter), which a second
  *               launch sums: REQUIRED, MOE_A2A_E_WORKSPACE if missing or too small;
- *             - some hundreds of rows and a long K, most of all a local K that is not a multiple of 64: groups on 256 x 256
- *               tiles.  OPTIONAL in so far as with NULL, too few bytes or a pointer off its alignment the call goes on
- *               as if this form did not exist (and may then be one of the first kind);
+ *             - other groups than those, or groups on 256 x 256 tiles, where these are faster by estimate: OPTIONAL in so
+ *               far as with NULL, too few bytes or a pointer off its alignment the call goes on as if only the
+ *               first kind existed (and may then be one of it);
  *             - groups where they pay although the tiles fill most of the chip (160 or more of 256 x 128):
  *               OPTIONAL -- with NULL or too few bytes all shards are summed by one workgroup per tile, up
  *               to a fifth slower;
