@@ -12,6 +12,7 @@ one bf16 rounding: |out - exact| <= 2^-8 |exact| + 1e-6 (2^-9 is half a unit in 
 f32 accumulation adds less than 2^-15 relative over these K).
 """
 import ctypes
+import random
 import glob
 import os
 import re
@@ -266,6 +267,20 @@ def test_every_tile_of_odd_tile_counts(gpu_device, options, form, m, n):
     want = x.transpose(0, 1).reshape(m, W * kl).float() @ w.transpose(0, 1).reshape(n, W * kl).float().T
     torch.cuda.synchronize()
     assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6).all())
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="its operands do not exist: no call may reach a GPU")
+@pytest.mark.parametrize("W", [2, 8])
+def test_the_room_that_is_asked_for_is_enough(W):
+    """No shape is refused with the room that gemm_rs_workspace_used or _bytes tells, none among it (such a shape was, where a plan of
+    one group took the place of one that had to have room)."""
+    lib, rng = _lib.load(), random.Random(W)
+    for i in range(1500):
+        m, n = 8 * int(2 ** rng.uniform(0, 10)), 4 * int(2 ** rng.uniform(6, 11.5))
+        k = W * 8 * int(2 ** rng.uniform(3, 9))
+        for need in (lib.gemm_rs_workspace_used(m, n, k, W), lib.gemm_rs_workspace_bytes(m, n, k, W)):
+            rc = lib.gemm_rs_forward(4096, 4096, None, 4096, m, n, k, W, 0, 0, _lib.BF16, 4096 if need else None, need, None)
+            assert rc != E_WORKSPACE, (m, n, k)
 
 
 def launched(lib, call):
