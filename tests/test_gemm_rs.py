@@ -674,3 +674,18 @@ def test_workspace_of_a_stream_and_of_a_graph(gpu_device):
         torch.cuda.synchronize()
         assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
         assert all(bool((o == 7).all()) for o in other)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kl", [64, 200, 576, 776])  # whole slabs; rows as they lie; whole slabs; whole lines
+@pytest.mark.parametrize("m,n", [(2818, 3300), (1500, 7170), (7248, 2304), (868, 8400), (2304, 3700)])
+def test_wide_tiles_of_fewer_rows(gpu_device, m, n, kl):
+    """Outputs of more than 128 tiles of 256 x 256 that tiles with 192 or 128 of their rows in use cover in as many rounds of the CUs:
+    every row and column, a tile's last and the last tile's, with a bias.
+    f32 sums of 8 kl products of up to 0.05^2, rounded once: within 2^-8 of the f32 result and 2e-5."""
+    x, w = uniform((8, m, kl), torch.bfloat16, gpu_device, m + kl), uniform((8, n, kl), torch.bfloat16, gpu_device, n)
+    bias = uniform((n,), torch.bfloat16, gpu_device, 3)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    G.HipGemmReduceScatter(8).forward(x, w, bias, out=out)
+    want = product(x, w, bias)
+    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
