@@ -591,6 +591,23 @@ def test_tiles_by_whole_lines(gpu_device, options, dtype, form, W, m, n, kl, at)
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form,W,m,n,kl", [
+    (0, 8, 128, 1, 360), (0, 2, 65, 1, 72), (0, 8, 1, 32776, 720), (0, 1, 1, 33000, 712),
+    (256, 8, 1, 300, 712), (256, 8, 300, 1, 712), (256, 1, 1, 1, 776), (129, 8, 1, 300, 72), (129, 2, 300, 1, 104), (131, 3, 1, 200, 360),
+    (131, 8, 200, 1, 200), (132, 8, 1, 140, 456), (132, 1, 70, 1, 80), (130, 8, 1, 140, 72), (133, 8, 1, 300, 712), (133, 2, 1, 4, 136),
+])
+def test_operands_of_one_row(gpu_device, options, form, W, m, n, kl):
+    """Rows off the grid of cache lines whose shards begin less than a line behind the last one's end (test_tile_loop_addresses.py: every
+    request inside the operands).  f32 sums of W kl products of up to 0.05^2, rounded once: within 2^-8 of the f32 result and 1e-5."""
+    options.set("GEMM_TILE", form)
+    x, w, bias = (uniform(s, torch.bfloat16, gpu_device, m + n + i) for i, s in enumerate(((W, m, kl), (W, n, kl), (n,))))
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    G.HipGemmReduceScatter(W).forward(x, w, bias, out=out)
+    want = product(x, w, bias)
+    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-5).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("W,m,n,k,groups,narrow", [(8, 512, 5440, 17024, 4, "groups"), (8, 240, 4480, 24128, 8, "groups"),
                                                    (8, 1096, 6400, 6464, 2, "whole"), (4, 304, 5696, 11328, 4, "groups"),
                                                    (8, 120, 4160, 11008, 8, "groups")])
