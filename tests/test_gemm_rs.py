@@ -25,6 +25,8 @@ from kernel_amd import _lib
 from kernel_amd import gemm_rs as G
 from oracle import gemm_rs as O
 
+import tile_loops
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "gemm_rs.h")
 GOLDEN = sorted(glob.glob(os.path.join(ROOT, "tests", "golden", "gemm_rs_*.npz")))
@@ -281,6 +283,22 @@ def test_the_room_that_is_asked_for_is_enough(W):
         for need in (lib.gemm_rs_workspace_used(m, n, k, W), lib.gemm_rs_workspace_bytes(m, n, k, W)):
             rc = lib.gemm_rs_forward(4096, 4096, None, 4096, m, n, k, W, 0, 0, _lib.BF16, 4096 if need else None, need, None)
             assert rc != E_WORKSPACE, (m, n, k)
+
+
+ROOM_OF_EARLIER = [  # W, m, n, kl, bytes, kernels: what gemm_rs_workspace_bytes has told of for these, and is enough for them
+    (16, 153, 10936, 2304, 4 * 153 * 10936 * 4, "split reduce"), (8, 1976, 2304, 3216, 2 * 1976 * 2304 * 4, "split reduce"),
+    (8, 1162, 3836, 3720, 2 * 1162 * 3836 * 4, "split reduce"), (8, 35928, 4, 392, 0, "narrow"), (8, 36053, 4, 4960, 0, "narrow"),
+]
+
+
+@pytest.mark.parametrize("W,m,n,kl,room,kernels", ROOM_OF_EARLIER)
+def test_room_that_was_enough_is(W, m, n, kl, room, kernels):
+    """Calls with less room than the form that is chosen now asks for: answered with as much as they were, and with the first byte of
+    it missing, or off its alignment, refused."""
+    call = lambda size, at=0: tile_loops.run([("call", 0, 0, m, n, kl, W, 0, 0, 0, 0, size, at)])[0][:-2]
+    assert call(room) == ["0", *kernels.split()]
+    if room:
+        assert call(room - 1) == call(room, 8) == call(0) == [str(E_WORKSPACE)]  # (less than the others have to have)
 
 
 def launched(lib, call):
@@ -642,6 +660,21 @@ def test_room_for_the_groups_is_optional(gpu_device, options, W, m, n, k, groups
         options.set("GEMM_TILE", 129)
         got.append(call(None, 0))
         assert all(how == [0, "gemm_rs_narrow"] and torch.equal(out, got[0][1]) for how, out in got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,m,n,kl,room,kernels", ROOM_OF_EARLIER)
+def test_results_with_room_that_was_enough(gpu_device, W, m, n, kl, room, kernels):
+    """f32 sums of W kl products of up to 0.05^2, rounded once: within 2^-8 of the f32 result and 2e-5."""
+    lib = _lib.load()
+    x, w = uniform((W, m, kl), torch.bfloat16, gpu_device, m), uniform((W, n, kl), torch.bfloat16, gpu_device, n)
+    out, ws = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device), torch.empty(max(room, 16), dtype=torch.uint8, device=gpu_device)
+    rc = []
+    names = launched(lib, lambda: rc.append(lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, W * kl, W, 0, 0, _lib.BF16,
+                                                                ws.data_ptr() if room else None, room, torch.cuda.current_stream().cuda_stream)))
+    assert rc == [0] and names == ["gemm_rs_" + k for k in kernels.split()]
+    want = product(x, w)
+    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
 
 
 @pytest.mark.gpu

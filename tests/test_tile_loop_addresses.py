@@ -1,46 +1,13 @@
 """Where the tile loops of gemm_rs read: on the CPU, from the kernels' own sources.
 
 The loops are cut out of ``kernel_amd/csrc``, compiled for the host with stand-ins for the matrix and buffer instructions
-(``tile_loop_walk.cpp``), and run thread by thread.  Every request inside a buffer has to lie in a row of an operand, and all rows have
+(``tile_loops.py``), and run thread by thread.  Every request inside a buffer has to lie in a row of an operand, and all rows have
 to be asked for.  No GPU, and nothing is read from the addresses."""
-import os
 import random
-import re
-import shutil
-import subprocess
 
 import pytest
 
-HERE = os.path.dirname(os.path.abspath(__file__))
-CSRC = os.path.join(os.path.dirname(HERE), "kernel_amd", "csrc")
-
-
-def between(text, first, last):
-    """From the line that starts with `first` up to the one that starts with `last`."""
-    begin = re.search("^" + re.escape(first), text, re.M).start()
-    return text[begin:begin + re.search("^" + re.escape(last), text[begin:], re.M).start()]
-
-
-@pytest.fixture(scope="module")
-def walk(tmp_path_factory):
-    clang = shutil.which("amdclang++") or shutil.which("clang++") or "/opt/rocm/llvm/bin/clang++"
-    if not os.path.exists(clang):
-        pytest.skip("no clang (the kernels' vector types are its own)")
-    to = tmp_path_factory.mktemp("walk")
-    g8, rs = (open(os.path.join(CSRC, name)).read() for name in ("gemm8_kernels.inc", "gemm_rs_kernels.inc"))
-    loops = between(g8, "constexpr int kG8Threads", "// fp8 x fp8") + between(g8, "constexpr int kG8GroupN", "constexpr int kG8GroupM")
-    loops = re.sub(r"\basm( volatile)?\s*\((?:[^()]|\([^()]*\))*\);", ";", loops + rs)  # (constraints of the GPU's registers)
-    (to / "loops.inc").write_text(loops)
-    subprocess.run([clang, "-x", "c++", "-std=c++17", "-O1", "-w", "-ffp-contract=off", "-I", str(to),
-                    os.path.join(HERE, "tile_loop_walk.cpp"), "-o", str(to / "walk")], check=True)
-
-    def run(launches):
-        lines = "".join(" ".join(map(str, l)) + "\n" for l in launches)
-        got = subprocess.run([str(to / "walk")], input=lines, capture_output=True, text=True, check=True).stdout.splitlines()
-        assert len(got) == len(launches)
-        return [tuple(map(int, line.split())) for line in got]
-
-    return run
+import tile_loops
 
 
 def launch(form, m, n, kl, W, groups, pitch, cols, at=(0, 0), gap=(0, 0)):
@@ -64,8 +31,9 @@ def launches(ms, ns, kls, rng):
                         yield launch("s", m, n, kl, W, W, rng.choice((256, 208, 16)), rng.choice((256, 176, 64)), at, gap)
 
 
-def check(walk, cases):
-    for case, (requests, outside, missed) in zip(cases, walk(cases)):
+def check(cases):
+    for case, got in zip(cases, tile_loops.run(cases)):
+        requests, outside, missed = map(int, got)
         assert outside == 0 and missed == 0 and requests > 0, (case, requests, outside, missed)
 
 
@@ -73,25 +41,25 @@ KLS = (64, 72, 80, 96, 104, 128, 136, 184, 192, 200, 264, 312, 360, 456, 712, 72
 
 
 @pytest.mark.parametrize("m,n", [(1, 1), (1, 300), (65, 1), (1, 40), (130, 2), (2, 130)])
-def test_operands_of_one_row_or_two(walk, m, n):
+def test_operands_of_one_row_or_two(m, n):
     """Shards one row apart begin less than a line behind the last one's end: what takes a request there is a step backwards, also
     for the rows that do not exist."""
-    check(walk, list(launches([m], [n], KLS, random.Random(m + n))))
+    check(list(launches([m], [n], KLS, random.Random(m + n))))
 
 
 @pytest.mark.parametrize("seed", range(4))
-def test_any_operands(walk, seed):
+def test_any_operands(seed):
     rng = random.Random(seed)
     size = lambda most: int(2 ** rng.uniform(0, most))
     cases = []
     for _ in range(12):
         cases += launches([size(9.2)], [size(9.2)], [8 * rng.randrange(8, 100)], rng)
-    check(walk, cases)
+    check(cases)
 
 
 @pytest.mark.parametrize("m,n,kl,W,form,pitch,cols", [
     (128, 1, 360, 8, "n", 128, 128), (65, 1, 72, 2, "n", 128, 128), (520, 1, 360, 8, "n", 256, 128),
     (1, 32776, 720, 8, "wl", 256, 256), (1, 33000, 712, 1, "wl", 256, 256),
 ])
-def test_operands_of_one_row_as_the_library_multiplies_them(walk, m, n, kl, W, form, pitch, cols):
-    check(walk, [launch(form, m, n, kl, W, 1, pitch, cols)])
+def test_operands_of_one_row_as_the_library_multiplies_them(m, n, kl, W, form, pitch, cols):
+    check([launch(form, m, n, kl, W, 1, pitch, cols)])

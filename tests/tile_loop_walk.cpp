@@ -1,17 +1,25 @@
-// The tile loops of gemm_rs, compiled for the host: every request that a workgroup's threads make is looked at instead of made.
-// loops.inc is cut from the kernels' sources by test_tile_loop_addresses.py, which builds and runs this.  Threads run one after
-// the other, so what they read from the LDS means nothing; the addresses they ask for do not depend on it.
+// The tile loops of gemm_rs and their entry point, compiled for the host: every request that a workgroup's threads make is looked at
+// instead of made.  loops.inc and entry.inc are cut from the kernels' sources by tile_loops.py, which builds and runs this.  Threads
+// run one after the other, so what they read from the LDS means nothing; the addresses they ask for do not depend on it.
 //
-// Standard input: one launch a line,
+// Standard input: a launch a line,
 //   form M N Kl W groups pitch cols a_at b_at a_gap b_gap     (gaps in 16-byte vectors, at: the operands' own, modulo a line)
-// Standard output: for each the requests inside the buffers, those of them outside the operands' rows, and the 16-byte vectors of the
-// operands' rows that a workgroup has to have and did not ask for.
+// or a call of gemm_rs_forward (bytes of workspace, which begins `ws_at` bytes behind a 16-byte boundary; 0 bytes: none),
+//   call walk option M N Kl W a_at b_at a_gap b_gap bytes ws_at
+// Standard output: of a launch, and of a call's whose launches are to be walked, the requests inside the buffers, those of them outside
+// the operands' rows, and the 16-byte vectors of the operands' rows that nothing asked for; of a call before that the status and
+// the kernels, and of any call the bytes that gemm_rs_workspace_used and _bytes answer at the end.
 #include <stddef.h>
 #include <stdint.h>
 #include <stdio.h>
 
 #include <algorithm>
+#include <cmath>
+#include <string>
 #include <vector>
+
+#include "gemm_rs.h"
+#include "moe_a2a.h"
 
 #define __device__
 #define __host__
@@ -21,7 +29,12 @@
 #define __launch_bounds__(...)
 #define __align__(N) __attribute__((aligned(N)))
 #define __syncthreads()
-struct Dim { unsigned x, y; };
+struct dim3 {
+  unsigned x, y;
+  dim3(unsigned x = 1, unsigned y = 1) : x(x), y(y) {}
+};
+typedef dim3 Dim;
+typedef void* hipStream_t;
 static Dim threadIdx, blockIdx, blockDim, gridDim;
 struct uint2 { uint32_t x, y; };
 struct uint4 { uint32_t x, y, z, w; };
@@ -41,6 +54,7 @@ struct Bf16 {
   static float hi(uint32_t) { return 0; }
   static uint32_t pack(float, float) { return 0; }
 };
+struct F16 : Bf16 {};
 template <class E> f32x4_t mfma_16x16x32(const u32x4_t&, const u32x4_t&, const f32x4_t& c) { return c; }
 template <class E> f32x16_t mfma_32x32x16(const uint4&, const uint4&, const f32x16_t& c) { return c; }
 template <class E> void store4(uint16_t*, const f32x4_t&) {}
@@ -98,14 +112,62 @@ static void walk(F kernel, Dim grid, int threads) {
       for (threadIdx.x = 0; threadIdx.x < (unsigned)threads; ++threadIdx.x) kernel();
 }
 
+static void place(int M, int N, int Kl, int W, int a_at, int b_at, long long a_gap, long long b_gap, bool walked) {
+  const int kvec = Kl / 8;
+  op_a = {(1ull << 44) + 16 * a_at, (long long)M * kvec + a_gap, M, kvec, W, std::vector<uint8_t>(walked ? (size_t)W * M * kvec : 0)};
+  op_b = {(1ull << 45) + 16 * b_at, (long long)N * kvec + b_gap, N, kvec, W, std::vector<uint8_t>(walked ? (size_t)W * N * kvec : 0)};
+  requests = outside = 0;
+}
+static void report() {
+  long long missed = 0;
+  for (const Operand* o : {&op_a, &op_b}) missed += std::count(o->asked.begin(), o->asked.end(), 0);
+  printf("%lld %lld %lld", requests, outside, missed);
+}
+
+// What the entry point is made of besides.
+enum { KID_GEMM_RS_WIDE, KID_GEMM_RS_TILE, KID_GEMM_RS_REDUCE, KID_GEMM_RS_NARROW, KID_GEMM_RS_SPLIT };
+static const char* const kNames[] = {"wide", "tile", "reduce", "narrow", "split"};
+static int forced;
+static int option(int) { return forced; }
+static bool aligned16(const void* p) { return (uintptr_t)p % 16 == 0; }
+static int ceil_div(int a, int b) { return (a + b - 1) / b; }
+static std::string launched;
+static bool walked;
+template <class T> struct same_type { typedef T type; };
+template <class... A>
+static int launch(int kid, void (*kernel)(A...), Dim grid, Dim block, size_t, hipStream_t, typename same_type<A>::type... args) {
+  launched += std::string(" ") + kNames[kid];
+  if (walked && kid != KID_GEMM_RS_REDUCE && kernel != (void (*)(A...))nullptr) walk([&] { kernel(args...); }, grid, (int)block.x);
+  return 0;
+}
+#include "entry.inc"
+
+static void call() {
+  int walk_it, M, N, Kl, W, a_at, b_at, ws_at;
+  long long a_gap, b_gap, bytes;
+  if (scanf("%d %d %d %d %d %d %d %d %lld %lld %lld %d", &walk_it, &forced, &M, &N, &Kl, &W, &a_at, &b_at, &a_gap, &b_gap, &bytes, &ws_at) != 12) return;
+  walked = walk_it != 0;
+  place(M, N, Kl, W, a_at, b_at, a_gap, b_gap, walked);
+  launched.clear();
+  std::vector<uint4> out(walked ? (size_t)M * N / 8 + 1 : 1), room(walked ? bytes / 16 + 2 : 2);
+  const int rc = gemm_rs_forward((const void*)op_a.at, (const void*)op_b.at, nullptr, out.data(), M, N, Kl * W, W, op_a.shard * 8, op_b.shard * 8,
+                                 MOE_A2A_BF16, bytes ? (char*)room.data() + ws_at : nullptr, (size_t)bytes, nullptr);
+  printf("%d%s ", rc, launched.c_str());
+  if (walked) report();
+  printf(" %zu %zu\n", gemm_rs_workspace_used(M, N, Kl * W, W), gemm_rs_workspace_bytes(M, N, Kl * W, W));
+}
+
 int main() {
   char form[16];
-  int M, N, Kl, W, groups, pitch, cols, a_at, b_at, a_gap, b_gap;
-  while (scanf("%15s %d %d %d %d %d %d %d %d %d %d %d", form, &M, &N, &Kl, &W, &groups, &pitch, &cols, &a_at, &b_at, &a_gap, &b_gap) == 12) {
-    const int kvec = Kl / 8;
-    op_a = {(1ull << 44) + 16 * a_at, (long long)M * kvec + a_gap, M, kvec, W, std::vector<uint8_t>((size_t)W * M * kvec)};
-    op_b = {(1ull << 45) + 16 * b_at, (long long)N * kvec + b_gap, N, kvec, W, std::vector<uint8_t>((size_t)W * N * kvec)};
-    requests = outside = 0;
+  while (scanf("%15s", form) == 1) {
+    if (form[0] == 'c') {
+      call();
+      continue;
+    }
+    int M, N, Kl, W, groups, pitch, cols, a_at, b_at;
+    long long a_gap, b_gap;
+    if (scanf("%d %d %d %d %d %d %d %d %d %lld %lld", &M, &N, &Kl, &W, &groups, &pitch, &cols, &a_at, &b_at, &a_gap, &b_gap) != 11) return 1;
+    place(M, N, Kl, W, a_at, b_at, a_gap, b_gap, true);
     GemmRsArgs g{(const uint4*)op_a.at, (const uint4*)op_b.at, nullptr, M, N, Kl, W, op_a.shard, op_b.shard, (float)W, W / groups};
     std::vector<uint16_t> out((size_t)M * N);
     std::vector<float> partial((size_t)groups * M * N);
@@ -140,10 +202,8 @@ int main() {
         if (cols == 128) groups > 1 ? ROWS_K(128, true) : ROWS_K(128, false);
         else groups > 1 ? ROWS_K(64, true) : ROWS_K(64, false);
     }
-    long long missed = 0;
-    for (const Operand* o : {&op_a, &op_b}) missed += std::count(o->asked.begin(), o->asked.end(), 0);
-    printf("%lld %lld %lld\n", requests, outside, missed);
-    fflush(stdout);
+    report();
+    printf("\n");
   }
   return 0;
 }
