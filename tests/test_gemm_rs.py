@@ -548,6 +548,34 @@ def uniform(shape, dtype, dev, seed):
     return torch.empty(*shape, dtype=dtype, device=dev).uniform_(-0.05, 0.05, generator=g)
 
 
+def check_off_the_line_grid(dev, dtype, W, m, n, kl, at):
+    """The product of shards whose rows lie off the grid of cache lines, with an infinite element in either operand's last column and its
+    first.  Operands that start 16 `at` bytes into a line, and shards 24 and 40 elements apart whose gaps hold NaN.  f32 sums of W kl
+    products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 result and 1e-5."""
+    lib, gaps = _lib.load(), (24, 40)
+    flat, parts = [], []
+    for rows, gap, seed in ((m, gaps[0], 1), (n, gaps[1], 2)):
+        t = torch.full((8 * at + W * (rows * kl + gap),), float("nan"), dtype=dtype, device=dev)
+        part = t[8 * at:].view(W, rows * kl + gap)[:, :rows * kl].unflatten(1, (rows, kl))
+        part.copy_(uniform((W, rows, kl), dtype, dev, seed + kl))
+        flat.append(t)
+        parts.append(part)
+    x, w = parts
+    x[W - 1, m - 1, kl - 1] = float("inf")
+    x[0, m // 2, 0] = float("-inf")
+    w[0, n - 1, kl - 1] = float("-inf")
+    w[W - 1, 5, 0] = float("inf")
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=dev)
+    ws = torch.empty(max(16, lib.gemm_rs_workspace_bytes(m, n, kl * W, W)), dtype=torch.uint8, device=dev)
+    assert lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, kl * W, W, m * kl + gaps[0], n * kl + gaps[1],
+                               _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(),
+                               torch.cuda.current_stream().cuda_stream) == 0
+    want = product(x, w)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
+    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("W,m,n,kl", [
     (2, 65, 8, 64), (2, 256, 256, 72), (8, 257, 260, 64), (4, 392, 600, 360), (8, 72, 4100, 96), (3, 520, 2052, 200),
@@ -574,44 +602,38 @@ def test_wide_tiles_with_the_shards_in_groups(gpu_device, options, dtype, W, m, 
 @pytest.mark.parametrize("form,W,m,n,kl,at", [
     (256, 8, 2056, 264, 712, 0), (256, 3, 1030, 520, 728, 3), (256, 2, 520, 260, 1000, 5),  # rows alike eight, four apart, too few
     (256, 1, 300, 256, 904, 7), (256, 2, 4104, 72, 720, 1), (256, 4, 1291, 40, 744, 2),  # one shard; half lines; classes of unequal length
-    (133, 8, 1030, 264, 72, 3), (133, 2, 1040, 260, 136, 5), (133, 4, 530, 520, 200, 6), (133, 2, 257, 256, 264, 1),  # two slabs, three, four, five
-    (129, 4, 520, 264, 136, 3), (131, 3, 400, 264, 200, 6), (132, 2, 264, 520, 72, 1), (130, 4, 300, 264, 456, 7),
+    (256, 2, 6160, 6144, 72, 3), (256, 1, 6144, 6152, 136, 5), (256, 2, 6150, 6144, 200, 6), (256, 1, 6152, 6144, 264, 1),  # two slabs, three, four, five
+    (133, 8, 2060, 1032, 72, 3), (133, 8, 2060, 1032, 136, 5), (133, 4, 4120, 1032, 200, 6), (133, 8, 2060, 1032, 264, 1),
+    (133, 8, 1030, 264, 584, 3), (133, 2, 1040, 260, 648, 5), (133, 4, 530, 520, 712, 6), (133, 2, 257, 256, 776, 1),
+    (129, 4, 520, 264, 776, 3), (131, 3, 400, 264, 200, 6), (132, 2, 264, 520, 72, 1), (130, 4, 300, 264, 456, 7),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 def test_tiles_by_whole_lines(gpu_device, options, dtype, form, W, m, n, kl, at):
     """Rows off the grid of cache lines on the tiles of eight waves: chunks that lag a request behind, at the first and last slabs of
-    shards and past the last one, rows of x that lie alike dealt to the same tile, with an infinite element in either operand's last column
-    and its first.  Operands that start 16 `at` bytes into a line, and shards 24 and 40 elements apart whose gaps hold NaN.  f32 sums
-    of W kl products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 result and 1e-5."""
-    lib, gaps = _lib.load(), (24, 40)
+    shards and past the last one, rows of x that lie alike dealt to the same tile (check_off_the_line_grid)."""
     options.set("GEMM_TILE", form)
-    flat, parts = [], []
-    for rows, gap, seed in ((m, gaps[0], 1), (n, gaps[1], 2)):
-        t = torch.full((8 * at + W * (rows * kl + gap),), float("nan"), dtype=dtype, device=gpu_device)
-        part = t[8 * at:].view(W, rows * kl + gap)[:, :rows * kl].unflatten(1, (rows, kl))
-        part.copy_(uniform((W, rows, kl), dtype, gpu_device, seed + kl))
-        flat.append(t)
-        parts.append(part)
-    x, w = parts
-    x[W - 1, m - 1, kl - 1] = float("inf")
-    x[0, m // 2, 0] = float("-inf")
-    w[0, n - 1, kl - 1] = float("-inf")
-    w[W - 1, 5, 0] = float("inf")
-    out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
-    ws = torch.empty(max(16, lib.gemm_rs_workspace_bytes(m, n, kl * W, W)), dtype=torch.uint8, device=gpu_device)
-    assert lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, kl * W, W, m * kl + gaps[0], n * kl + gaps[1],
-                               _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(),
-                               torch.cuda.current_stream().cuda_stream) == 0
-    want = product(x, w)
-    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
-    ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
-    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
+    check_off_the_line_grid(gpu_device, dtype, W, m, n, kl, at)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,W,m,n,kl,at", [
+    (129, 2, 2304, 2570, 72, 3), (129, 3, 2312, 2440, 200, 5), (129, 1, 2305, 2432, 680, 1), (129, 8, 2296, 2561, 96, 4),
+    (133, 8, 1030, 264, 72, 3), (133, 2, 1040, 260, 136, 5), (133, 4, 530, 520, 200, 6), (133, 2, 257, 256, 264, 1), (129, 4, 520, 264, 136, 3),
+    (129, 2, 300, 200, 160, 2), (131, 4, 400, 264, 224, 4), (132, 3, 264, 520, 416, 0), (130, 8, 520, 264, 96, 6), (130, 2, 300, 132, 352, 5),  # half lines
+    (133, 8, 1030, 264, 96, 3), (133, 2, 257, 256, 672, 1), (133, 4, 530, 520, 736, 6), (133, 2, 1000, 264, 1184, 2),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_tiles_of_rows_as_they_lie(gpu_device, options, dtype, form, W, m, n, kl, at):
+    """Short shards off the grid of cache lines, which 256 x 128 tiles with all rows in use and 256 x 256 tiles in groups request as they lie,
+    and shards on half lines, where the other 256 x 128 tiles do (check_off_the_line_grid)."""
+    options.set("GEMM_TILE", form)
+    check_off_the_line_grid(gpu_device, dtype, W, m, n, kl, at)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("form,W,m,n,kl", [
     (0, 8, 128, 1, 360), (0, 2, 65, 1, 72), (0, 8, 1, 32776, 720), (0, 1, 1, 33000, 712),
-    (256, 8, 1, 300, 712), (256, 8, 300, 1, 712), (256, 1, 1, 1, 776), (129, 8, 1, 300, 72), (129, 2, 300, 1, 104), (131, 3, 1, 200, 360),
+    (256, 8, 1, 300, 712), (256, 8, 300, 1, 712), (256, 1, 1, 1, 776), (129, 8, 1, 300, 72), (129, 2, 300, 1, 104), (129, 8, 1, 300, 776), (129, 2, 300, 1, 712), (131, 3, 1, 200, 360),
     (131, 8, 200, 1, 200), (132, 8, 1, 140, 456), (132, 1, 70, 1, 80), (130, 8, 1, 140, 72), (133, 8, 1, 300, 712), (133, 2, 1, 4, 136),
 ])
 def test_operands_of_one_row(gpu_device, options, form, W, m, n, kl):

@@ -24,11 +24,11 @@ def launches(ms, ns, kls, rng):
                     for form in ("wl", "wr"):
                         yield launch(form, m, n, kl, W, 1, rng.choice((256, 192, 128)), 256, at, gap)
                     for groups in {1, W if n % 4 == 0 else 1}:  # (partial products are written four columns at a time)
-                        yield launch("n", m, n, kl, W, groups, rng.choice((256, 192, 128)), 128, at, gap)
+                        yield launch(rng.choice(("nl", "nr")), m, n, kl, W, groups, rng.choice((256, 192, 128)), 128, at, gap)
                         if m <= 64:
                             yield launch(rng.choice(("rl", "rr")), m, n, kl, W, groups, 64, rng.choice((64, 128)), at, gap)
                     if W > 1 and n % 4 == 0:
-                        yield launch("s", m, n, kl, W, W, rng.choice((256, 208, 16)), rng.choice((256, 176, 64)), at, gap)
+                        yield launch(rng.choice(("sl", "sr")), m, n, kl, W, W, rng.choice((256, 208, 16)), rng.choice((256, 176, 64)), at, gap)
 
 
 def check(cases):
@@ -57,9 +57,24 @@ def test_any_operands(seed):
     check(cases)
 
 
-@pytest.mark.parametrize("m,n,kl,W,form,pitch,cols", [
-    (128, 1, 360, 8, "n", 128, 128), (65, 1, 72, 2, "n", 128, 128), (520, 1, 360, 8, "n", 256, 128),
-    (1, 32776, 720, 8, "wl", 256, 256), (1, 33000, 712, 1, "wl", 256, 256),
-])
-def test_operands_of_one_row_as_the_library_multiplies_them(m, n, kl, W, form, pitch, cols):
-    check([launch(form, m, n, kl, W, 1, pitch, cols)])
+def check_calls(cases):
+    """(option, m, n, kl, W, at, gap) through gemm_rs_forward, with room for any partial products."""
+    lines = [("call", 1, option, m, n, kl, W, *at, *gap, 4 * W * m * n, 0) for option, m, n, kl, W, at, gap in cases]
+    for case, got in zip(cases, tile_loops.run(lines)):
+        requests, outside, missed = map(int, got[-5:-2])
+        assert got[0] == "0" and outside == 0 and missed == 0 and requests > 0, (case, got)
+
+
+@pytest.mark.parametrize("m,n,kl,W", [(128, 1, 360, 8), (65, 1, 72, 2), (520, 1, 360, 8), (520, 1, 776, 2), (1, 32776, 720, 8), (1, 33000, 712, 1)])
+def test_operands_of_one_row_as_the_library_multiplies_them(m, n, kl, W):
+    check_calls([(0, m, n, kl, W, (0, 0), (0, 0))])
+
+
+@pytest.mark.parametrize("seed", range(3))
+def test_calls_as_the_library_multiplies_them(seed):
+    rng, cases = random.Random(seed), []
+    while len(cases) < 24:
+        W, m, n, kl = rng.choice((1, 2, 3, 8)), int(2 ** rng.uniform(0, 11)), 4 * int(2 ** rng.uniform(0, 9)), 8 * rng.randrange(8, 70)
+        if W * (m + n) * kl <= 4 << 20:
+            cases.append((rng.choice((0, 0, 256, 129, 130, 131, 132, 133)), m, n, kl, W, (rng.randrange(8), rng.randrange(8)), (rng.choice((0, 3)), rng.choice((0, 6)))))
+    check_calls(cases)

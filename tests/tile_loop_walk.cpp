@@ -183,14 +183,16 @@ int main() {
         break;
       case 1: {
         const Dim grid{(unsigned)(8 * ((tm * tn * groups + 7) / 8)), 1};
-#define SPLIT(LINES) walk([&] { gemm_rs_split_kernel<Bf16, LINES>(g, partial.data(), tm, tn, groups, pitch, cols); }, grid, kG8Threads)
-        if (whole) SPLIT(false);
-        else SPLIT(true);
+#define SPLIT(ALONG) walk([&] { gemm_rs_split_kernel<Bf16, ALONG>(g, partial.data(), tm, tn, groups, pitch, cols); }, grid, kG8Threads)
+        if (whole) SPLIT(kG8Whole);
+        else if (form[1] == 'l') SPLIT(kG8Lines);
+        else SPLIT(kG8Ragged);
         break;
       }
       case 2:
-#define NARROW(P, LINES, SP) walk([&] { gemm_rs_narrow_kernel<Bf16, LINES, SP, P>(g, out.data(), partial.data(), tm, tn, groups, 1); }, Dim{eighths, y}, kG8Threads)
-#define NARROW_OF(P) (whole ? (groups > 1 ? NARROW(P, false, true) : NARROW(P, false, false)) : groups > 1 ? NARROW(P, true, true) : NARROW(P, true, false))
+#define NARROW(P, ALONG, SP) walk([&] { gemm_rs_narrow_kernel<Bf16, ALONG, SP, P>(g, out.data(), partial.data(), tm, tn, groups, 1); }, Dim{eighths, y}, kG8Threads)
+#define NARROW_A(P, SP) (whole ? NARROW(P, kG8Whole, SP) : form[1] == 'l' ? NARROW(P, kG8Lines, SP) : NARROW(P, kG8Ragged, SP))
+#define NARROW_OF(P) (groups > 1 ? NARROW_A(P, true) : NARROW_A(P, false))
         if (groups == 1) gridDim.y = 1;
         if (pitch == 256) NARROW_OF(256);
         else if (pitch == 192) NARROW_OF(192);
