@@ -548,11 +548,11 @@ def uniform(shape, dtype, dev, seed):
     return torch.empty(*shape, dtype=dtype, device=dev).uniform_(-0.05, 0.05, generator=g)
 
 
-def check_off_the_line_grid(dev, dtype, W, m, n, kl, at):
+def check_off_the_line_grid(dev, dtype, W, m, n, kl, at, gaps=(24, 40)):
     """The product of shards whose rows lie off the grid of cache lines, with an infinite element in either operand's last column and its
-    first.  Operands that start 16 `at` bytes into a line, and shards 24 and 40 elements apart whose gaps hold NaN.  f32 sums of W kl
-    products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 result and 1e-5."""
-    lib, gaps = _lib.load(), (24, 40)
+    first.  Operands that start 16 `at` bytes into a line, and shards so many elements apart whose gaps hold NaN.  f32 sums of W kl
+    products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 result and 1e-5.  The kernels that ran."""
+    lib = _lib.load()
     flat, parts = [], []
     for rows, gap, seed in ((m, gaps[0], 1), (n, gaps[1], 2)):
         t = torch.full((8 * at + W * (rows * kl + gap),), float("nan"), dtype=dtype, device=dev)
@@ -567,13 +567,16 @@ def check_off_the_line_grid(dev, dtype, W, m, n, kl, at):
     w[W - 1, 5, 0] = float("inf")
     out = torch.full((m, n), float("nan"), dtype=dtype, device=dev)
     ws = torch.empty(max(16, lib.gemm_rs_workspace_bytes(m, n, kl * W, W)), dtype=torch.uint8, device=dev)
-    assert lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, kl * W, W, m * kl + gaps[0], n * kl + gaps[1],
-                               _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(),
-                               torch.cuda.current_stream().cuda_stream) == 0
+    rc = []
+    kernels = launched(lib, lambda: rc.append(lib.gemm_rs_forward(
+        x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, kl * W, W, m * kl + gaps[0], n * kl + gaps[1],
+        _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)))
+    assert rc == [0]
     want = product(x, w)
     assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
     ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
     assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
+    return kernels
 
 
 @pytest.mark.gpu
@@ -628,6 +631,18 @@ def test_tiles_of_rows_as_they_lie(gpu_device, options, dtype, form, W, m, n, kl
     and shards on half lines, where the other 256 x 128 tiles do (check_off_the_line_grid)."""
     options.set("GEMM_TILE", form)
     check_off_the_line_grid(gpu_device, dtype, W, m, n, kl, at)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,m,n,kl,kernels", [
+    (256, 520, 264, 776, "wide"), (133, 520, 264, 776, "split reduce"), (129, 520, 264, 776, "narrow"), (131, 400, 264, 360, "narrow"),
+    (132, 300, 264, 200, "narrow"), (130, 300, 264, 456, "narrow reduce"), (0, 40, 8200, 2728, "tile reduce"),  # (more than 84 MiB of weights)
+])
+def test_shards_far_apart(gpu_device, options, form, m, n, kl, kernels):
+    """Two shards of either operand, more than a 32-bit offset apart (2 GiB): the same form as of shards that are near, and rows as they lie
+    (check_off_the_line_grid)."""
+    options.set("GEMM_TILE", form)
+    assert check_off_the_line_grid(gpu_device, torch.bfloat16, 2, m, n, kl, 3, ((1 << 30) + 24, (1 << 30) + 40)) == ["gemm_rs_" + k for k in kernels.split()]
 
 
 @pytest.mark.gpu

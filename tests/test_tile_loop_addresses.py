@@ -78,3 +78,14 @@ def test_calls_as_the_library_multiplies_them(seed):
         if W * (m + n) * kl <= 4 << 20:
             cases.append((rng.choice((0, 0, 256, 129, 130, 131, 132, 133)), m, n, kl, W, (rng.randrange(8), rng.randrange(8)), (rng.choice((0, 3)), rng.choice((0, 6)))))
     check_calls(cases)
+
+
+FAR = 1 << 27  # 16-byte vectors: 2 GiB
+
+
+@pytest.mark.parametrize("gap", [(FAR, FAR), (FAR, 0), (0, FAR), (FAR - 40000, 5), (FAR // 2, FAR - 70000)])
+@pytest.mark.parametrize("form,m,n,kl", [(256, 300, 264, 712), (129, 300, 264, 776), (131, 400, 264, 360), (132, 130, 264, 72), (130, 300, 132, 456),
+                                         (133, 300, 264, 712), (0, 37, 16, 712)])
+def test_shards_far_apart(form, m, n, kl, gap):
+    """Further than a 32-bit offset reaches, or just not."""
+    check_calls([(form, m, n, kl, W, (3, 5), gap) for W in (2, 7)])
