@@ -141,8 +141,9 @@ def test_host_side_argument_checks():
     assert call(M=64, N=7168, K=18432) == E_WORKSPACE
     assert call(M=64, N=7168, K=18432, ws=A, wsb=need - 1) == E_WORKSPACE
     assert lib.gemm_rs_workspace_bytes(8192, 4096, 14336, 8) == 0  # whole slabs per shard, enough tiles
-    # ragged shards on 256 x 256 tiles: room for both operands in rows padded to whole 64-column slabs
-    # (optional: without it the product runs on the rows as they lie)
+    # shards off the line grid on 256 x 256 tiles: the bytes of both operands in rows padded to whole 64-column slabs, as it has
+    # told since these were copied there (unused; gemm_rs_workspace_used leaves them out)
+    assert lib.gemm_rs_workspace_used(8192, 8192, 29568, 8) == 0
     assert lib.gemm_rs_workspace_bytes(8192, 8192, 29568, 8) == 8 * (8192 + 8192) * 3712 * 2
     # a few hundred rows: 256 x 128 tiles with the shards in four groups
     assert lib.gemm_rs_workspace_bytes(512, 4096, 12288, 8) == 4 * 512 * 4096 * 4
@@ -225,14 +226,14 @@ def test_reference_shapes_at_full_size(gpu_device, spec):
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", [256, 129, 131, 132, 130, 128, 32])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("k", [1024, 1440, 4 * 72], ids=["k256", "k360", "k72"])
+@pytest.mark.parametrize("k", [1024, 1440, 4 * 72, 4 * 840], ids=["k256", "k360", "k72", "k840"])
 def test_each_kernel_form(gpu_device, options, form, dtype, k):
     """256 x 256 tiles, 256 x 128 tiles (129; 131 / 132: 192 / 128 of their rows in use, the former on
     the map that deals the tiles out evenly; 130: with per-shard partial products), 128 x 128 tiles and
     their per-shard partial products (32) on one shape with ragged
     edges (M and N not multiples of the tiles); local K a multiple of the 64-column slab, five slabs
     and a short one (360: the wide tiles start the last slab of a shard early and mask what it
-    shares with the one before), and one slab and a bit (72)."""
+    shares with the one before), one slab and a bit (72), and fourteen (840: by whole lines)."""
     options.set("GEMM_TILE", form)
     W, m, n = 4, 392, 600
     g = torch.Generator().manual_seed(form)
@@ -244,8 +245,7 @@ def test_each_kernel_form(gpu_device, options, form, dtype, k):
     x, w, b = G.pack_world(datas, gpu_device)
     exact = O.exact_world(datas)
     ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
-    # ragged shards on the wide tiles: on the zero-padded copy of the operands (with the workspace) and
-    # in place (without it: the early-starting last slab of a shard)
+    # (False: a workspace only where the call is refused without)
     for pad_ragged in (True, False):
         out = G.HipGemmReduceScatter(W, pad_ragged=pad_ragged).forward(x, w, b).cpu()
         err = (out.double() - exact).abs()
@@ -271,18 +271,18 @@ def test_every_tile_of_odd_tile_counts(gpu_device, options, form, m, n):
     assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6).all())
 
 
-@pytest.mark.skipif(torch.cuda.is_available(), reason="its operands do not exist: no call may reach a GPU")
 @pytest.mark.parametrize("W", [2, 8])
 def test_the_room_that_is_asked_for_is_enough(W):
     """No shape is refused with the room that gemm_rs_workspace_used or _bytes tells, none among it (such a shape was, where a plan of
-    one group took the place of one that had to have room)."""
-    lib, rng = _lib.load(), random.Random(W)
+    one group took the place of one that had to have room).  The entry point, compiled for the host: nothing is launched."""
+    rng, shapes = random.Random(W), []
     for i in range(1500):
         m, n = 8 * int(2 ** rng.uniform(0, 10)), 4 * int(2 ** rng.uniform(6, 11.5))
-        k = W * 8 * int(2 ** rng.uniform(3, 9))
-        for need in (lib.gemm_rs_workspace_used(m, n, k, W), lib.gemm_rs_workspace_bytes(m, n, k, W)):
-            rc = lib.gemm_rs_forward(4096, 4096, None, 4096, m, n, k, W, 0, 0, _lib.BF16, 4096 if need else None, need, None)
-            assert rc != E_WORKSPACE, (m, n, k)
+        shapes.append((m, n, 8 * int(2 ** rng.uniform(3, 9)), W, 0, 0, 0, 0))
+    told = [got[-2:] for got in tile_loops.run([("call", 0, 0, *s, 0, 0) for s in shapes])]
+    calls = [("call", 0, 0, *s, need, 0) for s, needs in zip(shapes, told) for need in needs]
+    for call, got in zip(calls, tile_loops.run(calls)):
+        assert got[0] == "0", (call, got)
 
 
 ROOM_OF_EARLIER = [  # W, m, n, kl, bytes, kernels: what gemm_rs_workspace_bytes has told of for these, and is enough for them
@@ -428,11 +428,11 @@ def test_few_rows_by_whole_lines(gpu_device, dtype, m, W, n, kl, at):
 @pytest.mark.gpu
 @pytest.mark.parametrize("form,W,m", [(0, 4, 64), (0, 1, 5), (256, 4, 392), (129, 4, 392), (131, 4, 392), (132, 4, 392),
                                       (130, 4, 392), (128, 4, 392), (32, 4, 392)])
-@pytest.mark.parametrize("kl", [72, 352, 360, 456])
+@pytest.mark.parametrize("kl", [72, 352, 360, 456, 840])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 def test_non_finite_elements_of_ragged_shards(gpu_device, options, dtype, kl, form, W, m):
     """Infinities and NaN in the columns that a last slab which starts early shares with the one before (and elsewhere), in
-    either operand, padded and in place: NaN and infinite of the same sign exactly where the f32 product is, and the other
+    either operand: NaN and infinite of the same sign exactly where the f32 product is, and the other
     results as everywhere (f32 sums rounded once: 2^-8 or 2^-11 of the result, and 1e-6)."""
     options.set("GEMM_TILE", form)
     n, inf, nan = 600, float("inf"), float("nan")
@@ -447,13 +447,12 @@ def test_non_finite_elements_of_ragged_shards(gpu_device, options, dtype, kl, fo
     x[0, 0, shared[0]] = -inf
     want = x.transpose(0, 1).reshape(m, W * kl).float() @ w.transpose(0, 1).reshape(n, W * kl).float().T
     ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
-    for pad_ragged in (True, False):
-        out = G.HipGemmReduceScatter(W, pad_ragged=pad_ragged).forward(x, w).float()
-        torch.cuda.synchronize()
-        assert torch.equal(out.isnan(), want.isnan()), pad_ragged
-        assert torch.equal(out.isposinf(), want.isposinf()) and torch.equal(out.isneginf(), want.isneginf()), pad_ragged
-        finite = want.isfinite()
-        assert bool(((out - want).abs() <= want.abs() * ulp + 1e-6)[finite].all()), pad_ragged
+    out = G.HipGemmReduceScatter(W).forward(x, w).float()
+    torch.cuda.synchronize()
+    assert torch.equal(out.isnan(), want.isnan())
+    assert torch.equal(out.isposinf(), want.isposinf()) and torch.equal(out.isneginf(), want.isneginf())
+    finite = want.isfinite()
+    assert bool(((out - want).abs() <= want.abs() * ulp + 1e-6)[finite].all())
 
 
 @pytest.mark.gpu
@@ -763,16 +762,27 @@ def test_workspace_of_a_stream_and_of_a_graph(gpu_device):
         assert all(bool((o == 7).all()) for o in other)
 
 
+FEWER_ROWS = [(m, n, kl, rows) for m, n, rows in ((2818, 3300, 192), (1500, 7170, 192), (868, 8400, 128), (2304, 3700, 192))
+              for kl in (64, 200, 576, 776)]  # whole slabs; rows as they lie; whole slabs; whole lines
+FEWER_ROWS += [(7248, 2304, kl, 192) for kl in (64, 576, 776)]
+
+
+@pytest.mark.parametrize("m,n,kl,rows", FEWER_ROWS)
+def test_rows_in_use_of_wide_tiles(m, n, kl, rows):
+    """(tiles down, tiles across, rows in use, how they are dealt to the dies)"""
+    kernel, _, _, in_use, _ = tile_loops.run([("call", 2, 0, m, n, kl, 8, 0, 0, 0, 0, 0, 0)])[0][1].split(",")
+    assert (kernel, int(in_use)) == ("wide", rows)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("kl", [64, 200, 576, 776])  # whole slabs; rows as they lie; whole slabs; whole lines
-@pytest.mark.parametrize("m,n", [(2818, 3300), (1500, 7170), (7248, 2304), (868, 8400), (2304, 3700)])
-def test_wide_tiles_of_fewer_rows(gpu_device, m, n, kl):
-    """Outputs of more than 128 tiles of 256 x 256 that tiles with 192 or 128 of their rows in use cover in as many rounds of the CUs:
-    every row and column, a tile's last and the last tile's, with a bias.
+@pytest.mark.parametrize("m,n,kl,rows", FEWER_ROWS)
+def test_wide_tiles_of_fewer_rows(gpu_device, m, n, kl, rows):
+    """Outputs of more than 128 tiles of 256 x 256 that tiles with 192 or 128 of their rows in use cover in as many rounds of the CUs
+    (test_rows_in_use_of_wide_tiles): every row and column, a tile's last and the last tile's, with a bias.
     f32 sums of 8 kl products of up to 0.05^2, rounded once: within 2^-8 of the f32 result and 2e-5."""
     x, w = uniform((8, m, kl), torch.bfloat16, gpu_device, m + kl), uniform((8, n, kl), torch.bfloat16, gpu_device, n)
     bias = uniform((n,), torch.bfloat16, gpu_device, 3)
     out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
-    G.HipGemmReduceScatter(8).forward(x, w, bias, out=out)
+    assert launched(_lib.load(), lambda: G.HipGemmReduceScatter(8).forward(x, w, bias, out=out)) == ["gemm_rs_wide"]
     want = product(x, w, bias)
     assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())

@@ -5,7 +5,7 @@
 // Standard input: a launch a line,
 //   form M N Kl W groups pitch cols a_at b_at a_gap b_gap     (gaps in 16-byte vectors, at: the operands' own, modulo a line)
 // or a call of gemm_rs_forward (bytes of workspace, which begins `ws_at` bytes behind a 16-byte boundary; 0 bytes: none),
-//   call walk option M N Kl W a_at b_at a_gap b_gap bytes ws_at
+//   call what option M N Kl W a_at b_at a_gap b_gap bytes ws_at     (what: 0, 1 to walk its launches, 2 to print their whole numbers)
 // Standard output: of a launch, and of a call's whose launches are to be walked, the requests inside the buffers, those of them outside
 // the operands' rows, and the 16-byte vectors of the operands' rows that nothing asked for; of a call before that the status and
 // the kernels, and of any call the bytes that gemm_rs_workspace_used and _bytes answer at the end.
@@ -132,21 +132,26 @@ static int option(int) { return forced; }
 static bool aligned16(const void* p) { return (uintptr_t)p % 16 == 0; }
 static int ceil_div(int a, int b) { return (a + b - 1) / b; }
 static std::string launched;
-static bool walked;
+static bool walked, numbers;
+template <class T>
+static void show(const T& v) {
+  if constexpr (std::is_integral_v<T>) launched += "," + std::to_string(v);
+}
 template <class T> struct same_type { typedef T type; };
 template <class... A>
 static int launch(int kid, void (*kernel)(A...), Dim grid, Dim block, size_t, hipStream_t, typename same_type<A>::type... args) {
   launched += std::string(" ") + kNames[kid];
+  if (numbers) (show(args), ...);
   if (walked && kid != KID_GEMM_RS_REDUCE && kernel != (void (*)(A...))nullptr) walk([&] { kernel(args...); }, grid, (int)block.x);
   return 0;
 }
 #include "entry.inc"
 
 static void call() {
-  int walk_it, M, N, Kl, W, a_at, b_at, ws_at;
+  int what, M, N, Kl, W, a_at, b_at, ws_at;
   long long a_gap, b_gap, bytes;
-  if (scanf("%d %d %d %d %d %d %d %d %lld %lld %lld %d", &walk_it, &forced, &M, &N, &Kl, &W, &a_at, &b_at, &a_gap, &b_gap, &bytes, &ws_at) != 12) return;
-  walked = walk_it != 0;
+  if (scanf("%d %d %d %d %d %d %d %d %lld %lld %lld %d", &what, &forced, &M, &N, &Kl, &W, &a_at, &b_at, &a_gap, &b_gap, &bytes, &ws_at) != 12) return;
+  walked = what == 1, numbers = what == 2;
   place(M, N, Kl, W, a_at, b_at, a_gap, b_gap, walked);
   launched.clear();
   std::vector<uint4> out(walked ? (size_t)M * N / 8 + 1 : 1), room(walked ? bytes / 16 + 2 : 2);
