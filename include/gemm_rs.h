@@ -54,7 +54,9 @@ extern "C" {
  * when that fills the CUs better), 130 those with one partial product per shard, 133 the 256 x 256 tiles with
  * one partial product per shard, 128 the 128 x 128
  * tiles, 32 those with one partial product per shard.  All unsplit forms give identical bits, except that the
- * 256 x 256 tiles sum in another order where the local K is not a multiple of 64.
+ * 256 x 256 tiles sum in another order where the local K is not a multiple of 64.  There, with long shards or large outputs, and in groups of
+ * shards too, the order also depends on where input begins within a line of 128 bytes and on which rows share a tile, so on M: the same
+ * row, in a view that begins elsewhere or beside other rows, may be rounded otherwise.  The same call on the same addresses gives the same bits.
  */
 size_t gemm_rs_workspace_bytes(int M, int N, int K, int W);
 size_t gemm_rs_workspace_used(int M, int N, int K, int W);

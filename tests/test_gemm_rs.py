@@ -633,6 +633,28 @@ def test_tiles_of_rows_as_they_lie(gpu_device, options, dtype, form, W, m, n, kl
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kl", [256, 96, 136, 360, 776, 840])
+def test_same_bits(gpu_device, options, kl):
+    """What include/gemm_rs.h says of the order of sums: the same in all unsplit forms, but for 256 x 256 tiles off the grid of 64, and the same
+    wherever the operands begin, but for these tiles by whole lines (from twelve slabs on, here)."""
+    W, m, n, results = 4, 392, 600, {}
+    for at in (0, 24, 40):  # elements: on the grid of cache lines, and 48 and 80 bytes off it
+        x, w = (torch.empty(8 * 8 + W * r * kl, dtype=torch.bfloat16, device=gpu_device)[at:at + W * r * kl].view(W, r, kl) for r in (m, n))
+        x.copy_(uniform((W, m, kl), torch.bfloat16, gpu_device, kl))
+        w.copy_(uniform((W, n, kl), torch.bfloat16, gpu_device, kl + 1))
+        for form in (129, 131, 132, 128, 256):
+            options.set("GEMM_TILE", form)
+            out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+            G.HipGemmReduceScatter(W).forward(x, w, out=out)
+            results[form, at] = out.view(torch.int16)
+    for (form, at), got in results.items():
+        if form != 256 or kl % 64 == 0:
+            assert torch.equal(got, results[129, 0]), (form, at)
+        elif kl <= 11 * 64:
+            assert torch.equal(got, results[256, 0]), at
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("form,m,n,kl,kernels", [
     (256, 520, 264, 776, "wide"), (133, 520, 264, 776, "split reduce"), (129, 520, 264, 776, "narrow"), (131, 400, 264, 360, "narrow"),
     (132, 300, 264, 200, "narrow"), (130, 300, 264, 456, "narrow reduce"), (0, 40, 8200, 2728, "tile reduce"),  # (more than 84 MiB of weights)
