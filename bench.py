@@ -1000,7 +1000,7 @@ def gemm_rs_leg(args, lib, torch, dev):
                     kernels_us=summarise(per), kernel_us=round(t_us, 2),
                     reference_speed_of_light_us_per_gpu_of_8=sol_us.get((m, n, k)))
         # algorithmic bytes: operands in and the result out, once (what a split form writes and reads again
-        # as partial products, or a padded copy, is the implementation's own traffic and earns nothing)
+        # as partial products is the implementation's own traffic and earns nothing)
         gemm_bytes = (m + n) * k * 2 + m * n * 2
         if gemm_bytes / (HBM_PEAK_GBPS * 1e3) > flops / (MFMA_PEAK_TFLOPS * 1e6):
             gbps = gemm_bytes / t_us / 1e3

@@ -82,7 +82,7 @@ class HipGemmReduceScatter:
     def __init__(self, world_size: int, pad_ragged: bool = True):
         self.world_size = int(world_size)
         # False: a shape whose workspace is optional (partial products of groups of shards, where they only pay) is
-        # multiplied without it
+        # multiplied without it.  (Nothing is padded: the name is that of the first such workspace, a copy of the operands.)
         self.pad_ragged = bool(pad_ragged)
         self.lib = _lib.load()
         self._workspaces = {}  # (device, stream) -> workspace of the calls on that stream
