@@ -141,13 +141,18 @@ def test_host_side_argument_checks():
     assert call(M=64, N=7168, K=18432) == E_WORKSPACE
     assert call(M=64, N=7168, K=18432, ws=A, wsb=need - 1) == E_WORKSPACE
     assert lib.gemm_rs_workspace_bytes(8192, 4096, 14336, 8) == 0  # whole slabs per shard, enough tiles
-    # shards off the line grid on 256 x 256 tiles: the bytes of both operands in rows padded to whole 64-column slabs, as it has
-    # told since these were copied there (unused; gemm_rs_workspace_used leaves them out)
-    assert lib.gemm_rs_workspace_used(8192, 8192, 29568, 8) == 0
+    # ragged shards on 256 x 256 tiles: room for both operands in rows padded to whole 64-column slabs
+    # (optional: without it the product runs on the rows as they lie)
     assert lib.gemm_rs_workspace_bytes(8192, 8192, 29568, 8) == 8 * (8192 + 8192) * 3712 * 2
     # a few hundred rows: 256 x 128 tiles with the shards in four groups
     assert lib.gemm_rs_workspace_bytes(512, 4096, 12288, 8) == 4 * 512 * 4096 * 4
     assert lib.gemm_rs_workspace_bytes(64, 64, 100, 8) == 0  # invalid shape: no size
+
+
+def test_bytes_told_of_and_not_used():
+    """Shards off the line grid on 256 x 256 tiles: the room that gemm_rs_workspace_bytes tells of has not been used since operands were
+    copied there."""
+    assert _lib.load().gemm_rs_workspace_used(8192, 8192, 29568, 8) == 0
 
 
 @pytest.mark.parametrize("m,n,k,groups", [
@@ -226,14 +231,14 @@ def test_reference_shapes_at_full_size(gpu_device, spec):
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", [256, 129, 131, 132, 130, 128, 32])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("k", [1024, 1440, 4 * 72, 4 * 840], ids=["k256", "k360", "k72", "k840"])
+@pytest.mark.parametrize("k", [1024, 1440, 4 * 72], ids=["k256", "k360", "k72"])
 def test_each_kernel_form(gpu_device, options, form, dtype, k):
     """256 x 256 tiles, 256 x 128 tiles (129; 131 / 132: 192 / 128 of their rows in use, the former on
     the map that deals the tiles out evenly; 130: with per-shard partial products), 128 x 128 tiles and
     their per-shard partial products (32) on one shape with ragged
     edges (M and N not multiples of the tiles); local K a multiple of the 64-column slab, five slabs
     and a short one (360: the wide tiles start the last slab of a shard early and mask what it
-    shares with the one before), one slab and a bit (72), and fourteen (840: by whole lines)."""
+    shares with the one before), and one slab and a bit (72)."""
     options.set("GEMM_TILE", form)
     W, m, n = 4, 392, 600
     g = torch.Generator().manual_seed(form)
@@ -245,11 +250,20 @@ def test_each_kernel_form(gpu_device, options, form, dtype, k):
     x, w, b = G.pack_world(datas, gpu_device)
     exact = O.exact_world(datas)
     ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
-    # (False: a workspace only where the call is refused without)
+    # ragged shards on the wide tiles: on the zero-padded copy of the operands (with the workspace) and
+    # in place (without it: the early-starting last slab of a shard)
     for pad_ragged in (True, False):
         out = G.HipGemmReduceScatter(W, pad_ragged=pad_ragged).forward(x, w, b).cpu()
         err = (out.double() - exact).abs()
         assert bool((err <= exact.abs() * ulp + 1e-6).all()), (pad_ragged, float(err.max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [256, 129, 131, 132, 130, 128, 32])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_each_kernel_form_by_whole_lines(gpu_device, options, form, dtype):
+    """The same with fourteen slabs to a shard, the last a short one, which tiles of 256 rows request by whole lines."""
+    test_each_kernel_form(gpu_device, options, form, dtype, 4 * 840)
 
 
 @pytest.mark.gpu
@@ -271,10 +285,23 @@ def test_every_tile_of_odd_tile_counts(gpu_device, options, form, m, n):
     assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6).all())
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="its operands do not exist: no call may reach a GPU")
 @pytest.mark.parametrize("W", [2, 8])
 def test_the_room_that_is_asked_for_is_enough(W):
     """No shape is refused with the room that gemm_rs_workspace_used or _bytes tells, none among it (such a shape was, where a plan of
-    one group took the place of one that had to have room).  The entry point, compiled for the host: nothing is launched."""
+    one group took the place of one that had to have room)."""
+    lib, rng = _lib.load(), random.Random(W)
+    for i in range(1500):
+        m, n = 8 * int(2 ** rng.uniform(0, 10)), 4 * int(2 ** rng.uniform(6, 11.5))
+        k = W * 8 * int(2 ** rng.uniform(3, 9))
+        for need in (lib.gemm_rs_workspace_used(m, n, k, W), lib.gemm_rs_workspace_bytes(m, n, k, W)):
+            rc = lib.gemm_rs_forward(4096, 4096, None, 4096, m, n, k, W, 0, 0, _lib.BF16, 4096 if need else None, need, None)
+            assert rc != E_WORKSPACE, (m, n, k)
+
+
+@pytest.mark.parametrize("W", [2, 8])
+def test_the_room_that_is_told_is_enough_on_the_host(W):
+    """The same of the entry point compiled for the host, which runs everywhere: nothing is launched."""
     rng, shapes = random.Random(W), []
     for i in range(1500):
         m, n = 8 * int(2 ** rng.uniform(0, 10)), 4 * int(2 ** rng.uniform(6, 11.5))
@@ -428,11 +455,11 @@ def test_few_rows_by_whole_lines(gpu_device, dtype, m, W, n, kl, at):
 @pytest.mark.gpu
 @pytest.mark.parametrize("form,W,m", [(0, 4, 64), (0, 1, 5), (256, 4, 392), (129, 4, 392), (131, 4, 392), (132, 4, 392),
                                       (130, 4, 392), (128, 4, 392), (32, 4, 392)])
-@pytest.mark.parametrize("kl", [72, 352, 360, 456, 840])
+@pytest.mark.parametrize("kl", [72, 352, 360, 456])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 def test_non_finite_elements_of_ragged_shards(gpu_device, options, dtype, kl, form, W, m):
     """Infinities and NaN in the columns that a last slab which starts early shares with the one before (and elsewhere), in
-    either operand: NaN and infinite of the same sign exactly where the f32 product is, and the other
+    either operand, padded and in place: NaN and infinite of the same sign exactly where the f32 product is, and the other
     results as everywhere (f32 sums rounded once: 2^-8 or 2^-11 of the result, and 1e-6)."""
     options.set("GEMM_TILE", form)
     n, inf, nan = 600, float("inf"), float("nan")
@@ -447,12 +474,22 @@ def test_non_finite_elements_of_ragged_shards(gpu_device, options, dtype, kl, fo
     x[0, 0, shared[0]] = -inf
     want = x.transpose(0, 1).reshape(m, W * kl).float() @ w.transpose(0, 1).reshape(n, W * kl).float().T
     ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
-    out = G.HipGemmReduceScatter(W).forward(x, w).float()
-    torch.cuda.synchronize()
-    assert torch.equal(out.isnan(), want.isnan())
-    assert torch.equal(out.isposinf(), want.isposinf()) and torch.equal(out.isneginf(), want.isneginf())
-    finite = want.isfinite()
-    assert bool(((out - want).abs() <= want.abs() * ulp + 1e-6)[finite].all())
+    for pad_ragged in (True, False):
+        out = G.HipGemmReduceScatter(W, pad_ragged=pad_ragged).forward(x, w).float()
+        torch.cuda.synchronize()
+        assert torch.equal(out.isnan(), want.isnan()), pad_ragged
+        assert torch.equal(out.isposinf(), want.isposinf()) and torch.equal(out.isneginf(), want.isneginf()), pad_ragged
+        finite = want.isfinite()
+        assert bool(((out - want).abs() <= want.abs() * ulp + 1e-6)[finite].all()), pad_ragged
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,W,m", [(0, 4, 64), (0, 1, 5), (256, 4, 392), (129, 4, 392), (131, 4, 392), (132, 4, 392),
+                                      (130, 4, 392), (128, 4, 392), (32, 4, 392)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_non_finite_elements_of_long_ragged_shards(gpu_device, options, dtype, form, W, m):
+    """The same with fourteen slabs to a shard, which tiles of 256 rows request by whole lines."""
+    test_non_finite_elements_of_ragged_shards(gpu_device, options, dtype, 840, form, W, m)
 
 
 @pytest.mark.gpu
@@ -547,6 +584,66 @@ def uniform(shape, dtype, dev, seed):
     return torch.empty(*shape, dtype=dtype, device=dev).uniform_(-0.05, 0.05, generator=g)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,m,n,kl", [
+    (2, 65, 8, 64), (2, 256, 256, 72), (8, 257, 260, 64), (4, 392, 600, 360), (8, 72, 4100, 96), (3, 520, 2052, 200),
+    (4, 1040, 1000, 128),  # more than a round of tiles
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_wide_tiles_with_the_shards_in_groups(gpu_device, options, dtype, W, m, n, kl):
+    """Every row and column at the edges of tiles, slabs and groups, with a bias and an infinite element on either side.  f32
+    sums of W kl products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 product and 1e-5."""
+    options.set("GEMM_TILE", 133)
+    x, w, bias = (uniform(s, dtype, gpu_device, m + n + i) for i, s in enumerate(((W, m, kl), (W, n, kl), (n,))))
+    x[W - 1, m - 1, kl - 1] = float("inf")
+    w[0, n - 1, kl - 8] = float("-inf")
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
+    kernels = launched(_lib.load(), lambda: G.HipGemmReduceScatter(W).forward(x, w, bias, out=out))
+    assert kernels == ["gemm_rs_split", "gemm_rs_reduce"]
+    want = product(x, w, bias)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
+    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form,W,m,n,kl,at", [
+    (256, 8, 2056, 264, 712, 0), (256, 3, 1030, 520, 728, 3), (256, 2, 520, 260, 1000, 5),  # rows alike eight, four apart, too few
+    (256, 1, 300, 256, 904, 7), (256, 2, 4104, 72, 720, 1), (256, 4, 1291, 40, 744, 2),  # one shard; half lines; classes of unequal length
+    (133, 8, 1030, 264, 72, 3), (133, 2, 1040, 260, 136, 5), (133, 4, 530, 520, 200, 6), (133, 2, 257, 256, 264, 1),  # two slabs, three, four, five
+    (129, 4, 520, 264, 136, 3), (131, 3, 400, 264, 200, 6), (132, 2, 264, 520, 72, 1), (130, 4, 300, 264, 456, 7),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_tiles_by_whole_lines(gpu_device, options, dtype, form, W, m, n, kl, at):
+    """Rows off the grid of cache lines on the tiles of eight waves: chunks that lag a request behind, at the first and last slabs of
+    shards and past the last one, rows of x that lie alike dealt to the same tile, with an infinite element in either operand's last column
+    and its first.  Operands that start 16 `at` bytes into a line, and shards 24 and 40 elements apart whose gaps hold NaN.  f32 sums
+    of W kl products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 result and 1e-5."""
+    lib, gaps = _lib.load(), (24, 40)
+    options.set("GEMM_TILE", form)
+    flat, parts = [], []
+    for rows, gap, seed in ((m, gaps[0], 1), (n, gaps[1], 2)):
+        t = torch.full((8 * at + W * (rows * kl + gap),), float("nan"), dtype=dtype, device=gpu_device)
+        part = t[8 * at:].view(W, rows * kl + gap)[:, :rows * kl].unflatten(1, (rows, kl))
+        part.copy_(uniform((W, rows, kl), dtype, gpu_device, seed + kl))
+        flat.append(t)
+        parts.append(part)
+    x, w = parts
+    x[W - 1, m - 1, kl - 1] = float("inf")
+    x[0, m // 2, 0] = float("-inf")
+    w[0, n - 1, kl - 1] = float("-inf")
+    w[W - 1, 5, 0] = float("inf")
+    out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
+    ws = torch.empty(max(16, lib.gemm_rs_workspace_bytes(m, n, kl * W, W)), dtype=torch.uint8, device=gpu_device)
+    assert lib.gemm_rs_forward(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), m, n, kl * W, W, m * kl + gaps[0], n * kl + gaps[1],
+                               _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(),
+                               torch.cuda.current_stream().cuda_stream) == 0
+    want = product(x, w)
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
+    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
+
+
 def check_off_the_line_grid(dev, dtype, W, m, n, kl, at, gaps=(24, 40)):
     """The product of shards whose rows lie off the grid of cache lines, with an infinite element in either operand's last column and its
     first.  Operands that start 16 `at` bytes into a line, and shards so many elements apart whose gaps hold NaN.  f32 sums of W kl
@@ -579,40 +676,16 @@ def check_off_the_line_grid(dev, dtype, W, m, n, kl, at, gaps=(24, 40)):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("W,m,n,kl", [
-    (2, 65, 8, 64), (2, 256, 256, 72), (8, 257, 260, 64), (4, 392, 600, 360), (8, 72, 4100, 96), (3, 520, 2052, 200),
-    (4, 1040, 1000, 128),  # more than a round of tiles
-])
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-def test_wide_tiles_with_the_shards_in_groups(gpu_device, options, dtype, W, m, n, kl):
-    """Every row and column at the edges of tiles, slabs and groups, with a bias and an infinite element on either side.  f32
-    sums of W kl products of up to 0.05^2, rounded once: within 2^-8 (fp16: 2^-11) of the f32 product and 1e-5."""
-    options.set("GEMM_TILE", 133)
-    x, w, bias = (uniform(s, dtype, gpu_device, m + n + i) for i, s in enumerate(((W, m, kl), (W, n, kl), (n,))))
-    x[W - 1, m - 1, kl - 1] = float("inf")
-    w[0, n - 1, kl - 8] = float("-inf")
-    out = torch.full((m, n), float("nan"), dtype=dtype, device=gpu_device)
-    kernels = launched(_lib.load(), lambda: G.HipGemmReduceScatter(W).forward(x, w, bias, out=out))
-    assert kernels == ["gemm_rs_split", "gemm_rs_reduce"]
-    want = product(x, w, bias)
-    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
-    ulp, finite = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11, want.isfinite()
-    assert bool(((out.float() - want).abs() <= want.abs() * ulp + 1e-5)[finite].all())
-
-
-@pytest.mark.gpu
 @pytest.mark.parametrize("form,W,m,n,kl,at", [
-    (256, 8, 2056, 264, 712, 0), (256, 3, 1030, 520, 728, 3), (256, 2, 520, 260, 1000, 5),  # rows alike eight, four apart, too few
-    (256, 1, 300, 256, 904, 7), (256, 2, 4104, 72, 720, 1), (256, 4, 1291, 40, 744, 2),  # one shard; half lines; classes of unequal length
     (256, 2, 6160, 6144, 72, 3), (256, 1, 6144, 6152, 136, 5), (256, 2, 6150, 6144, 200, 6), (256, 1, 6152, 6144, 264, 1),  # two slabs, three, four, five
     (133, 8, 2060, 1032, 72, 3), (133, 8, 2060, 1032, 136, 5), (133, 4, 4120, 1032, 200, 6), (133, 8, 2060, 1032, 264, 1),
     (133, 8, 1030, 264, 584, 3), (133, 2, 1040, 260, 648, 5), (133, 4, 530, 520, 712, 6), (133, 2, 257, 256, 776, 1),
-    (129, 4, 520, 264, 776, 3), (131, 3, 400, 264, 200, 6), (132, 2, 264, 520, 72, 1), (130, 4, 300, 264, 456, 7),
+    (129, 4, 520, 264, 776, 3),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-def test_tiles_by_whole_lines(gpu_device, options, dtype, form, W, m, n, kl, at):
-    """Rows off the grid of cache lines on the tiles of eight waves: chunks that lag a request behind, at the first and last slabs of
-    shards and past the last one, rows of x that lie alike dealt to the same tile (check_off_the_line_grid)."""
+def test_tiles_by_whole_lines_from_where_these_begin(gpu_device, options, dtype, form, W, m, n, kl, at):
+    """The same where whole lines are chosen on both sides of gemm_rs_along: short shards of large outputs or of more tiles than a round of the
+    CUs, and long ones (check_off_the_line_grid)."""
     options.set("GEMM_TILE", form)
     check_off_the_line_grid(gpu_device, dtype, W, m, n, kl, at)
 
@@ -784,6 +857,21 @@ def test_workspace_of_a_stream_and_of_a_graph(gpu_device):
         assert all(bool((o == 7).all()) for o in other)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("kl", [64, 200, 576, 776])  # whole slabs; rows as they lie; whole slabs; whole lines
+@pytest.mark.parametrize("m,n", [(2818, 3300), (1500, 7170), (7248, 2304), (868, 8400), (2304, 3700)])
+def test_wide_tiles_of_fewer_rows(gpu_device, m, n, kl):
+    """Outputs of more than 128 tiles of 256 x 256 that tiles with 192 or 128 of their rows in use cover in as many rounds of the CUs:
+    every row and column, a tile's last and the last tile's, with a bias.
+    f32 sums of 8 kl products of up to 0.05^2, rounded once: within 2^-8 of the f32 result and 2e-5."""
+    x, w = uniform((8, m, kl), torch.bfloat16, gpu_device, m + kl), uniform((8, n, kl), torch.bfloat16, gpu_device, n)
+    bias = uniform((n,), torch.bfloat16, gpu_device, 3)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    G.HipGemmReduceScatter(8).forward(x, w, bias, out=out)
+    want = product(x, w, bias)
+    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
+
+
 FEWER_ROWS = [(m, n, kl, rows) for m, n, rows in ((2818, 3300, 192), (1500, 7170, 192), (868, 8400, 128), (2304, 3700, 192))
               for kl in (64, 200, 576, 776)]  # whole slabs; rows as they lie; whole slabs; whole lines
 FEWER_ROWS += [(7248, 2304, kl, 192) for kl in (64, 576, 776)]
@@ -797,14 +885,8 @@ def test_rows_in_use_of_wide_tiles(m, n, kl, rows):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,kl,rows", FEWER_ROWS)
-def test_wide_tiles_of_fewer_rows(gpu_device, m, n, kl, rows):
-    """Outputs of more than 128 tiles of 256 x 256 that tiles with 192 or 128 of their rows in use cover in as many rounds of the CUs
-    (test_rows_in_use_of_wide_tiles): every row and column, a tile's last and the last tile's, with a bias.
-    f32 sums of 8 kl products of up to 0.05^2, rounded once: within 2^-8 of the f32 result and 2e-5."""
+@pytest.mark.parametrize("m,n,kl,rows", [shape for shape in FEWER_ROWS if shape[:2] in ((2818, 3300), (868, 8400))])
+def test_wide_tiles_are_what_runs(gpu_device, m, n, kl, rows):
+    """(test_wide_tiles_of_fewer_rows has the results)"""
     x, w = uniform((8, m, kl), torch.bfloat16, gpu_device, m + kl), uniform((8, n, kl), torch.bfloat16, gpu_device, n)
-    bias = uniform((n,), torch.bfloat16, gpu_device, 3)
-    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
-    assert launched(_lib.load(), lambda: G.HipGemmReduceScatter(8).forward(x, w, bias, out=out)) == ["gemm_rs_wide"]
-    want = product(x, w, bias)
-    assert bool(((out.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5).all())
+    assert launched(_lib.load(), lambda: G.HipGemmReduceScatter(8).forward(x, w)) == ["gemm_rs_wide"]
